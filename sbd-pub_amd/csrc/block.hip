@@ -85,78 +85,189 @@ __device__ __forceinline__ void block_put(double v, int idx, double *sh, int str
   if ((threadIdx.x & 63) == 0) sh[(threadIdx.x >> 6) * stride + idx] = w;
 }
 
-template <typename TA, typename TB>
-__device__ __forceinline__ void gram_tile(const TA *const *pa, int ma, const TB *const *pb, int mb, size_t n,
-                                          double (&s)[8][8]) {
-  const TA *a[8];
-  const TB *b[8];
-#pragma unroll
-  for (int q = 0; q < 8; q++) {
-    a[q] = pa[q < ma ? q : 0];
-    b[q] = pb[q < mb ? q : 0];
-  }
-#pragma unroll
-  for (int x = 0; x < 8; x++)
-#pragma unroll
-    for (int y = 0; y < 8; y++) s[x][y] = 0.0;
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    double av[8], bv[8];
-#pragma unroll
-    for (int q = 0; q < 8; q++) {
-      av[q] = (double)a[q][i];
-      bv[q] = (double)b[q][i];
-    }
-#pragma unroll
-    for (int x = 0; x < 8; x++)
-#pragma unroll
-      for (int y = 0; y < 8; y++) s[x][y] += av[x] * bv[y];
-  }
+// Two consecutive values of a column from element i on, widened; columns
+// start at any multiple of their element size (N may be odd), which is all
+// that a global load of several words needs.
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef double d4v __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void load2(const double *p, double (&v)[2]) {
+  const d2u t = *reinterpret_cast<const d2u *>(p);
+  v[0] = t.x;
+  v[1] = t.y;
 }
+__device__ __forceinline__ void load2(const float *p, double (&v)[2]) {
+  const f2u t = *reinterpret_cast<const f2u *>(p);
+  v[0] = (double)t.x;
+  v[1] = (double)t.y;
+}
+
+constexpr int kGramChunk = 16;   // elements of every column per wavefront step
+constexpr int kGramBlocks = 512;
 
 // part[blk * (na*nb) + a*nb + b] = this block's share of A_a . B_b, for the
-// na = A.nd + A.nf and nb = B.nd + B.nf columns (tiles of 8 x 8 that do not
-// straddle the FP64/FP32 boundary of either list).
+// na <= 64 and nb <= 16 columns of A and B, on the FP64 matrix cores: a
+// wavefront takes 16 elements of every column per step; lane l holds, for
+// column l % 16 of each tile of 16 columns, the elements 4 (l/16) .. + 3,
+// and the q-th of them of all lanes are one 16x16x4 operand (the order of
+// the elements within the contraction is free).  A column's 16 elements are
+// one or two cache lines, every column is read once, and the sums stay in
+// NA x 4 accumulator registers until the end, so the kernel is bound by
+// reading the columns.  The tile of dot products per thread that this
+// replaces summed 64 values per tile over the lanes by shuffles for 4
+// elements per thread: 244 -> 106 us on average over the passes of 33 to 64
+// FP32 columns of 1M elements against 4 (a three-root solve).
+template <int NA>
 __global__ void __launch_bounds__(kBT) k_bgram(Cols A, Cols B, size_t n, double *__restrict__ part) {
-  __shared__ double sh[4 * 64];
+  __shared__ double sh[4][256];
   const int na = A.nd + A.nf, nb = B.nd + B.nf, tot = na * nb;
-  for (int sa = 0; sa < 2; sa++) {
-    const int nsa = sa ? A.nf : A.nd, offa = sa ? A.nd : 0;
-    for (int ga = 0; ga < nsa; ga += 8) {
-      const int ma = min(8, nsa - ga);
-      for (int sb = 0; sb < 2; sb++) {
-        const int nsb = sb ? B.nf : B.nd, offb = sb ? B.nd : 0;
-        for (int gb = 0; gb < nsb; gb += 8) {
-          const int mb = min(8, nsb - gb);
-          double s[8][8];
-          if (!sa && !sb) gram_tile<double, double>(A.d + ga, ma, B.d + gb, mb, n, s);
-          else if (!sa) gram_tile<double, float>(A.d + ga, ma, B.f + gb, mb, n, s);
-          else if (!sb) gram_tile<float, double>(A.f + ga, ma, B.d + gb, mb, n, s);
-          else gram_tile<float, float>(A.f + ga, ma, B.f + gb, mb, n, s);
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int col = lane & 15, e0 = 4 * (lane >> 4);
+  // this lane's columns; a lane past the end repeats column 0 (its products
+  // are not stored)
+  const double *ad[NA], *bd = nullptr;
+  const float *af[NA], *bf = nullptr;
 #pragma unroll
-          for (int x = 0; x < 8; x++)
+  for (int t = 0; t < NA; t++) {
+    const int k = 16 * t + col < na ? 16 * t + col : 0;
+    ad[t] = k < A.nd ? A.d[k] : nullptr;
+    af[t] = k < A.nd ? nullptr : A.f[k - A.nd];
+  }
+  {
+    const int k = col < nb ? col : 0;
+    if (k < B.nd) bd = B.d[k];
+    else bf = B.f[k - B.nd];
+  }
+  d4v acc[NA];
 #pragma unroll
-            for (int y = 0; y < 8; y++) block_put(s[x][y], x * 8 + y, sh, 64);
-          __syncthreads();
-          const int t = threadIdx.x;
-          if (t < 64 && (t >> 3) < ma && (t & 7) < mb) {
-            const double v = ((sh[t] + sh[64 + t]) + sh[128 + t]) + sh[192 + t];
-            part[(size_t)blockIdx.x * tot + (size_t)(offa + ga + (t >> 3)) * nb + offb + gb + (t & 7)] = v;
-          }
-          __syncthreads();
-        }
-      }
+  for (int t = 0; t < NA; t++) acc[t] = d4v{0.0, 0.0, 0.0, 0.0};
+  auto get4 = [](const double *d, const float *f, size_t i, double (&v)[4]) {
+    if (d) {
+      const d2u x = *reinterpret_cast<const d2u *>(d + i), y = *reinterpret_cast<const d2u *>(d + i + 2);
+      v[0] = x.x, v[1] = x.y, v[2] = y.x, v[3] = y.y;
+    } else {
+      const f4u x = *reinterpret_cast<const f4u *>(f + i);
+      v[0] = x.x, v[1] = x.y, v[2] = x.z, v[3] = x.w;
     }
+  };
+  auto step = [&](const double (&bv)[4], const double (&av)[NA][4]) {
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+#pragma unroll
+      for (int t = 0; t < NA; t++) acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[t][q], bv[q], acc[t], 0, 0, 0);
+  };
+  const size_t nch = n / kGramChunk;
+  const size_t w0 = (size_t)blockIdx.x * 4 + wv, ws = (size_t)gridDim.x * 4;
+  for (size_t ch = w0; ch < nch; ch += ws) {
+    const size_t i = ch * kGramChunk + e0;
+    double bv[4], av[NA][4];
+    get4(bd, bf, i, bv);
+#pragma unroll
+    for (int t = 0; t < NA; t++) get4(ad[t], af[t], i, av[t]);
+    step(bv, av);
+  }
+  if (w0 == 0 && nch * kGramChunk < n) {  // the last, partial chunk
+    double bv[4], av[NA][4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const size_t i = nch * kGramChunk + e0 + q;
+      const bool in = i < n;
+      bv[q] = !in ? 0.0 : bd ? bd[i] : (double)bf[i];
+#pragma unroll
+      for (int t = 0; t < NA; t++) av[t][q] = !in ? 0.0 : ad[t] ? ad[t][i] : (double)af[t][i];
+    }
+    step(bv, av);
+  }
+  // the four wavefronts' tiles in order; accumulator r of lane l is row
+  // 4 r + l / 16, column l % 16
+#pragma unroll
+  for (int t = 0; t < NA; t++) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) sh[wv][(4 * r + (lane >> 4)) * 16 + col] = acc[t][r];
+    __syncthreads();
+    const int a = 16 * t + (threadIdx.x >> 4), b = threadIdx.x & 15;
+    if (a < na && b < nb)
+      part[(size_t)blockIdx.x * tot + (size_t)a * nb + b] =
+          ((sh[0][threadIdx.x] + sh[1][threadIdx.x]) + sh[2][threadIdx.x]) + sh[3][threadIdx.x];
+    __syncthreads();
   }
 }
 
-// out[t] = sum over blocks b (in order) of part[b*tot + t]
-__global__ void k_bsum(int tot, int nblk, const double *__restrict__ part, double *__restrict__ out) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= tot) return;
+// out[t] = fixed-order sum over the nblk blocks of part[b*tot + t]: 32
+// outputs per block, thread row q of 8 adds b = q, q + 8, ... (rows of 32
+// consecutive outputs, so the loads are coalesced and independent), then
+// the 8 rows in order.  One thread per output adding the partials one after
+// the other took 211 us for 1024 blocks; this takes 6 us for 512.
+__global__ void __launch_bounds__(256) k_bsum(int tot, int nblk, const double *__restrict__ part,
+                                              double *__restrict__ out) {
+  __shared__ double sh[8][32];
+  const int t = blockIdx.x * 32 + (threadIdx.x & 31), q = threadIdx.x >> 5;
   double s = 0.0;
-  for (int b = 0; b < nblk; b++) s += part[(size_t)b * tot + t];
-  out[t] = s;
+  if (t < tot) {
+#pragma unroll 8
+    for (int b = q; b < nblk; b += 8) s += part[(size_t)b * tot + t];
+  }
+  sh[q][threadIdx.x & 31] = s;
+  __syncthreads();
+  if (q == 0 && t < tot) {
+    for (int k = 1; k < 8; k++) s += sh[k][threadIdx.x];
+    out[t] = s;
+  }
+}
+
+// Modified Gram-Schmidt among the vectors of one block without the host:
+// p_out[blk] = this block's share of x . v
+__global__ void __launch_bounds__(kBT) k_mgs_dot(const double *__restrict__ x, const double *__restrict__ v, size_t n,
+                                                 double *__restrict__ p_out) {
+  __shared__ double sh[4];
+  const size_t stride = (size_t)gridDim.x * blockDim.x;
+  double s = 0.0;
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) s += x[i] * v[i];
+  block_put(s, 0, sh, 1);
+  __syncthreads();
+  if (threadIdx.x == 0) p_out[blockIdx.x] = ((sh[0] + sh[1]) + sh[2]) + sh[3];
+}
+
+// Sum of nblk partials by the first wavefront, in a fixed order, to *s.
+__device__ __forceinline__ void sum_parts(const double *part, int nblk, double *s) {
+  if (threadIdx.x < 64) {
+    double v = 0.0;
+    for (int b = threadIdx.x; b < nblk; b += 64) v += part[b];
+    v = wave_sum(v);
+    if (threadIdx.x == 0) *s = v;
+  }
+}
+
+// v -= (x . v)/|x|^2 x with x . v in p_in and |x|^2 in *n2 (0: x was
+// dropped, v stays), and the next projection's share of next . v to p_out.
+__global__ void __launch_bounds__(kBT) k_mgs_step(const double *__restrict__ x, const double *next, double *v,
+                                                  size_t n, const double *__restrict__ p_in, int nblk,
+                                                  const double *__restrict__ n2, double *__restrict__ p_out) {
+  __shared__ double sh[4], dot;
+  sum_parts(p_in, nblk, &dot);
+  __syncthreads();
+  const double o = *n2 > 0.0 ? dot / *n2 : 0.0;
+  const size_t stride = (size_t)gridDim.x * blockDim.x;
+  double s = 0.0;
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+    const double t = v[i] - o * x[i];
+    v[i] = t;
+    s += (next == v ? t : next[i]) * t;
+  }
+  block_put(s, 0, sh, 1);
+  __syncthreads();
+  if (threadIdx.x == 0) p_out[blockIdx.x] = ((sh[0] + sh[1]) + sh[2]) + sh[3];
+}
+
+// *n2 = |v|^2 from the partials, or 0 when it has fallen to 1e-20 of *ref
+// or is not positive (the vector is dropped).
+__global__ void __launch_bounds__(64) k_mgs_norm(const double *__restrict__ part, int nblk,
+                                                 const double *__restrict__ ref, double *__restrict__ n2) {
+  __shared__ double s;
+  sum_parts(part, nblk, &s);
+  __syncthreads();
+  if (threadIdx.x == 0) *n2 = (s > 1e-20 * *ref && s > 0.0) ? s : 0.0;
 }
 
 // out_j = sum_k U[k + ld*j] in_k for j < nout <= kOutMax.  In place is
@@ -205,125 +316,131 @@ __global__ void __launch_bounds__(kBT) k_bcomb(Cols in, const double *__restrict
   }
 }
 
-// Residuals of the Ritz pairs j < nr <= kResMax:
+// Residuals of the Ritz pairs j < nr <= NR:
 //   w_j = sum_k U[k + ld*j] C_k,  hw_j = sum_k U[k + ld*j] HC_k,
 //   r_j = hw_j - E_j w_j,
 // written to out.p[j] (when not null) as r_j, or with precond as the
 // diagonal step r_j / (E_j - d) (E_j - d - reg when |E_j - d| <= reg);
-// part[blk*nr + j] = this block's share of |r_j|^2.
+// part[blk*nr + j] = this block's share of |r_j|^2.  A thread forms two
+// consecutive elements, so a coefficient read from LDS serves two; NR is
+// the smallest of 4, 8 and 16 that holds nr (with 16 for every block the
+// sums over unused pairs made this 344 us on average over a three-root
+// solve of 1M elements, now 71 us).
+template <int NR>
 __global__ void __launch_bounds__(kBT) k_bresid(Cols C, Cols HC, const double *__restrict__ U, int ld,
                                                 const double *__restrict__ E, int nr,
                                                 const double *__restrict__ hii, double reg, int precond,
                                                 OutD out, size_t n, double *__restrict__ part) {
-  __shared__ double u[kResMax * kNbMax];
-  __shared__ double e[kResMax];
-  __shared__ double sh[4 * kResMax];
+  __shared__ double u[kNbMax * NR];
+  __shared__ double e[NR];
+  __shared__ double sh[4 * NR];
   const int nin = C.nd + C.nf;
-  for (int t = threadIdx.x; t < nin * nr; t += blockDim.x) {
-    const int k = t % nin, j = t / nin;
-    u[j * kNbMax + k] = U[k + (size_t)ld * j];
+  for (int t = threadIdx.x; t < nin * NR; t += blockDim.x) {
+    const int k = t / NR, j = t % NR;
+    u[t] = j < nr ? U[k + (size_t)ld * j] : 0.0;
   }
-  if (threadIdx.x < nr) e[threadIdx.x] = E[threadIdx.x];
+  if (threadIdx.x < NR) e[threadIdx.x] = (int)threadIdx.x < nr ? E[threadIdx.x] : 0.0;
   __syncthreads();
-  double ss[kResMax];
+  double ss[NR];
 #pragma unroll
-  for (int j = 0; j < kResMax; j++) ss[j] = 0.0;
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    double w[kResMax], hw[kResMax];
+  for (int j = 0; j < NR; j++) ss[j] = 0.0;
+  const size_t stride = 2 * (size_t)gridDim.x * blockDim.x;
+  for (size_t i = 2 * ((size_t)blockIdx.x * blockDim.x + threadIdx.x); i < n; i += stride) {
+    const bool two = i + 1 < n;
+    const size_t il = two ? i : (i > 0 ? i - 1 : 0);  // the pair that is loaded (the last one shifted back)
+    double w[NR][2], hw[NR][2];
 #pragma unroll
-    for (int j = 0; j < kResMax; j++) w[j] = hw[j] = 0.0;
-    for (int s = 0; s < 2; s++) {
-      const int ns = s ? C.nf : C.nd, off = s ? C.nd : 0;
-      for (int k0 = 0; k0 < ns; k0 += 4) {  // loads of 4 columns and their products issue together
-        const int m = min(4, ns - k0);
-        double cv[4], hv[4];
+    for (int j = 0; j < NR; j++) w[j][0] = w[j][1] = hw[j][0] = hw[j][1] = 0.0;
+    auto add = [&](const double (&cv)[2], const double (&hv)[2], int k) {
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-          const int k = q < m ? k0 + q : k0;
-          cv[q] = s ? (double)C.f[k][i] : C.d[k][i];
-          hv[q] = s ? (double)HC.f[k][i] : HC.d[k][i];
+      for (int j = 0; j < NR; j++) {
+        const double f = u[k * NR + j];
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+          w[j][q] += f * cv[q];
+          hw[j][q] += f * hv[q];
         }
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-          if (q < m) {
-            const double *uk = u + off + k0 + q;
-#pragma unroll
-            for (int j = 0; j < kResMax; j++)
-              if (j < nr) {
-                w[j] += uk[j * kNbMax] * cv[q];
-                hw[j] += uk[j * kNbMax] * hv[q];
-              }
-          }
+      }
+    };
+    if (n > 1) {
+#pragma unroll 4
+      for (int k = 0; k < C.nd; k++) {
+        double cv[2], hv[2];
+        load2(C.d[k] + il, cv);
+        load2(HC.d[k] + il, hv);
+        add(cv, hv, k);
+      }
+#pragma unroll 4
+      for (int k = 0; k < C.nf; k++) {
+        double cv[2], hv[2];
+        load2(C.f[k] + il, cv);
+        load2(HC.f[k] + il, hv);
+        add(cv, hv, C.nd + k);
+      }
+    } else {
+      for (int k = 0; k < nin; k++) {
+        const double cv[2] = {k < C.nd ? C.d[k][0] : (double)C.f[k - C.nd][0], 0.0};
+        const double hv[2] = {k < C.nd ? HC.d[k][0] : (double)HC.f[k - C.nd][0], 0.0};
+        add(cv, hv, k);
       }
     }
-    const double d = hii[i];
 #pragma unroll
-    for (int j = 0; j < kResMax; j++)
-      if (j < nr) {
-        const double r = hw[j] - e[j] * w[j];
-        ss[j] += r * r;
-        if (out.p[j]) {
-          double v = r;
-          if (precond) {
-            const double den = e[j] - d;
-            v = fabs(den) > reg ? r / den : r / (den - reg);
+    for (int q = 0; q < 2; q++) {
+      const size_t o = il + q;
+      if (o < i || o >= n) continue;  // the element before a shifted pair is another thread's
+      const double d = hii[o];
+#pragma unroll
+      for (int j = 0; j < NR; j++)
+        if (j < nr) {
+          const double r = hw[j][q] - e[j] * w[j][q];
+          ss[j] += r * r;
+          if (out.p[j]) {
+            double v = r;
+            if (precond) {
+              const double den = e[j] - d;
+              v = fabs(den) > reg ? r / den : r / (den - reg);
+            }
+            out.p[j][o] = v;
           }
-          out.p[j][i] = v;
         }
-      }
+    }
   }
 #pragma unroll
-  for (int j = 0; j < kResMax; j++) block_put(ss[j], j, sh, kResMax);
+  for (int j = 0; j < NR; j++) block_put(ss[j], j, sh, NR);
   __syncthreads();
   const int t = threadIdx.x;
-  if (t < nr) part[(size_t)blockIdx.x * nr + t] = ((sh[t] + sh[kResMax + t]) + sh[2 * kResMax + t]) +
-                                                  sh[3 * kResMax + t];
+  if (t < nr) part[(size_t)blockIdx.x * nr + t] = ((sh[t] + sh[NR + t]) + sh[2 * NR + t]) + sh[3 * NR + t];
 }
 
-// t_j -= sum_k coef[k*nv + j] X_k for j < nv <= kResMax (one classical
-// Gram-Schmidt pass with reduced coefficients)
+// t_j -= sum_k coef[k*nv + j] X_k for j < nv <= NV (one classical
+// Gram-Schmidt pass with reduced coefficients), NV as NR of k_bresid
+template <int NV>
 __global__ void __launch_bounds__(kBT) k_bsub(Cols X, const double *__restrict__ coef, int nv, OutD t,
                                               size_t n) {
-  __shared__ double cf[kNbMax * kResMax];
+  __shared__ double cf[kNbMax * NV];
   const int nx = X.nd + X.nf;
-  for (int q = threadIdx.x; q < nx * nv; q += blockDim.x) cf[q] = coef[q];
+  for (int q = threadIdx.x; q < nx * NV; q += blockDim.x) {
+    const int k = q / NV, j = q % NV;
+    cf[q] = j < nv ? coef[(size_t)k * nv + j] : 0.0;
+  }
   __syncthreads();
   const size_t stride = (size_t)gridDim.x * blockDim.x;
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    double acc[kResMax];
+    double acc[NV];
 #pragma unroll
-    for (int j = 0; j < kResMax; j++) acc[j] = j < nv ? t.p[j][i] : 0.0;
-    for (int s = 0; s < 2; s++) {
-      const int ns = s ? X.nf : X.nd, off = s ? X.nd : 0;
-      for (int k0 = 0; k0 < ns; k0 += 8) {
-        const int m = min(8, ns - k0);
-        double v[8];
+    for (int j = 0; j < NV; j++) acc[j] = j < nv ? t.p[j][i] : 0.0;
+    auto sub = [&](double v, int k) {
 #pragma unroll
-        for (int q = 0; q < 8; q++) {
-          const int k = q < m ? k0 + q : k0;
-          v[q] = s ? (double)X.f[k][i] : X.d[k][i];
-        }
+      for (int j = 0; j < NV; j++) acc[j] -= cf[k * NV + j] * v;
+    };
+#pragma unroll 8
+    for (int k = 0; k < X.nd; k++) sub(X.d[k][i], k);
+#pragma unroll 8
+    for (int k = 0; k < X.nf; k++) sub((double)X.f[k][i], X.nd + k);
 #pragma unroll
-        for (int q = 0; q < 8; q++)
-          if (q < m) {
-            const double *ck = cf + (size_t)(off + k0 + q) * nv;
-#pragma unroll
-            for (int j = 0; j < kResMax; j++)
-              if (j < nv) acc[j] -= ck[j] * v[q];
-          }
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < kResMax; j++)
+    for (int j = 0; j < NV; j++)
       if (j < nv) t.p[j][i] = acc[j];
   }
-}
-
-__global__ void __launch_bounds__(kBT) k_axpy_s(double *__restrict__ y, const double *__restrict__ x, double a,
-                                                size_t n) {
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) y[i] += a * x[i];
 }
 
 // dst = s * src, stored as TO
@@ -487,13 +604,16 @@ int davidson_block(Context &c, int nroots, int block, int max_it, double eps, do
   const int keep = keep_of(m);
   if (!c.blk_part) c.blk_part = (double *)dalloc(c, sizeof(double) * kBG * 2 * kNbMax * kResMax);
   if (!c.blk_small)
-    c.blk_small = (double *)dalloc(c, sizeof(double) * (2 * kNbMax * kNbMax + kNbMax * kResMax + 4 * kNbMax));
+    c.blk_small = (double *)dalloc(
+        c, sizeof(double) * (2 * kNbMax * kNbMax + kNbMax * kResMax + 4 * kNbMax + kResMax * kResMax + kResMax));
   double *U = c.blk_small;                           // kNbMax x kNbMax, column-major: all Ritz pairs, ascending
   double *Ed = U + kNbMax * kNbMax;                  // their values
   double *Us = Ed + kNbMax;                          // selected pairs (residuals, restarts)
   double *Es = Us + kNbMax * kNbMax;                 // their values
   double *coef = Es + kNbMax;                        // CGS coefficients (d x nv)
   double *nrm = coef + kNbMax * kResMax;             // residual norms^2
+  double *mref = nrm + 2 * kNbMax;                   // Gram matrix of one block's vectors (kResMax^2)
+  double *mnorm = mref + kResMax * kResMax;          // their squared norms in Gram-Schmidt (kResMax)
   double *part = c.blk_part;
   c.blk_m_used = m;
   c.blk_keep_used = keep;
@@ -548,9 +668,16 @@ int davidson_block(Context &c, int nroots, int block, int max_it, double eps, do
   // (device) and, when host is given, to the host
   auto gram = [&](const Cols &A, const Cols &B, double *dst, double *host) {
     const int na = A.nd + A.nf, nb = B.nd + B.nf, tot = na * nb;
-    hipLaunchKernelGGL(k_bgram, g, bt, 0, c.stream, A, B, N, part);
+    if (na > 64 || nb > 16) throw Error(3, "davidson_block: too many columns for one Gram pass");
+    // at least 4 chunks of elements per wavefront, so that the blocks'
+    // partial sums stay few against the columns that are read
+    const int nblk = (int)std::max<size_t>(1, std::min<size_t>(kGramBlocks, N / (4 * 4 * kGramChunk)));
+    const dim3 gg(nblk);
+    if (na <= 16) hipLaunchKernelGGL(k_bgram<1>, gg, bt, 0, c.stream, A, B, N, part);
+    else if (na <= 32) hipLaunchKernelGGL(k_bgram<2>, gg, bt, 0, c.stream, A, B, N, part);
+    else hipLaunchKernelGGL(k_bgram<4>, gg, bt, 0, c.stream, A, B, N, part);
     check_launch("k_bgram");
-    hipLaunchKernelGGL(k_bsum, dim3((tot + 255) / 256), dim3(256), 0, c.stream, tot, kBG, part, dst);
+    hipLaunchKernelGGL(k_bsum, dim3((tot + 31) / 32), dim3(256), 0, c.stream, tot, nblk, part, dst);
     check_launch("k_bsum");
     if (host) {
       SBDX_HIP(hipMemcpyAsync(host, dst, sizeof(double) * tot, hipMemcpyDeviceToHost, c.stream));
@@ -689,25 +816,39 @@ int davidson_block(Context &c, int nroots, int block, int max_it, double eps, do
     check_launch("k_store");
   };
   // modified Gram-Schmidt of the FP64 vectors vs among themselves; a
-  // vector whose squared norm falls to 1e-20 of ref[j] or to zero is
-  // dropped; returns the kept ones with their norms (not yet scaled)
-  auto mgs = [&](const std::vector<double *> &vs, const std::vector<double> &ref, std::vector<double *> &kept,
+  // vector whose squared norm falls to 1e-20 of ref[j] (its squared norm
+  // before the projections, device) or to zero is dropped; returns the kept
+  // ones with their norms (not yet scaled).  The projections run back to
+  // back on the stream (a dropped vector's norm is 0 there and projects
+  // nothing), the norms come to the host once at the end.
+  auto mgs = [&](const std::vector<double *> &vs, const double *ref, size_t ref_stride, std::vector<double *> &kept,
                  std::vector<double> &knorm, std::vector<int> &kidx) {
+    const int nv = (int)vs.size();
+    const int nblk = (int)std::max<size_t>(1, std::min<size_t>(kBG / 2, (N + 4 * kBT - 1) / (4 * kBT)));
+    double *p0 = part, *p1 = part + kBG;
+    for (int j = 0; j < nv; j++) {
+      hipLaunchKernelGGL(k_mgs_dot, dim3(nblk), bt, 0, c.stream, j > 0 ? vs[0] : vs[j], vs[j], N, p0);
+      check_launch("k_mgs_dot");
+      for (int k = 0; k < j; k++) {
+        hipLaunchKernelGGL(k_mgs_step, dim3(nblk), bt, 0, c.stream, vs[k], k + 1 < j ? vs[k + 1] : vs[j], vs[j], N,
+                           p0, nblk, mnorm + k, p1);
+        check_launch("k_mgs_step");
+        std::swap(p0, p1);
+      }
+      hipLaunchKernelGGL(k_mgs_norm, dim3(1), dim3(64), 0, c.stream, p0, nblk, ref + ref_stride * j, mnorm + j);
+      check_launch("k_mgs_norm");
+    }
+    double hn[kResMax];
+    SBDX_HIP(hipMemcpyAsync(hn, mnorm, sizeof(double) * nv, hipMemcpyDeviceToHost, c.stream));
+    SBDX_HIP(hipStreamSynchronize(c.stream));
     kept.clear();
     knorm.clear();
     kidx.clear();
-    for (size_t j = 0; j < vs.size(); j++) {
-      double *v = vs[j];
-      for (size_t k = 0; k < kept.size(); k++) {
-        const double o = device_dot(c, kept[k], v, N) / (knorm[k] * knorm[k]);
-        hipLaunchKernelGGL(k_axpy_s, g, bt, 0, c.stream, v, kept[k], -o, N);
-        check_launch("k_axpy_s");
-      }
-      const double n2 = device_dot(c, v, v, N);
-      if (!(n2 > 1e-20 * ref[j]) || !(n2 > 0.0)) continue;
-      kept.push_back(v);
-      knorm.push_back(std::sqrt(n2));
-      kidx.push_back((int)j);
+    for (int j = 0; j < nv; j++) {
+      if (!(hn[j] > 0.0)) continue;
+      kept.push_back(vs[j]);
+      knorm.push_back(std::sqrt(hn[j]));
+      kidx.push_back(j);
     }
   };
 
@@ -883,12 +1024,11 @@ int davidson_block(Context &c, int nroots, int block, int max_it, double eps, do
   }
   int d = 0;
   {
-    std::vector<double> ref(block);
-    for (int j = 0; j < block; j++) ref[j] = device_dot(c, Rs[j], Rs[j], N);
     std::vector<double *> kept, first(Rs.begin(), Rs.begin() + block);
     std::vector<double> kn;
     std::vector<int> ki;
-    mgs(first, ref, kept, kn, ki);
+    gram(dcols(first), dcols(first), mref, nullptr);  // squared norms on the diagonal
+    mgs(first, mref, (size_t)block + 1, kept, kn, ki);
     if ((int)kept.size() < nroots) throw Error(1, "davidson_block: start vectors are linearly dependent");
     for (size_t k = 0; k < kept.size(); k++) {
       par[k] = spar[ki[k]];
@@ -927,11 +1067,16 @@ int davidson_block(Context &c, int nroots, int block, int max_it, double eps, do
       upload_sel(P, d);
       OutD o{};
       for (int q = 0; q < nres; q++) o.p[q] = Rs[q];
-      hipLaunchKernelGGL(k_bresid, g, bt, 0, c.stream, cols(false, 0, d), cols(true, 0, d), (const double *)Us,
-                         kNbMax, (const double *)Es, nres, (const double *)c.hii, eps_reg, use_mlp_now ? 0 : 1, o,
-                         N, part);
+      const dim3 gr((unsigned)std::max<size_t>(1, std::min<size_t>(kBG, (N + 2 * kBT - 1) / (2 * kBT))));
+      auto go = [&](auto fn) {
+        hipLaunchKernelGGL(fn, gr, bt, 0, c.stream, cols(false, 0, d), cols(true, 0, d), (const double *)Us, kNbMax,
+                           (const double *)Es, nres, (const double *)c.hii, eps_reg, use_mlp_now ? 0 : 1, o, N, part);
+      };
+      if (nres <= 4) go(k_bresid<4>);
+      else if (nres <= 8) go(k_bresid<8>);
+      else go(k_bresid<16>);
       check_launch("k_bresid");
-      hipLaunchKernelGGL(k_bsum, dim3(1), dim3(256), 0, c.stream, nres, kBG, part, nrm);
+      hipLaunchKernelGGL(k_bsum, dim3(1), dim3(256), 0, c.stream, nres, (int)gr.x, part, nrm);
       check_launch("k_bsum");
       SBDX_HIP(hipMemcpyAsync(hR.data(), nrm, sizeof(double) * nres, hipMemcpyDeviceToHost, c.stream));
       SBDX_HIP(hipStreamSynchronize(c.stream));
@@ -1048,20 +1193,22 @@ int davidson_block(Context &c, int nroots, int block, int max_it, double eps, do
     {
       ProfScope ps(c, "blk_orth");
       const int ns = (int)sel.size();
-      std::vector<double> ref(ns);
-      for (int q = 0; q < ns; q++) ref[q] = device_dot(c, sel[q], sel[q], N);
+      gram(dcols(sel), dcols(sel), mref, nullptr);  // squared norms on the diagonal
       OutD t{};
       for (int q = 0; q < ns; q++) t.p[q] = sel[q];
       for (int pass = 0; pass < 2; pass++) {  // classical Gram-Schmidt, twice
         const Cols X = cols(false, 0, d);
         gram(X, dcols(sel), coef, nullptr);
-        hipLaunchKernelGGL(k_bsub, g, bt, 0, c.stream, X, (const double *)coef, ns, t, N);
+        auto go = [&](auto fn) { hipLaunchKernelGGL(fn, g, bt, 0, c.stream, X, (const double *)coef, ns, t, N); };
+        if (ns <= 4) go(k_bsub<4>);
+        else if (ns <= 8) go(k_bsub<8>);
+        else go(k_bsub<16>);
         check_launch("k_bsub");
       }
       std::vector<double *> kept;
       std::vector<double> kn;
       std::vector<int> ki;
-      mgs(sel, ref, kept, kn, ki);
+      mgs(sel, mref, (size_t)ns + 1, kept, kn, ki);
       nv = (int)kept.size();
       for (int q = 0; q < nv; q++) {
         // each correction stays in its Ritz pair's sector; projecting it
