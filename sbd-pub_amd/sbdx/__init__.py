@@ -386,7 +386,12 @@ class TPBOperator:
         diagonal elements).  Returns (energies, W, products, converged)."""
         if W0 is None:
             W0 = np.zeros((nroots, self.ndet))
-            order = np.argsort(self.make_diag(), kind="stable")[:nroots]
+            # the nroots lowest elements, ties by index: only those up to the
+            # nroots-th value are sorted
+            hii = self.make_diag()
+            k = min(nroots, self.ndet)
+            low = np.flatnonzero(hii <= np.partition(hii, k - 1)[k - 1])
+            order = low[np.argsort(hii[low], kind="stable")][:k]
             for j, i in enumerate(order):
                 W0[j, i] = 1.0
         W = np.ascontiguousarray(W0, dtype=np.float64).reshape(nroots, self.ndet).copy()
