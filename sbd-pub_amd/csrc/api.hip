@@ -209,12 +209,14 @@ static Context *create_core(int L, std::vector<uint64_t> as, std::vector<uint64_
     }
     build_spin_tables(c, c.A, as);
     build_singles_ell(c, c.A);
+    build_rdm_tables(c, c.A, as, true, as == bs);
     if (as == bs) {
       c.B = c.A;
       c.B.alias = true;
     } else {
       build_spin_tables(c, c.B, bs);
       build_singles_ell(c, c.B);
+      build_rdm_tables(c, c.B, bs, false, true);
     }
     c.hii = (double *)dalloc(c, sizeof(double) * c.N);
     compute_diag(c);

@@ -83,15 +83,31 @@ struct SpinTables {
   // n < 8192.
   uint32_t *ell3 = nullptr;
   bool has_ell3 = false;
-  // The singles grouped by pair index pq (for the RDM's mixed term):
-  // pm_off[K+1]; pm_ent = bra | ket << 32 | (sign<0) << 63, rows ascending
-  // within a pair.  The same grouping as a sliced ELL over the pair bins
-  // (n < 32768): bins by entry count into slices of 64 lanes, entry k of
-  // lane l of slice s at pb[pb_off[s] + 64 k + l] = bra | ket << 15 |
-  // (sign<0) << 31 (padding: bra = ket = n), pb_len[s] entries per lane,
-  // pb_perm[64 s + l] the lane's bin (0xffffffff past K).
-  uint64_t *pm_off = nullptr;
-  uint64_t *pm_ent = nullptr;
+  // Tables of the RDM's mixed term (build_rdm_tables).
+  // As the alpha set: the singles with p > q and the identity pairs (I, I)
+  // of p == q, grouped by pair index: ra_ent = I | J << 32 | (sign<0) << 63
+  // and work items ra_item = (pair index, first entry, last entry, 0).
+  uint64_t *ra_ent = nullptr;
+  uint4 *ra_item = nullptr;
+  int ra_nitem = 0;
+  // As the beta set (n < 32768): blocks of singles as columns of orbitals.
+  // A particle column is a string k with one electron less: its members are
+  // the strings k + u, and every pair of members (k + u, k + v) is a single;
+  // a hole column is a string with one electron more, members K - u.  Four
+  // columns make a step; the word of lane l of step s, rc_tab[64 s + l],
+  // holds for column 4 s + l / 16 and tile t the member of orbital 16 t + l
+  // % 16 in bits 16 t .. 16 t + 15: string | (sign<0) << 15, or n when there
+  // is none.  A column whose members lie in one tile is taken over that tile
+  // alone, any other over all tiles; steps of one kind and tile choice are
+  // contiguous: rc_range[i] = (first step, last step, tile or -1, hole).
+  uint64_t *rc_tab = nullptr;
+  int4 rc_range[24];
+  int rc_nrange = 0;
+  // The singles that no column covers, by pair index rs: each pair's entries
+  // in runs of at most one length, chosen to make up to 8 slices of 64 runs;
+  // entry k of lane l of slice s at pb[pb_off[s] + 64 k + l] = bra | ket <<
+  // 15 | (sign<0) << 31 (padding: bra = ket = n), pb_len[s] entries per
+  // lane, pb_perm[64 s + l] the lane's pair (0xffffffff for none).
   uint32_t *pb = nullptr, *pb_len = nullptr, *pb_perm = nullptr;
   uint64_t *pb_off = nullptr;
   int pb_nslice = 0;
@@ -314,6 +330,7 @@ void check_launch(const char *what);
 void build_spin_tables(Context &c, SpinTables &t, const std::vector<uint64_t> &strs);
 void build_singles_ell(Context &c, SpinTables &t);
 void build_singles_ell_parts(Context &c, SpinTables &t, int nparts);
+void build_rdm_tables(Context &c, SpinTables &t, const std::vector<uint64_t> &strs, bool as_alpha, bool as_beta);
 void compute_diag(Context &c);
 void sign_convert(Context &c, const double *in, double *out);      // out = S*in
 void sign_convert_noprof(Context &c, const double *in, double *out);  // out = S*in, no profiling events

@@ -6,12 +6,13 @@
 // reference, w_bra*w_ket*(interleaved sign), equals w'_bra*w'_ket times the
 // one-spin table sign (alpha single, beta single, or their product for the
 // mixed term), so the per-pair sums below factor over the other spin:
-//   ZeroDiff  -> row/column sums of w'^2 and their occupation-weighted sums
-//   OneDiff   -> per single pair: T = s*sum_m w'[I,m]w'[J,m] and
-//                Tk[k] = s*sum_m w'[I,m]w'[J,m] n_k(m) (other-spin spectators)
-//   TwoDiff   -> per same-spin double pair: T; mixed: T[pq][rs] summed over
-//                all (alpha single, beta single) pairs, then placed with the
-//                reference's spin-orbital ordering rules.
+//   same spin -> dots of the rows of w' (strings of this spin): rho[I] =
+//                <I|I>, G[I,J] per single and double pair of strings
+//   two spins -> T[pq][rs] = sum over the alpha pairs (I, J) of pq and the
+//                beta pairs (i, j) of rs of s_a s_b w'[I,i] w'[J,j], where the
+//                pairs of an orbital with itself (p == q: I = J with p
+//                occupied) stand for the occupation numbers; then placed with
+//                the reference's spin-orbital ordering rules.
 #include <memory>
 #include <mutex>
 #include <string>
@@ -54,115 +55,72 @@ __device__ __forceinline__ int row_of(const uint64_t *off, int n, uint64_t e) {
   return lo;
 }
 
-// Per row r of w (rows x M): rho[r] = sum_m w^2 and mrow[r][k] = sum_m w^2 n_k(m)
-__global__ void __launch_bounds__(256) k_rdm_diag_rows(int M, int L, const uint64_t *__restrict__ ostr,
-                                                       const double *__restrict__ w,
-                                                       double *__restrict__ rho,
-                                                       double *__restrict__ mrow) {
+// Per row r of w (rows x M): rho[r] = sum_m w^2
+__global__ void __launch_bounds__(256) k_rdm_diag_rows(int M, const double *__restrict__ w,
+                                                       double *__restrict__ rho) {
   __shared__ double sh[256];
-  __shared__ double acc[64];
   const int r = blockIdx.x;
-  if (threadIdx.x < 64) acc[threadIdx.x] = 0.0;
-  __syncthreads();
   double s = 0.0;
   for (int m = threadIdx.x; m < M; m += 256) {
     const double v = w[(size_t)r * M + m];
-    const double v2 = v * v;
-    s += v2;
-    if (mrow) {
-      uint64_t occ = ostr[m];
-      while (occ) {
-        const int k = __ffsll((unsigned long long)occ) - 1;
-        occ &= occ - 1;
-        atomicAdd(&acc[k], v2);
-      }
-    }
+    s += v * v;
   }
   const double t = blk_sum256(s, sh);
   if (threadIdx.x == 0) rho[r] = t;
-  if (mrow && threadIdx.x < L) mrow[(size_t)r * L + threadIdx.x] = acc[threadIdx.x];
 }
 
-// ZeroDiff contributions from rho (both spins) and M[p][r] = sum_I n_p(I) mrow[I][r]
-__global__ void k_rdm_diag_scatter(int L, int na, int nb, const uint64_t *__restrict__ astr,
-                                   const uint64_t *__restrict__ bstr,
-                                   const double *__restrict__ rho_a, const double *__restrict__ rho_b,
-                                   const double *__restrict__ mrow, double *__restrict__ one,
-                                   double *__restrict__ two) {
-  // one thread per (p, r) pair of orbitals
-  const int p = blockIdx.x, r = threadIdx.x;
-  if (r >= L) return;
-  const size_t L2 = (size_t)L * L, L4 = L2 * L2;
-  double m = 0.0, aa = 0.0, bb = 0.0;
-  for (int I = 0; I < na; I++) {
-    const uint64_t s = astr[I];
-    if ((s >> p) & 1ull) {
-      m += mrow[(size_t)I * L + r];
-      if (r != p && ((s >> r) & 1ull)) aa += rho_a[I];
+// Same-spin ZeroDiff of one spin: rho[r * rstride] weights string r.
+// one[p,p] += rho n_p and, for p != r, two[p,r,p,r] += rho n_p n_r and
+// two[p,r,r,p] -= the same.  A wavefront walks kDiagStr strings, lane = r;
+// the sums over the strings are collected in LDS (no two lanes of a
+// wavefront share an element).  One block per orbital walking all strings
+// was a serial chain of loads: 3.7 ms for 8000 strings.
+constexpr int kDiagStr = 32;
+__global__ void __launch_bounds__(256) k_rdm_diag_pairs(int n, int L, int spin, const uint64_t *__restrict__ str,
+                                                        const double *__restrict__ rho, size_t rstride,
+                                                        double *__restrict__ one, double *__restrict__ two) {
+  extern __shared__ double lds[];  // [L][L]
+  const int L2 = L * L;
+  for (int i = threadIdx.x; i < L2; i += 256) lds[i] = 0.0;
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const int r0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * kDiagStr;
+  for (int k = 0; k < kDiagStr && r0 + k < n; k++) {
+    const uint64_t s = str[r0 + k];
+    const double v = rho[(size_t)(r0 + k) * rstride];
+    if ((s >> lane) & 1ull)
+      for (uint64_t o = s; o; o &= o - 1) atomicAdd(&lds[(__ffsll((unsigned long long)o) - 1) * L + lane], v);
+  }
+  __syncthreads();
+  const size_t K = (size_t)L2, bs = (size_t)(3 * spin) * K * K;
+  for (int i = threadIdx.x; i < L2; i += 256) {
+    const double v = lds[i];
+    if (v == 0.0) continue;
+    const size_t p = i / L, r = i % L;
+    if (p == r) {
+      atomicAdd(&one[spin * K + p + L * p], v);
+    } else {
+      atomicAdd(&two[bs + p + L * r + K * (p + L * r)], v);
+      atomicAdd(&two[bs + p + L * r + K * (r + L * p)], -v);
     }
   }
-  for (int ib = 0; ib < nb; ib++) {
-    const uint64_t s = bstr[ib];
-    if (((s >> p) & 1ull) && r != p && ((s >> r) & 1ull)) bb += rho_b[ib];
-  }
-  // alpha-beta pairs: two[2][p,r,p,r] and two[1][r,p,r,p]
-  two[2 * L4 + p + L * r + L2 * p + L2 * L * r] += m;
-  two[1 * L4 + r + L * p + L2 * r + L2 * L * p] += m;
-  // same-spin ordered pairs (p,r), p != r: [p,r,p,r] += w^2 and [p,r,r,p] -= w^2
-  if (r != p) {
-    two[0 * L4 + p + L * r + L2 * p + L2 * L * r] += aa;
-    two[0 * L4 + p + L * r + L2 * r + L2 * L * p] -= aa;
-    two[3 * L4 + p + L * r + L2 * p + L2 * L * r] += bb;
-    two[3 * L4 + p + L * r + L2 * r + L2 * L * p] -= bb;
-  }
-  if (r == 0) {
-    double da = 0.0, db = 0.0;
-    for (int I = 0; I < na; I++)
-      if ((astr[I] >> p) & 1ull) da += rho_a[I];
-    for (int ib = 0; ib < nb; ib++)
-      if ((bstr[ib] >> p) & 1ull) db += rho_b[ib];
-    one[p + L * p] += da;
-    one[L2 + p + L * p] += db;
-  }
 }
 
-// Single pairs of one spin: block per pair e; rows of w are this spin's strings.
-//   out[e*(L+1)]     = s * sum_m w[I,m] w[J,m]
-//   out[e*(L+1)+1+k] = s * sum_m w[I,m] w[J,m] n_k(m)    (other-spin strings)
-// Pairs e0 <= e < e1 only; out holds pair e at (e - e0).
-__global__ void __launch_bounds__(256) k_rdm_single_pairs(int n, int M, int L, uint64_t e0, uint64_t e1,
+// Single pairs of one spin, e0 <= e < e1: out[e - e0] = s * sum_m w[I,m] w[J,m]
+__global__ void __launch_bounds__(256) k_rdm_single_pairs(int n, int M, uint64_t e0, uint64_t e1,
                                                           const uint64_t *__restrict__ s_off,
                                                           const uint64_t *__restrict__ s_ent,
-                                                          const uint64_t *__restrict__ ostr,
                                                           const double *__restrict__ w,
                                                           double *__restrict__ out) {
   __shared__ double sh[256];
-  __shared__ double acc[64];
   for (uint64_t e = e0 + blockIdx.x; e < e1; e += gridDim.x) {
-  const int I = row_of(s_off, n, e);
-  const uint64_t ent = s_ent[e];
-  const size_t J = (uint32_t)(ent & 0xffffffffull);
-  const double sg = (ent >> 63) ? -1.0 : 1.0;
-  if (threadIdx.x < 64) acc[threadIdx.x] = 0.0;
-  __syncthreads();
-  double s = 0.0;
-  for (int m = threadIdx.x; m < M; m += 256) {
-    const double v = w[(size_t)I * M + m] * w[J * M + m];
-    s += v;
-    if (v != 0.0) {
-      uint64_t occ = ostr[m];
-      while (occ) {
-        const int k = __ffsll((unsigned long long)occ) - 1;
-        occ &= occ - 1;
-        atomicAdd(&acc[k], v);
-      }
-    }
-  }
-  const double t = blk_sum256(s, sh);
-  double *o = out + (e - e0) * (size_t)(L + 1);
-  if (threadIdx.x == 0) o[0] = sg * t;
-  if (threadIdx.x < L) o[1 + threadIdx.x] = sg * acc[threadIdx.x];
-  __syncthreads();
+    const int I = row_of(s_off, n, e);
+    const uint64_t ent = s_ent[e];
+    const size_t J = (uint32_t)(ent & 0xffffffffull);
+    double s = 0.0;
+    for (int m = threadIdx.x; m < M; m += 256) s += w[(size_t)I * M + m] * w[J * M + m];
+    const double t = blk_sum256(s, sh);
+    if (threadIdx.x == 0) out[e - e0] = (ent >> 63) ? -t : t;
   }
 }
 
@@ -214,22 +172,29 @@ __global__ void __launch_bounds__(256) k_rdm_double_gram(int n, uint64_t e0, uin
   out[e - e0] = sg * G[(size_t)I * n + J];
 }
 
-// OneDiff scatter for the single pairs e0 <= e < e1 of one spin (si =
-// spin); T holds pair e at (e - e0).
+// Same-spin OneDiff scatter for the single pairs e0 <= e < e1 of one spin:
+// the pair's dot product from T (pair e at (e - e0)) or, when T is null,
+// with its sign from the Gram matrix G.
 __global__ void k_rdm_single_scatter(int n, int L, int spin, uint64_t e0, uint64_t e1,
                                      const uint64_t *__restrict__ s_off,
                                      const uint64_t *__restrict__ s_ent,
                                      const uint64_t *__restrict__ str,
-                                     const double *__restrict__ T, double *__restrict__ one,
-                                     double *__restrict__ two) {
+                                     const double *__restrict__ T, const double *__restrict__ G,
+                                     double *__restrict__ one, double *__restrict__ two) {
   const uint64_t e = e0 + (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= e1) return;
   const size_t L2 = (size_t)L * L, L4 = L2 * L2, L3 = L2 * L;
   const int I = row_of(s_off, n, e);
-  const uint32_t pq = (uint32_t)((s_ent[e] >> 32) & 0x7fffffffull);
+  const uint64_t ent = s_ent[e];
+  const uint32_t pq = (uint32_t)((ent >> 32) & 0x7fffffffull);
   const int p = pq / L, q = pq % L;  // p = bra-only (cr), q = ket-only (an)
-  const double *t = T + (e - e0) * (size_t)(L + 1);
-  const double t0 = t[0];
+  double t0;
+  if (T) {
+    t0 = T[e - e0];
+  } else {
+    const double g = G[(size_t)I * n + (uint32_t)(ent & 0xffffffffull)];
+    t0 = (ent >> 63) ? -g : g;
+  }
   atomicAdd(&one[spin * L2 + p + (size_t)L * q], t0);
   const size_t bs = (size_t)(3 * spin) * L4;  // same-spin block
   uint64_t occ = str[I];
@@ -241,14 +206,6 @@ __global__ void k_rdm_single_scatter(int n, int L, int spin, uint64_t e0, uint64
     atomicAdd(&two[bs + k + L * q + L2 * k + L3 * p], t0);
     atomicAdd(&two[bs + q + L * k + L2 * k + L3 * p], -t0);
     atomicAdd(&two[bs + k + L * q + L2 * p + L3 * k], -t0);
-  }
-  const size_t b1 = (size_t)(spin + 2 * (1 - spin)) * L4;  // [si + 2 sj]
-  const size_t b2 = (size_t)((1 - spin) + 2 * spin) * L4;  // [sj + 2 si]
-  for (int k = 0; k < L; k++) {
-    const double tk = t[1 + k];
-    if (tk == 0.0) continue;
-    atomicAdd(&two[b1 + q + L * k + L2 * p + L3 * k], tk);
-    atomicAdd(&two[b2 + k + L * q + L2 * k + L3 * p], tk);
   }
 }
 
@@ -270,149 +227,307 @@ __global__ void k_rdm_double_scatter(int L, int spin, uint64_t e0, uint64_t e1,
   atomicAdd(&two[bs + b + L * a + L2 * (i + L * j)], -t);
 }
 
-// Mixed term: Tm[pq*K + rs] += sum_{e in S_a(I)} s_e sum_{ib} w[I,ib] sum_{f in S_b(ib)} s_f w[J_e, jb_f]
-template <int NT>
-__global__ void __launch_bounds__(1024) k_rdm_mixed(int nb, int K, const uint64_t *__restrict__ a_off,
-                                                    const uint64_t *__restrict__ a_ent,
-                                                    const uint64_t *__restrict__ b_off,
-                                                    const uint64_t *__restrict__ b_ent,
-                                                    const double *__restrict__ w,
-                                                    double *__restrict__ Tm) {
-  extern __shared__ double lds[];
-  double *wrow = lds;
-  double *trow = lds + nb;
-  const int I = blockIdx.x;
-  const int tid = threadIdx.x;
-  double wi[NT];
+// Two-spin term.  A block takes one work item: an alpha pair index pq (p >=
+// q; T[qp][sr] = T[pq][rs] gives the rest) and a run of its alpha pairs
+// (I, J, s_a).  Per alpha pair the rows x = s_a w[I,:] and y = w[J,:] are
+// staged in LDS, each followed by a zero, and
+//   T[pq][u v] += sum over the columns k of s_u s_v x[k + u] y[k + v]
+// is a product of two matrices gathered from them, (orbitals x columns)
+// times (columns x orbitals), on the FP64 matrix cores: a step of four
+// columns is one 16x16x4 operand per tile of 16 orbitals, lane l holding
+// orbital l % 16 of column l / 16 (SpinTables::rc_tab), read from LDS at the
+// table's string with the table's sign.  A hole column's members are K - u
+// and its element is -s_u s_v y[K - u] x[K - v].  The accumulators stay in
+// registers over the item's alpha pairs.  The singles outside the columns
+// (pb) are summed entry by entry, one pair bin per lane, into LDS.  The
+// occupation numbers, T[pq][kk] = sum_i n_k(i) x[i] y[i], are taken once per
+// item from the sum over its alpha pairs of x[i] y[i].  The item's row of T
+// is collected in LDS and added to T with atomics.
+// The columns hold several times more products than there are singles, at
+// many times the rate: the entry-by-entry form (436k multiply-adds per alpha
+// pair of a 8000-string set at 36 orbitals, two random 8-byte LDS reads
+// each, and the alpha pairs of q > p as well) and the occupation sums of
+// every single pair took 261 + 184 ms for 8000 x 8000 strings; this kernel
+// takes 46 ms (2583 x 1387 at 29 orbitals: 10.3 -> 1.9 ms, 500 x 500 at 16:
+// 1.16 -> 0.13 ms).  What bounds it there is the chain of an alpha pair
+// (stage two rows, barrier, steps): with 130 KB staged one block of 8
+// wavefronts fits in a CU; the matrix instructions alone would take 18 ms.
+// Two wavefronts per SIMD (512 threads) leave 256 registers each for up to 9
+// tiles of accumulators (twice, as the compiler pipelines them), the x y
+// products and the gathers; with 4 tiles of orbitals a block takes two of
+// them as rows (UT) and blockIdx.y says which.
+constexpr int kMmThreads = 512;
+constexpr int kMmWaves = kMmThreads / 64;
+constexpr int kMmRho = 16;  // x y products per thread kept in registers (ROWS): nb <= 8192
+
+typedef double d4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ double signed_by(double v, uint32_t high) {
+  return __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, v) ^ ((uint64_t)high << 32));
+}
+// A row of w: staged in LDS with a zero behind it (LDS), or where it is, n
+// values long (no member: string n, a zero).
+template <bool LDS>
+struct Row {
+  const double *p;
+  uint32_t n;
+  __device__ __forceinline__ double at(uint32_t i) const { return LDS || i < n ? p[i] : 0.0; }
+};
+// the value of tile t's member in the row, with its sign (and `flip`)
+template <bool LDS>
+__device__ __forceinline__ double member(const Row<LDS> &row, uint64_t w, int t, uint32_t flip) {
+  const uint32_t v = (uint32_t)(w >> (16 * t));
+  return signed_by(row.at(v & 0x7fffu), ((v & 0x8000u) << 16) ^ flip);
+}
+
+// The steps s0 + wave, + waves, ... < s1 of columns over all tiles: two
+// steps at a time, one's gathers under the other's matrix instructions, the
+// table words of the next two in flight.
+template <int NT, int UT, bool LDS>
+__device__ __forceinline__ void rdm_steps_all(d4 (&acc)[UT][NT], const uint64_t *__restrict__ tab, int s0, int s1,
+                                              int u0, Row<LDS> a_row, Row<LDS> b_row, uint32_t flip) {
+  const int lane = threadIdx.x & 63;
+  int s = s0 + (int)(threadIdx.x >> 6);
+  if (s >= s1) return;
+  auto word = [&](int q) { return tab[(size_t)64 * (q < s1 ? q : s) + lane]; };
+  auto gather = [&](uint64_t w, double (&a)[UT], double (&b)[NT]) {
 #pragma unroll
-  for (int t = 0; t < NT; t++) {
-    const int ib = tid + t * 1024;
-    wi[t] = ib < nb ? w[(size_t)I * nb + ib] : 0.0;
+    for (int t = 0; t < UT; t++) a[t] = member(a_row, w, u0 + t, flip);
+#pragma unroll
+    for (int t = 0; t < NT; t++) b[t] = member(b_row, w, t, 0u);
+  };
+  auto mac = [&](const double (&a)[UT], const double (&b)[NT]) {
+#pragma unroll
+    for (int i = 0; i < UT; i++)
+#pragma unroll
+      for (int j = 0; j < NT; j++) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
+  };
+  uint64_t w0 = word(s), w1 = word(s + kMmWaves);
+  for (; s + kMmWaves < s1; s += 2 * kMmWaves) {
+    double a0[UT], b0[NT], a1[UT], b1[NT];
+    gather(w0, a0, b0);
+    gather(w1, a1, b1);
+    w0 = word(s + 2 * kMmWaves);
+    w1 = word(s + 3 * kMmWaves);
+    mac(a0, b0);
+    mac(a1, b1);
   }
-  for (uint64_t e = a_off[I]; e < a_off[I + 1]; e++) {
-    const uint64_t ent = a_ent[e];
-    const size_t J = (uint32_t)(ent & 0xffffffffull);
-    const double sa = (ent >> 63) ? -1.0 : 1.0;
-    const size_t pq = (ent >> 32) & 0x7fffffffull;
-    __syncthreads();
-    for (int i = tid; i < nb; i += 1024) wrow[i] = w[J * nb + i];
-    for (int i = tid; i < K; i += 1024) trow[i] = 0.0;
-    __syncthreads();
-#pragma unroll
-    for (int t = 0; t < NT; t++) {
-      const int ib = tid + t * 1024;
-      if (ib < nb && wi[t] != 0.0) {
-        for (uint64_t f = b_off[ib]; f < b_off[ib + 1]; f++) {
-          const uint64_t be = b_ent[f];
-          const double v = wi[t] * wrow[(uint32_t)(be & 0xffffffffull)];
-          atomicAdd(&trow[(be >> 32) & 0x7fffffffull], (be >> 63) ? -v : v);
-        }
-      }
-    }
-    __syncthreads();
-    for (int i = tid; i < K; i += 1024) {
-      const double v = trow[i];
-      if (v != 0.0) atomicAdd(&Tm[pq * K + i], sa * v);
-    }
+  if (s < s1) {
+    double a0[UT], b0[NT];
+    gather(w0, a0, b0);
+    mac(a0, b0);
   }
 }
 
-// The same mixed term with no atomics: one block per alpha pair index pq
-// loops over the alpha singles (I -> J, s_a) with that pq (a_pm), staging
-// x[I,:] and x[J,:] in LDS (each followed by a zero).  The beta singles are
-// grouped by their pair index rs into bins laid out as a sliced ELL (b_pb:
-// 64 bins per slice, entry k of lane l at b_off[s] + 64 k + l, packed
-// ib | jb << 15 | (s_b<0) << 31, padding reading the zeros): wavefront w
-// owns slices w, w + 16, ..., each lane one bin, and adds s_a times
-// sum s_b x[I,ib] x[J,jb] over its bin to a register; after the last alpha
-// single the registers are Tm's row pq.  Table loads are coalesced (one
-// 256-byte row per wavefront step) and no two lanes share a bin.  Needs
-// nb < 8192 (the staged rows: at most 8 values per thread) and at most
-// 16 * MS slices.
-template <int MS>
-__global__ void __launch_bounds__(1024) k_rdm_mixed_pq(int nb, int K, int nslice,
-                                                       const uint64_t *__restrict__ a_off,
-                                                       const uint64_t *__restrict__ a_ent,
-                                                       const uint32_t *__restrict__ b_pb,
-                                                       const uint64_t *__restrict__ b_off,
-                                                       const uint32_t *__restrict__ b_len,
-                                                       const uint32_t *__restrict__ b_perm,
-                                                       const double *__restrict__ w, double *__restrict__ Tm) {
-  extern __shared__ double lds[];
-  double *xI = lds, *xJ = lds + nb + 1;
-  const int pq = blockIdx.x;
-  const uint64_t e0 = a_off[pq], e1 = a_off[pq + 1];
-  if (e0 == e1) return;  // uniform per block, before any barrier (Tm's row stays 0)
-  const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
-  double acc[MS];
+// The same over one tile t: one matrix instruction per step, so four steps
+// at a time into two accumulators (an instruction waits for the sum it adds
+// to).
+template <bool LDS>
+__device__ __forceinline__ void rdm_steps_one(d4 &acc, const uint64_t *__restrict__ tab, int s0, int s1, int t,
+                                              Row<LDS> a_row, Row<LDS> b_row, uint32_t flip) {
+  const int lane = threadIdx.x & 63;
+  int s = s0 + (int)(threadIdx.x >> 6);
+  if (s >= s1) return;
+  auto word = [&](int q) { return tab[(size_t)64 * (q < s1 ? q : s) + lane]; };
+  d4 odd = {0.0, 0.0, 0.0, 0.0};
+  uint64_t w[4];
 #pragma unroll
-  for (int j = 0; j < MS; j++) acc[j] = 0.0;
-  for (uint64_t e = e0; e < e1; e++) {
-    const uint64_t ent = a_ent[e];
-    const size_t I = (uint32_t)(ent & 0xffffffffull);
-    const size_t J = (uint32_t)((ent >> 32) & 0x7fffffffull);
-    const double sa = (ent >> 63) ? -1.0 : 1.0;
-    // both rows loaded before the barrier that ends the previous alpha
-    // single's reads (nb + 1 <= 8192: at most 8 values per thread and row)
-    double vi[8], vj[8];
+  for (int q = 0; q < 4; q++) w[q] = word(s + q * kMmWaves);
+  for (; s + 3 * kMmWaves < s1; s += 4 * kMmWaves) {
+    double a[4], b[4];
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-      const int i = tid + k * 1024;
-      vi[k] = i < nb ? w[I * nb + i] : 0.0;
-      vj[k] = i < nb ? w[J * nb + i] : 0.0;
+    for (int q = 0; q < 4; q++) {
+      a[q] = member(a_row, w[q], t, flip);
+      b[q] = member(b_row, w[q], t, 0u);
     }
-    __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-      const int i = tid + k * 1024;
-      if (i <= nb) {
-        xI[i] = vi[k];
-        xJ[i] = vj[k];
+    for (int q = 0; q < 4; q++) w[q] = word(s + (4 + q) * kMmWaves);
+#pragma unroll
+    for (int q = 0; q < 4; q += 2) {
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q], b[q], acc, 0, 0, 0);
+      odd = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q + 1], b[q + 1], odd, 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 3; q++)
+    if (s + q * kMmWaves < s1)
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(member(a_row, w[q], t, flip), member(b_row, w[q], t, 0u), acc, 0, 0,
+                                                 0);
+  acc += odd;
+}
+
+struct RdmRanges {
+  int4 r[24];
+  int n;
+};
+
+// ROWS: the two rows in LDS and the x y sums in registers; otherwise (rows
+// too long) both rows are read where they are and the sums are in LDS.
+template <int NT, int UT, bool ROWS>
+__global__ void __launch_bounds__(kMmThreads) k_rdm_mixed(int nb, int K, int L, const uint4 *__restrict__ items,
+                                                          const uint64_t *__restrict__ a_ent, RdmRanges rg,
+                                                          const uint64_t *__restrict__ tab, int nslice,
+                                                          const uint32_t *__restrict__ pb,
+                                                          const uint64_t *__restrict__ pb_off,
+                                                          const uint32_t *__restrict__ pb_len,
+                                                          const uint32_t *__restrict__ pb_perm,
+                                                          const uint64_t *__restrict__ b_str,
+                                                          const double *__restrict__ w, double *__restrict__ Tm) {
+  extern __shared__ double lds[];
+  double *trow = lds;             // [K]
+  double *xs = lds + K;           // ROWS: x then a zero; else the x y sums
+  double *ys = xs + nb + 1;       // ROWS: y then a zero
+  const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
+  const int u0 = UT < NT ? (int)blockIdx.y * UT : 0;
+  const bool rest = u0 == 0;  // entries outside the columns and occupation numbers: once
+  const uint4 it = items[blockIdx.x];
+  for (int i = tid; i < K; i += kMmThreads) trow[i] = 0.0;
+  if (!ROWS)
+    for (int i = tid; i < nb; i += kMmThreads) xs[i] = 0.0;
+  __syncthreads();
+  d4 acc[UT][NT];
+#pragma unroll
+  for (int i = 0; i < UT; i++)
+#pragma unroll
+    for (int j = 0; j < NT; j++) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
+  double rho[ROWS ? kMmRho : 1];
+#pragma unroll
+  for (int k = 0; k < (ROWS ? kMmRho : 1); k++) rho[k] = 0.0;
+  for (uint32_t e = it.y; e < it.z; e++) {
+    const uint64_t ent = a_ent[e];
+    const double *xg = w + (size_t)(uint32_t)(ent & 0xffffffffull) * nb;
+    const double *yg = w + (size_t)((ent >> 32) & 0x7fffffffull) * nb;
+    const uint32_t neg = (uint32_t)(ent >> 63) << 31;
+    const Row<ROWS> x = {ROWS ? xs : xg, (uint32_t)nb}, y = {ROWS ? ys : yg, (uint32_t)nb};
+    if (ROWS) {
+      // half a row of each at a time, every load before the first store; the
+      // first half is loaded before the barrier that ends the previous
+      // pair's reads (nb < 8192: two halves of 8 values per thread)
+      double vx[8], vy[8];
+      auto load = [&](int i0) {
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+          const int i = i0 + k * kMmThreads;
+          vx[k] = i < nb ? signed_by(xg[i], neg) : 0.0;
+          vy[k] = i < nb ? yg[i] : 0.0;
+        }
+      };
+      auto store = [&](int i0) {
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+          const int i = i0 + k * kMmThreads;
+          if (i <= nb) {
+            xs[i] = vx[k];
+            ys[i] = vy[k];
+          }
+        }
+      };
+      load(tid);
+      __syncthreads();
+      store(tid);
+      if (nb >= 8 * kMmThreads) {
+        load(tid + 8 * kMmThreads);
+        store(tid + 8 * kMmThreads);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < kMmRho; k++) {
+        const int i = tid + k * kMmThreads;
+        if (i < nb) rho[k] += xs[i] * ys[i];
+      }
+    } else {
+      for (int i = tid; i < nb; i += kMmThreads) xs[i] += signed_by(xg[i], neg) * yg[i];
+    }
+    const uint32_t sx = ROWS ? 0u : neg;  // the alpha sign, where x is not staged with it
+    for (int q = 0; q < rg.n; q++) {
+      const int4 r = rg.r[q];
+      const Row<ROWS> ar = r.w ? y : x, br = r.w ? x : y;
+      const uint32_t flip = sx ^ (r.w ? 0x80000000u : 0u);
+      if (r.z < 0) {
+        rdm_steps_all<NT, UT, ROWS>(acc, tab, r.x, r.y, u0, ar, br, flip);
+      } else if (r.z >= u0 && r.z < u0 + UT) {
+        const int t = r.z;
+        if (t == 0) rdm_steps_one<ROWS>(acc[0][0], tab, r.x, r.y, t, ar, br, flip);
+        if constexpr (NT > 1)
+          if (t == 1) rdm_steps_one<ROWS>(acc[1][1], tab, r.x, r.y, t, ar, br, flip);
+        if constexpr (NT > 2)
+          if (t == 2) rdm_steps_one<ROWS>(acc[UT == 2 ? 0 : 2][2], tab, r.x, r.y, t, ar, br, flip);
+        if constexpr (NT > 3)
+          if (t == 3) rdm_steps_one<ROWS>(acc[1][3], tab, r.x, r.y, t, ar, br, flip);
       }
     }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < MS; j++) {
-      const int sl = wv + 16 * j;
-      if (sl < nslice) {
-        const uint32_t len = b_len[sl];
-        const uint32_t *p = b_pb + b_off[sl] + lane;
+    if (rest)
+      for (int sl = wv; sl < nslice; sl += kMmWaves) {
+        const uint32_t len = pb_len[sl];
+        const uint32_t *p = pb + pb_off[sl] + lane;
         double s = 0.0;
-#pragma unroll 4
+#pragma unroll 8
         for (uint32_t k = 0; k < len; k++) {
           const uint32_t wd = p[64 * (size_t)k];
-          const double v = xI[wd & 0x7fffu] * xJ[(wd >> 15) & 0x7fffu];
-          s += (wd >> 31) ? -v : v;
+          const uint32_t i = wd & 0x7fffu, j = (wd >> 15) & 0x7fffu;
+          s += signed_by(x.at(i) * y.at(j), (wd & 0x80000000u) ^ sx);
         }
-        acc[j] += sa * s;
+        const uint32_t bin = pb_perm[sl * 64 + lane];
+        if (bin != 0xffffffffu) atomicAdd(&trow[bin], s);
+      }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < UT; i++)
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        // accumulator r of lane l: row 4 r + l / 16, column l % 16
+        const int u = 16 * (u0 + i) + 4 * r + (lane >> 4), v = 16 * j + (lane & 15);
+        if (u < L && v < L && u != v) atomicAdd(&trow[u * L + v], acc[i][j][r]);
+      }
+  if (rest) {  // the occupation numbers: lane = orbital, wavefront = a run of strings
+    if (ROWS) {
+#pragma unroll
+      for (int k = 0; k < kMmRho; k++) {
+        const int i = tid + k * kMmThreads;
+        if (i < nb) xs[i] = rho[k];
       }
     }
+    __syncthreads();
+    const int per = (nb + kMmWaves - 1) / kMmWaves;
+    const int i0 = wv * per, i1 = i0 + per < nb ? i0 + per : nb;
+    double s = 0.0;
+#pragma unroll 8
+    for (int i = i0; i < i1; i++) s += ((b_str[i] >> lane) & 1ull) ? xs[i] : 0.0;
+    if (lane < L) atomicAdd(&trow[lane * (L + 1)], s);
   }
-#pragma unroll
-  for (int j = 0; j < MS; j++) {
-    const int sl = wv + 16 * j;
-    if (sl < nslice) {
-      const uint32_t bin = b_perm[sl * 64 + lane];
-      if (bin != 0xffffffffu) Tm[(size_t)pq * K + bin] = acc[j];
-    }
+  __syncthreads();
+  for (int i = tid; i < K; i += kMmThreads) {
+    const double v = trow[i];
+    if (v != 0.0) atomicAdd(&Tm[(size_t)it.x * K + i], v);
   }
 }
 
-// Place Tm[pq][rs] (alpha p->q, beta r->s) with TwoDiffCorrelation's rules on
-// the sorted spin orbitals I<J (bra-only 2p, 2r+1) and A<B (ket-only 2q, 2s+1).
+// Place T[pq][rs] (alpha p, q; beta r, s; rows p >= q are stored).  Two
+// excitations (p != q and r != s) follow TwoDiffCorrelation's rules on the
+// sorted spin orbitals I<J (bra-only 2p, 2r+1) and A<B (ket-only 2q, 2s+1);
+// an excitation beside an occupation number, or two occupation numbers,
+// OneDiff's and ZeroDiff's: (q, s, p, r) in the alpha-beta block, (s, q, r,
+// p) in the beta-alpha block.
 __global__ void k_rdm_mixed_place(int L, const double *__restrict__ Tm, double *__restrict__ two) {
   const size_t K = (size_t)L * L;
   const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= K * K) return;
-  const double t = Tm[idx];
-  if (t == 0.0) return;
   const int pq = (int)(idx / K), rs = (int)(idx % K);
   const int p = pq / L, q = pq % L, r = rs / L, s = rs % L;
+  const double t = p >= q ? Tm[idx] : Tm[(size_t)(q * L + p) * K + s * L + r];
+  if (t == 0.0) return;
+  const size_t L2 = K, L4 = K * K;
+  if (p == q || r == s) {
+    atomicAdd(&two[2 * L4 + q + L * s + L2 * (p + L * r)], t);
+    atomicAdd(&two[1 * L4 + s + L * q + L2 * (r + L * p)], t);
+    return;
+  }
   const int i = 2 * p, j = 2 * r + 1, a = 2 * q, b = 2 * s + 1;
   const int I = i < j ? i : j, J = i < j ? j : i, A = a < b ? a : b, B = a < b ? b : a;
   const size_t oi = I >> 1, si = I & 1, oa = A >> 1, sa = A & 1;
   const size_t oj = J >> 1, sj = J & 1, ob = B >> 1;
-  const size_t L2 = K, L4 = K * K;
   // distinct (pq, rs) can land on one element, hence the atomics
   if (si == sa) {
     atomicAdd(&two[(si + 2 * sj) * L4 + oa + L * ob + L2 * (oi + L * oj)], t);
@@ -425,13 +540,27 @@ __global__ void k_rdm_mixed_place(int L, const double *__restrict__ Tm, double *
 
 void transpose_into(Context &c, const double *in, double *out, int R, int Cc);
 
-template <int NT>
-static void launch_rdm_mixed(Context &c, const double *w, double *Tm, size_t lds) {
-  auto fn = k_rdm_mixed<NT>;
+template <int NT, int UT, bool ROWS>
+static void launch_rdm_mixed(Context &c, const double *w, double *Tm) {
+  auto fn = k_rdm_mixed<NT, UT, ROWS>;
+  const size_t lds = sizeof(double) * ((size_t)c.K + (ROWS ? 2 * (c.nb + 1) : c.nb));
   SBDX_HIP(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL(fn, dim3((unsigned)c.na), dim3(1024), lds, c.stream, (int)c.nb, c.K, c.A.s_off,
-                     c.A.s_ent, c.B.s_off, c.B.s_ent, w, Tm);
+  RdmRanges rg{};
+  rg.n = c.B.rc_nrange;
+  for (int i = 0; i < rg.n; i++) rg.r[i] = c.B.rc_range[i];
+  if (c.A.ra_nitem == 0) return;
+  hipLaunchKernelGGL(fn, dim3((unsigned)c.A.ra_nitem, NT / UT), dim3(kMmThreads), lds, c.stream, (int)c.nb, c.K, c.L,
+                     (const uint4 *)c.A.ra_item, (const uint64_t *)c.A.ra_ent, rg, (const uint64_t *)c.B.rc_tab,
+                     c.B.pb_nslice, (const uint32_t *)c.B.pb, (const uint64_t *)c.B.pb_off,
+                     (const uint32_t *)c.B.pb_len, (const uint32_t *)c.B.pb_perm, (const uint64_t *)c.B.str, w, Tm);
   check_launch("k_rdm_mixed");
+}
+template <bool ROWS>
+static void launch_rdm_mixed(Context &c, const double *w, double *Tm) {
+  if (c.L <= 16) launch_rdm_mixed<1, 1, ROWS>(c, w, Tm);
+  else if (c.L <= 32) launch_rdm_mixed<2, 2, ROWS>(c, w, Tm);
+  else if (c.L <= 48) launch_rdm_mixed<3, 3, ROWS>(c, w, Tm);
+  else launch_rdm_mixed<4, 2, ROWS>(c, w, Tm);
 }
 
 // p[0, n) = 0 (a fill kernel rather than hipMemsetAsync, so the work is a
@@ -447,13 +576,13 @@ static void zero(Context &c, double *p, size_t n) {
 }
 
 // Working memory of one RDM evaluation: per-string sums, the mixed-term
-// accumulator Tm[K][K], and room for ts_cap single pairs ((L+1) values each)
-// and td_cap double pairs (the pair tables are processed in chunks of that
-// many entries).
+// accumulator Tm[K][K], and room for ts_cap single pairs and td_cap double
+// pairs (without G the pair tables are processed in chunks of that many
+// entries; with G only td_cap counts).
 struct RdmWork {
-  double *rho_a, *rho_b, *mrow, *Tm, *Ts, *Td;
+  double *rho_a, *rho_b, *Tm, *Ts, *Td;
   size_t ts_cap, td_cap;
-  double *G = nullptr;  // room for max(na, nb)^2 values, or null (dot products per double pair)
+  double *G = nullptr;  // room for max(na, nb)^2 values, or null (dot products per pair)
 };
 
 // Everything after the sign conversion: W' (alpha-first, device) to one and
@@ -462,51 +591,51 @@ static void rdm_run(Context &c, const double *Wp, double *one, double *two, cons
   const int L = c.L;
   const size_t L2 = (size_t)L * L, L4 = L2 * L2, K = (size_t)c.K;
   const int na = (int)c.na, nb = (int)c.nb;
-  const size_t lds = sizeof(double) * ((size_t)nb + K);
-  const int nt = (nb + 1023) / 1024;
-  // the pair-major kernel stages two rows, each followed by a zero
-  const size_t lds_pq = sizeof(double) * (2 * (size_t)nb + 2);
-  const bool by_pair = c.A.pm_ent && c.B.pb && c.B.pb_nslice <= 64 && nb < 8192 && lds_pq <= c.lds_limit;
-  if (!by_pair && (lds > c.lds_limit || nt > 32))
+  // beta sets up to 20000 strings and more, as far as one row and one row of
+  // Tm fit in LDS (and 16-bit string numbers in the tables)
+  const bool small = nb < 8192 && sizeof(double) * (2 * (size_t)nb + 2) <= c.lds_limit;
+  if (nb >= 32767 || (!small && sizeof(double) * ((size_t)nb + K) > c.lds_limit))
     throw Error(3, "rdm: beta string count too large for the LDS-staged mixed RDM kernel");
   zero(c, one, 2 * L2);
   zero(c, two, 4 * L4);
   zero(c, wk.Tm, K * K);
   // W'^T (beta-major) for the beta-side sums
   transpose_into(c, Wp, c.T1, na, nb);
-  // ZeroDiff
-  hipLaunchKernelGGL(k_rdm_diag_rows, dim3(na), dim3(256), 0, c.stream, nb, L, c.B.str, Wp, wk.rho_a, wk.mrow);
-  check_launch("k_rdm_diag_rows");
-  hipLaunchKernelGGL(k_rdm_diag_rows, dim3(nb), dim3(256), 0, c.stream, na, L, c.A.str, c.T1, wk.rho_b,
-                     (double *)nullptr);
-  check_launch("k_rdm_diag_rows");
-  hipLaunchKernelGGL(k_rdm_diag_scatter, dim3(L), dim3(64), 0, c.stream, L, na, nb, c.A.str, c.B.str,
-                     wk.rho_a, wk.rho_b, wk.mrow, one, two);
-  check_launch("k_rdm_diag_scatter");
-  // same-spin singles and doubles, alpha (rows of W') then beta (rows of
-  // W'^T), in chunks of the pair tables
+  // same-spin terms, alpha (rows of W') then beta (rows of W'^T), in chunks
+  // of the pair tables
   for (int spin = 0; spin < 2; spin++) {
     const SpinTables &t = spin ? c.B : c.A;
-    const SpinTables &o = spin ? c.A : c.B;
     const double *w = spin ? c.T1 : Wp;
     const int M = spin ? na : nb;
-    for (size_t e0 = 0; e0 < t.ns; e0 += wk.ts_cap) {
-      const size_t e1 = std::min(t.ns, e0 + wk.ts_cap);
-      hipLaunchKernelGGL(k_rdm_single_pairs, dim3((unsigned)std::min<size_t>(e1 - e0, 1u << 20)), dim3(256), 0,
-                         c.stream, t.n, M, L, (uint64_t)e0, (uint64_t)e1, t.s_off, t.s_ent, o.str, w, wk.Ts);
-      check_launch("k_rdm_single_pairs");
-      hipLaunchKernelGGL(k_rdm_single_scatter, dim3(cdiv(e1 - e0, 256)), dim3(256), 0, c.stream, t.n, L, spin,
-                         (uint64_t)e0, (uint64_t)e1, t.s_off, t.s_ent, t.str, wk.Ts, one, two);
-      check_launch("k_rdm_single_scatter");
-    }
-    const bool gram = wk.G && t.nd > 0;
+    const bool gram = wk.G != nullptr;
+    double *rho = spin ? wk.rho_b : wk.rho_a;
     if (gram) {
       // G = w w^T: w is n rows of M values, i.e. the column-major M x n
       // matrix B, and G = B^T B (n x n, symmetric)
-      const double one = 1.0, zero_d = 0.0;
+      const double one_d = 1.0, zero_d = 0.0;
       if (rocblas_dgemm((rocblas_handle)blas_handle(c), rocblas_operation_transpose, rocblas_operation_none, t.n,
-                        t.n, M, &one, w, M, w, M, &zero_d, wk.G, t.n) != rocblas_status_success)
+                        t.n, M, &one_d, w, M, w, M, &zero_d, wk.G, t.n) != rocblas_status_success)
         throw Error(3, "rdm: rocblas_dgemm (Gram matrix) failed");
+    } else {
+      hipLaunchKernelGGL(k_rdm_diag_rows, dim3(t.n), dim3(256), 0, c.stream, M, w, rho);
+      check_launch("k_rdm_diag_rows");
+    }
+    hipLaunchKernelGGL(k_rdm_diag_pairs, dim3(cdiv(t.n, 4 * kDiagStr)), dim3(256), sizeof(double) * L2, c.stream,
+                       t.n, L, spin, t.str, gram ? (const double *)wk.G : (const double *)rho,
+                       gram ? (size_t)t.n + 1 : 1, one, two);
+    check_launch("k_rdm_diag_pairs");
+    const size_t ts_cap = gram ? std::max<size_t>(t.ns, 1) : wk.ts_cap;
+    for (size_t e0 = 0; e0 < t.ns; e0 += ts_cap) {
+      const size_t e1 = std::min(t.ns, e0 + ts_cap);
+      if (!gram) {
+        hipLaunchKernelGGL(k_rdm_single_pairs, dim3((unsigned)std::min<size_t>(e1 - e0, 1u << 20)), dim3(256), 0,
+                           c.stream, t.n, M, (uint64_t)e0, (uint64_t)e1, t.s_off, t.s_ent, w, wk.Ts);
+        check_launch("k_rdm_single_pairs");
+      }
+      hipLaunchKernelGGL(k_rdm_single_scatter, dim3(cdiv(e1 - e0, 256)), dim3(256), 0, c.stream, t.n, L, spin,
+                         (uint64_t)e0, (uint64_t)e1, t.s_off, t.s_ent, t.str, gram ? nullptr : wk.Ts, wk.G, one,
+                         two);
+      check_launch("k_rdm_single_scatter");
     }
     for (size_t e0 = 0; e0 < t.nd; e0 += wk.td_cap) {
       const size_t e1 = std::min(t.nd, e0 + wk.td_cap);
@@ -525,24 +654,12 @@ static void rdm_run(Context &c, const double *Wp, double *one, double *two, cons
       check_launch("k_rdm_double_scatter");
     }
   }
-  // mixed alpha-single x beta-single
-  if (by_pair) {
-    const int ms = (c.B.pb_nslice + 15) / 16;
-    auto go = [&](auto fn) {
-      SBDX_HIP(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_pq));
-      hipLaunchKernelGGL(fn, dim3((unsigned)K), dim3(1024), lds_pq, c.stream, nb, (int)K, c.B.pb_nslice,
-                         c.A.pm_off, c.A.pm_ent, c.B.pb, c.B.pb_off, c.B.pb_len, c.B.pb_perm, Wp, wk.Tm);
-    };
-    if (ms <= 1) go(k_rdm_mixed_pq<1>);
-    else if (ms <= 2) go(k_rdm_mixed_pq<2>);
-    else go(k_rdm_mixed_pq<4>);
-    check_launch("k_rdm_mixed_pq");
-  } else if (nt <= 1) launch_rdm_mixed<1>(c, Wp, wk.Tm, lds);
-  else if (nt <= 2) launch_rdm_mixed<2>(c, Wp, wk.Tm, lds);
-  else if (nt <= 4) launch_rdm_mixed<4>(c, Wp, wk.Tm, lds);
-  else if (nt <= 8) launch_rdm_mixed<8>(c, Wp, wk.Tm, lds);
-  else if (nt <= 16) launch_rdm_mixed<16>(c, Wp, wk.Tm, lds);
-  else launch_rdm_mixed<32>(c, Wp, wk.Tm, lds);
+  // two spins: both rows staged when they fit beside the row of T (and the
+  // x y sums in registers), else read where they are
+  if (small && nb <= kMmRho * kMmThreads && sizeof(double) * (K + 2 * (size_t)nb + 2) <= c.lds_limit)
+    launch_rdm_mixed<true>(c, Wp, wk.Tm);
+  else
+    launch_rdm_mixed<false>(c, Wp, wk.Tm);
   hipLaunchKernelGGL(k_rdm_mixed_place, dim3(cdiv(K * K, 256)), dim3(256), 0, c.stream, L, wk.Tm, two);
   check_launch("k_rdm_mixed_place");
   SBDX_HIP(hipStreamSynchronize(c.stream));
@@ -550,13 +667,12 @@ static void rdm_run(Context &c, const double *Wp, double *one, double *two, cons
 
 void compute_rdm(Context &c, const double *Wp, double *one, double *two) {
   ProfScope ps(c, "rdm");
-  const size_t L = (size_t)c.L, K = (size_t)c.K;
+  const size_t K = (size_t)c.K;
   const size_t ns = std::max<size_t>(std::max(c.A.ns, c.B.ns), 1);
   const size_t nd = std::max<size_t>(std::max(c.A.nd, c.B.nd), 1);
-  TmpBuf b_rho_a(sizeof(double) * c.na), b_rho_b(sizeof(double) * c.nb), b_mrow(sizeof(double) * c.na * L),
-      b_tm(sizeof(double) * K * K), b_ts(sizeof(double) * ns * (L + 1)), b_td(sizeof(double) * nd);
-  RdmWork wk{(double *)b_rho_a.p, (double *)b_rho_b.p, (double *)b_mrow.p, (double *)b_tm.p,
-             (double *)b_ts.p,    (double *)b_td.p,    ns,                  nd};
+  TmpBuf b_rho_a(sizeof(double) * c.na), b_rho_b(sizeof(double) * c.nb), b_tm(sizeof(double) * K * K),
+      b_ts(sizeof(double) * ns), b_td(sizeof(double) * nd);
+  RdmWork wk{(double *)b_rho_a.p, (double *)b_rho_b.p, (double *)b_tm.p, (double *)b_ts.p, (double *)b_td.p, ns, nd};
   // the Gram matrices of the double pairs when a quarter of free memory
   // holds one (else a dot product per pair)
   const size_t mx = std::max(c.na, c.nb);
@@ -603,6 +719,8 @@ static double *scratch_address(int device) {
   return g_scratch_ptr[device];
 }
 
+// (na L of them are not used; they keep the largest instance that is
+// accepted where it has always been)
 size_t rdm_noalloc_fixed_doubles(const Context &c) {
   auto up = [](size_t n) { return (n + 31) & ~size_t(31); };  // 256-byte aligned regions
   return up(c.na) + up(c.nb) + up(c.na * (size_t)c.L) + up((size_t)c.K * c.K);
@@ -627,14 +745,13 @@ void compute_rdm_noalloc(Context &c, const double *Wp, double *one, double *two)
   RdmWork wk{};
   wk.rho_a = p, p += up(c.na);
   wk.rho_b = p, p += up(c.nb);
-  wk.mrow = p, p += up(c.na * L);
   wk.Tm = p, p += up(K * K);
   const size_t rem = kRdmScratchDoubles - (size_t)(p - base);
   const size_t ns = std::max<size_t>(std::max(c.A.ns, c.B.ns), 1);
   const size_t nd = std::max<size_t>(std::max(c.A.nd, c.B.nd), 1);
   // half the rest for single pairs, the remainder for double pairs
-  wk.ts_cap = std::min(ns, std::max<size_t>(64, (rem / 2) / (L + 1)));
-  wk.Ts = p, p += up(wk.ts_cap * (L + 1));
+  wk.ts_cap = std::min(ns, std::max<size_t>(64, rem / 2));
+  wk.Ts = p, p += up(wk.ts_cap);
   wk.td_cap = std::min(nd, kRdmScratchDoubles - (size_t)(p - base));
   wk.Td = p;
   rdm_run(c, Wp, one, two, wk);

@@ -564,80 +564,6 @@ void build_singles_ell(Context &c, SpinTables &t) {
   const int n = t.n;
   std::vector<uint64_t> off, ent;
   download_singles(c, t, off, ent);
-  // the singles grouped by pair index (counting sort, row order kept
-  // within a pair) for the RDM's mixed term
-  {
-    const size_t K = (size_t)c.K;
-    std::vector<uint64_t> poff(K + 1, 0);
-    for (size_t k = 0; k < t.ns; k++) poff[((ent[k] >> 32) & 0x7fffffffull) + 1]++;
-    for (size_t pq = 0; pq < K; pq++) poff[pq + 1] += poff[pq];
-    std::vector<uint64_t> pent(t.ns);
-    std::vector<uint64_t> fill(poff.begin(), poff.end() - 1);
-    for (int r = 0; r < n; r++)
-      for (uint64_t k = off[r]; k < off[r + 1]; k++) {
-        const uint64_t e = ent[k];
-        const uint64_t dst = fill[(e >> 32) & 0x7fffffffull]++;
-        const uint32_t ket = (uint32_t)(e & 0xffffffffull), neg = (uint32_t)(e >> 63);
-        pent[dst] = (uint64_t)r | ((uint64_t)ket << 32) | ((uint64_t)neg << 63);
-      }
-    t.pm_off = (uint64_t *)dalloc(c, sizeof(uint64_t) * (K + 1));
-    t.pm_ent = (uint64_t *)dalloc(c, sizeof(uint64_t) * std::max<size_t>(t.ns, 1));
-    SBDX_HIP(hipMemcpyAsync(t.pm_off, poff.data(), sizeof(uint64_t) * (K + 1), hipMemcpyHostToDevice, c.stream));
-    SBDX_HIP(hipMemcpyAsync(t.pm_ent, pent.data(), sizeof(uint64_t) * t.ns, hipMemcpyHostToDevice, c.stream));
-    // the same grouping as a sliced ELL over the pair bins (n <= 32767):
-    // bins sorted by entry count (descending) into slices of 64 lanes,
-    // entry k of lane l of slice s at pb_off[s] + 64 k + l, packed as
-    // bra | ket << 15 | (sign<0) << 31; padding entries bra = ket = n (a
-    // staged zero); pb_perm[64 s + l] = the lane's bin (0xffffffff past K)
-    t.pb_nslice = 0;
-    if (n < 32768) {
-      std::vector<uint32_t> bins(K);
-      for (size_t i = 0; i < K; i++) bins[i] = (uint32_t)i;
-      std::stable_sort(bins.begin(), bins.end(), [&](uint32_t a, uint32_t b) {
-        return (poff[a + 1] - poff[a]) > (poff[b + 1] - poff[b]);
-      });
-      const size_t nsl = (K + 63) / 64;
-      std::vector<uint32_t> perm(nsl * 64, 0xffffffffu), len(nsl);
-      std::vector<uint64_t> soff(nsl);
-      uint64_t tot = 0;
-      for (size_t sl = 0; sl < nsl; sl++) {
-        uint64_t mx = 0;
-        for (size_t l = 0; l < 64; l++) {
-          const size_t slot = sl * 64 + l;
-          if (slot < K) {
-            perm[slot] = bins[slot];
-            mx = std::max<uint64_t>(mx, poff[bins[slot] + 1] - poff[bins[slot]]);
-          }
-        }
-        soff[sl] = tot;
-        len[sl] = (uint32_t)mx;
-        tot += mx * 64;
-      }
-      const uint32_t pad = (uint32_t)n | ((uint32_t)n << 15);
-      std::vector<uint32_t> pb(std::max<uint64_t>(tot, 1), pad);
-      for (size_t sl = 0; sl < nsl; sl++)
-        for (size_t l = 0; l < 64; l++) {
-          const uint32_t bin = perm[sl * 64 + l];
-          if (bin == 0xffffffffu) continue;
-          for (uint64_t k = poff[bin]; k < poff[bin + 1]; k++) {
-            const uint64_t pe = pent[k];
-            const uint32_t bra = (uint32_t)(pe & 0xffffffffull), ket = (uint32_t)((pe >> 32) & 0x7fffffffull);
-            pb[soff[sl] + 64 * (k - poff[bin]) + l] = bra | (ket << 15) | ((uint32_t)(pe >> 63) << 31);
-          }
-        }
-      t.pb = (uint32_t *)dalloc(c, sizeof(uint32_t) * pb.size());
-      t.pb_off = (uint64_t *)dalloc(c, sizeof(uint64_t) * nsl);
-      t.pb_len = (uint32_t *)dalloc(c, sizeof(uint32_t) * nsl);
-      t.pb_perm = (uint32_t *)dalloc(c, sizeof(uint32_t) * perm.size());
-      SBDX_HIP(hipMemcpyAsync(t.pb, pb.data(), sizeof(uint32_t) * pb.size(), hipMemcpyHostToDevice, c.stream));
-      SBDX_HIP(hipMemcpyAsync(t.pb_off, soff.data(), sizeof(uint64_t) * nsl, hipMemcpyHostToDevice, c.stream));
-      SBDX_HIP(hipMemcpyAsync(t.pb_len, len.data(), sizeof(uint32_t) * nsl, hipMemcpyHostToDevice, c.stream));
-      SBDX_HIP(hipMemcpyAsync(t.pb_perm, perm.data(), sizeof(uint32_t) * perm.size(), hipMemcpyHostToDevice,
-                              c.stream));
-      t.pb_nslice = (int)nsl;
-    }
-    SBDX_HIP(hipStreamSynchronize(c.stream));
-  }
   std::vector<uint32_t> order(n);
   for (int i = 0; i < n; i++) order[i] = (uint32_t)i;
   std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) {
@@ -813,6 +739,275 @@ void build_singles_ell_parts(Context &c, SpinTables &t, int nparts) {
   }
   t.nparts = nparts;
   t.part_h = h;
+}
+
+// Tables of the RDM's mixed term (SpinTables::ra_*, rc_*, pb).
+//
+// Singles come in blocks.  The strings k + u that share the string k with
+// one electron less are singles of each other, all of them: in the set's
+// singles matrix they are a dense block over the orbitals u, with the sign
+// s_u s_v, s_u = (-1)^(electrons of k below u).  Each single (r, j) lies in
+// exactly one such block, k = r & j.  A block of m members holds m (m - 1)
+// ordered pairs and is a column of the matrix-core kernel, which costs its
+// tiles of 16 orbitals squared (4 cycles of a CU per tile pair and alpha
+// pair of strings); below kBlockWorth pairs per tile pair the entries one by
+// one are as cheap (some 0.3 cycles each) and its singles are left over.
+// What is left over is regrouped by the string K = r | j with one electron
+// more (members K - u, sign -s_u s_v) into sets of members whose pairs are
+// all left over, grown greedily from the member with the most partners; the
+// rest goes to the entry table.  On a set of the Hartree-Fock string, its
+// singles and doubles the first kind covers the moves of a particle, the
+// second those of a hole.
+namespace {
+constexpr int kBlockWorth = 12;
+
+struct Member {
+  uint64_t key;
+  uint32_t str;
+  uint8_t orb;
+};
+struct Column {
+  uint64_t key;
+  uint32_t first;  // members [first, first + m) of the owner's list
+  uint16_t m;
+  int8_t tile;  // the one tile of its members, or -1
+  uint8_t hole;
+};
+
+inline uint64_t bit_reverse(uint64_t v) {
+  uint64_t r = 0;
+  for (int i = 0; i < 64; i++) r |= ((v >> i) & 1ull) << (63 - i);
+  return r;
+}
+inline bool odd_below(uint64_t key, int orb) { return __builtin_popcountll(key & ((1ull << orb) - 1ull)) & 1; }
+}  // namespace
+
+void build_rdm_tables(Context &c, SpinTables &t, const std::vector<uint64_t> &strs, bool as_alpha, bool as_beta) {
+  const int n = t.n, L = c.L;
+  const size_t K = (size_t)c.K;
+  std::vector<uint64_t> off, ent;
+  download_singles(c, t, off, ent);
+  auto put = [&](void *&dst, const void *src, size_t bytes) {
+    dst = dalloc(c, bytes);
+    if (bytes) SBDX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c.stream));
+  };
+  std::vector<uint64_t> aent;
+  std::vector<uint4> items;
+  if (as_alpha) {
+    std::vector<size_t> cnt(K + 1, 0);
+    auto kept = [&](uint64_t e) {
+      const uint32_t pq = (uint32_t)((e >> 32) & 0x7fffffffull);
+      return pq / L > pq % L ? (int)pq : -1;
+    };
+    for (size_t k = 0; k < t.ns; k++) {
+      const int pq = kept(ent[k]);
+      if (pq >= 0) cnt[pq + 1]++;
+    }
+    for (int r = 0; r < n; r++)
+      for (uint64_t o = strs[r]; o; o &= o - 1) cnt[(size_t)__builtin_ctzll(o) * (L + 1) + 1]++;
+    for (size_t i = 0; i < K; i++) cnt[i + 1] += cnt[i];
+    std::vector<size_t> at(cnt.begin(), cnt.end() - 1);
+    aent.resize(cnt[K]);
+    for (int r = 0; r < n; r++) {
+      for (uint64_t k = off[r]; k < off[r + 1]; k++) {
+        const int pq = kept(ent[k]);
+        if (pq >= 0)
+          aent[at[pq]++] = (uint64_t)r | ((ent[k] & 0x7fffffffull) << 32) | (ent[k] & (1ull << 63));
+      }
+      for (uint64_t o = strs[r]; o; o &= o - 1)
+        aent[at[(size_t)__builtin_ctzll(o) * (L + 1)]++] = (uint64_t)r | ((uint64_t)r << 32);
+    }
+    // items of equal length: long ones amortize the sums over the block and
+    // the atomics at an item's end, short ones keep every CU busy (at least
+    // eight items per CU)
+    const size_t len = std::min<size_t>(32, std::max<size_t>(1, aent.size() / ((size_t)8 * c.n_cu)));
+    for (size_t i = 0; i < K; i++)
+      for (size_t e = cnt[i]; e < cnt[i + 1]; e += len)
+        items.push_back(make_uint4((unsigned)i, (unsigned)e, (unsigned)std::min(e + len, cnt[i + 1]), 0u));
+    t.ra_nitem = (int)items.size();
+    void *p;
+    put(p, aent.data(), sizeof(uint64_t) * aent.size());
+    t.ra_ent = (uint64_t *)p;
+    put(p, items.data(), sizeof(uint4) * items.size());
+    t.ra_item = (uint4 *)p;
+  }
+  t.rc_nrange = 0;
+  t.pb_nslice = 0;
+  if (!as_beta || n >= 32767) {
+    SBDX_HIP(hipStreamSynchronize(c.stream));
+    return;
+  }
+  // particle blocks: (string, removed orbital) sorted by the remainder
+  std::vector<Member> pm;
+  pm.reserve((size_t)n * 16);
+  for (int r = 0; r < n; r++)
+    for (uint64_t o = strs[r]; o; o &= o - 1) {
+      const int u = __builtin_ctzll(o);
+      pm.push_back({strs[r] ^ (1ull << u), (uint32_t)r, (uint8_t)u});
+    }
+  std::sort(pm.begin(), pm.end(), [](const Member &a, const Member &b) {
+    return a.key < b.key || (a.key == b.key && a.orb < b.orb);
+  });
+  std::vector<Column> cols;
+  std::vector<uint64_t> big((size_t)n, 0);  // bit u of big[r]: r - u is the remainder of a kept block
+  const int nt = (L + 15) / 16;
+  auto tile_of = [](uint32_t tiles) { return (tiles & (tiles - 1)) ? -1 : __builtin_ctz(tiles); };
+  auto worth = [&](int m, int tile) {
+    const int q = tile < 0 ? nt : 1;
+    return m > 1 && m * (m - 1) >= kBlockWorth * q * q;
+  };
+  for (size_t i = 0; i < pm.size();) {
+    size_t j = i;
+    uint32_t tiles = 0;
+    for (; j < pm.size() && pm[j].key == pm[i].key; j++) tiles |= 1u << (pm[j].orb >> 4);
+    if (worth((int)(j - i), tile_of(tiles))) {
+      for (size_t k = i; k < j; k++) big[pm[k].str] |= 1ull << pm[k].orb;
+      cols.push_back({pm[i].key, (uint32_t)i, (uint16_t)(j - i), (int8_t)tile_of(tiles), 0});
+    }
+    i = j;
+  }
+  // what they leave over, by r | j: entry indices with their missing orbital
+  struct Left {
+    uint64_t key;
+    uint32_t ent, str;
+    uint8_t miss, add;  // r = K - miss, j = K - add
+  };
+  std::vector<Left> left;
+  for (int r = 0; r < n; r++)
+    for (uint64_t k = off[r]; k < off[r + 1]; k++) {
+      const uint32_t pq = (uint32_t)((ent[k] >> 32) & 0x7fffffffull);
+      const int p = pq / L, q = pq % L;
+      if (!((big[r] >> p) & 1ull))
+        left.push_back({strs[r] | (1ull << q), (uint32_t)k, (uint32_t)r, (uint8_t)q, (uint8_t)p});
+    }
+  std::sort(left.begin(), left.end(), [](const Left &a, const Left &b) {
+    return a.key < b.key || (a.key == b.key && a.ent < b.ent);
+  });
+  std::vector<Member> hm;
+  std::vector<uint8_t> done(left.size(), 0);
+  for (size_t i = 0; i < left.size();) {
+    size_t j = i;
+    uint64_t adj[64] = {}, verts = 0;
+    uint32_t who[64] = {};
+    for (; j < left.size() && left[j].key == left[i].key; j++) {
+      adj[left[j].miss] |= 1ull << left[j].add;
+      verts |= 1ull << left[j].miss;
+      who[left[j].miss] = left[j].str;
+    }
+    int cls[64];
+    std::fill(cls, cls + 64, -1);
+    for (int nc = 0;; nc++) {
+      auto best = [&](uint64_t among) {  // the member with the most partners among `among`
+        int b = -1, bd = -1;
+        for (uint64_t o = among; o; o &= o - 1) {
+          const int v = __builtin_ctzll(o), dg = __builtin_popcountll(adj[v] & among);
+          if (dg > bd) b = v, bd = dg;
+        }
+        return b;
+      };
+      const int v0 = best(verts);
+      if (v0 < 0) break;
+      uint64_t set = 1ull << v0, cand = adj[v0] & verts;
+      while (cand) {
+        const int v = best(cand);
+        set |= 1ull << v;
+        cand &= adj[v];
+      }
+      uint32_t tiles = 0;
+      for (uint64_t o = set; o; o &= o - 1) tiles |= 1u << (__builtin_ctzll(o) >> 4);
+      if (!worth(__builtin_popcountll(set), tile_of(tiles))) break;
+      cols.push_back(
+          {left[i].key, (uint32_t)hm.size(), (uint16_t)__builtin_popcountll(set), (int8_t)tile_of(tiles), 1});
+      for (uint64_t o = set; o; o &= o - 1) {
+        const int v = __builtin_ctzll(o);
+        hm.push_back({left[i].key, who[v], (uint8_t)v});
+        cls[v] = nc;
+      }
+      verts &= ~set;
+    }
+    for (size_t k = i; k < j; k++) done[k] = cls[left[k].miss] >= 0 && cls[left[k].miss] == cls[left[k].add];
+    i = j;
+  }
+  // columns of one kind and tile together, each run padded to steps of 4
+  for (auto &cl : cols) cl.key = bit_reverse(cl.key);
+  std::sort(cols.begin(), cols.end(), [](const Column &a, const Column &b) {
+    if (a.hole != b.hole) return a.hole < b.hole;
+    if (a.tile != b.tile) return a.tile < b.tile;
+    return a.key < b.key;
+  });
+  std::vector<uint64_t> tab;
+  const uint64_t none = (uint64_t)n * 0x0001000100010001ull;
+  for (size_t i = 0; i < cols.size();) {
+    size_t j = i;
+    while (j < cols.size() && cols[j].hole == cols[i].hole && cols[j].tile == cols[i].tile) j++;
+    const int s0 = (int)(tab.size() / 64), ns = (int)((j - i + 3) / 4);
+    tab.resize(tab.size() + (size_t)64 * ns, none);
+    for (size_t k = i; k < j; k++) {
+      const Member *mb = (cols[k].hole ? hm.data() : pm.data()) + cols[k].first;
+      uint64_t *w = tab.data() + (size_t)64 * (s0 + (k - i) / 4) + 16 * ((k - i) % 4);
+      for (int q = 0; q < cols[k].m; q++) {
+        const int u = mb[q].orb, sh = 16 * (u >> 4);
+        const uint64_t v = mb[q].str | (odd_below(mb[q].key, u) ? 0x8000ull : 0ull);
+        w[u & 15] = (w[u & 15] & ~(0xffffull << sh)) | (v << sh);
+      }
+    }
+    if (t.rc_nrange >= 24) throw Error(3, "rdm tables: too many kinds of columns");
+    t.rc_range[t.rc_nrange++] = make_int4(s0, s0 + ns, cols[i].tile, cols[i].hole);
+    i = j;
+  }
+  void *p;
+  put(p, tab.data(), sizeof(uint64_t) * tab.size());
+  t.rc_tab = (uint64_t *)p;
+  // the entry table of the rest: every pair's entries in runs of at most
+  // `run`, the shortest for which 8 slices (one per wavefront) hold all runs
+  std::vector<std::vector<uint32_t>> bin(K);
+  size_t nrest = 0;
+  for (size_t k = 0; k < left.size(); k++) {
+    if (done[k]) continue;
+    const uint64_t e = ent[left[k].ent];
+    bin[(e >> 32) & 0x7fffffffull].push_back(left[k].str | ((uint32_t)(e & 0x7fffull) << 15) |
+                                             ((uint32_t)(e >> 63) << 31));
+    nrest++;
+  }
+  size_t run = std::max<size_t>(4, (nrest + 511) / 512);
+  auto runs_of = [&](size_t len) {
+    size_t q = 0;
+    for (const auto &v : bin) q += (v.size() + len - 1) / len;
+    return q;
+  };
+  for (; run < nrest && runs_of(run) > 512 && runs_of(2 * run) < runs_of(run); run += (run + 7) / 8) {
+  }
+  struct Run {
+    uint32_t pair, first, len;
+  };
+  std::vector<Run> runs;
+  for (size_t i = 0; i < K; i++)
+    for (size_t k = 0; k < bin[i].size(); k += run)
+      runs.push_back({(uint32_t)i, (uint32_t)k, (uint32_t)std::min(run, bin[i].size() - k)});
+  std::stable_sort(runs.begin(), runs.end(), [](const Run &a, const Run &b) { return a.len > b.len; });
+  const size_t nsl = (runs.size() + 63) / 64;
+  std::vector<uint32_t> perm(nsl * 64, 0xffffffffu), len(nsl);
+  std::vector<uint64_t> soff(nsl);
+  std::vector<uint32_t> pb;
+  for (size_t i = 0; i < runs.size(); i++) {
+    if (i % 64 == 0) {
+      soff[i / 64] = pb.size();
+      len[i / 64] = runs[i].len;
+      pb.resize(pb.size() + (size_t)64 * runs[i].len, (uint32_t)n | ((uint32_t)n << 15));
+    }
+    perm[i] = runs[i].pair;
+    for (uint32_t k = 0; k < runs[i].len; k++) pb[soff[i / 64] + 64 * k + i % 64] = bin[runs[i].pair][runs[i].first + k];
+  }
+  put(p, pb.data(), sizeof(uint32_t) * pb.size());
+  t.pb = (uint32_t *)p;
+  put(p, soff.data(), sizeof(uint64_t) * nsl);
+  t.pb_off = (uint64_t *)p;
+  put(p, len.data(), sizeof(uint32_t) * nsl);
+  t.pb_len = (uint32_t *)p;
+  put(p, perm.data(), sizeof(uint32_t) * perm.size());
+  t.pb_perm = (uint32_t *)p;
+  t.pb_nslice = (int)nsl;
+  SBDX_HIP(hipStreamSynchronize(c.stream));
 }
 
 void compute_diag(Context &c) {
