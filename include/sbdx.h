@@ -185,7 +185,10 @@ int sbdx_same_spin_form(sbdx_handle_t h, int precision, int *form, float *ms_spa
  * both signs) and slots per thread (1, 2, 4, 8; a row's slots are split
  * over blocks accordingly) that fit (no counterpart in the reference):
  * *width 0 before that, -1 when no width fits in LDS (row parts or the
- * CSR/global variants run), else 1, 2, 4 or 16; *slots_per_thread, *ms the
+ * CSR/global variants run), 32 for the block kernel of the general FP64 sigma
+ * (taken without timing wherever its tables hold the string sets;
+ * *slots_per_thread is then the slices of 64 strings per wave it is built
+ * for and *ms 0), else 1, 2, 4 or 16; *slots_per_thread, *ms the
  * winner and its time (with width -1: the row-parts kernel's slots per
  * thread, timed the same way on its first use; SBDX_PARTS_NT fixes it);
  * *multi (forms 0

@@ -83,6 +83,39 @@ struct SpinTables {
   // n < 8192.
   uint32_t *ell3 = nullptr;
   bool has_ell3 = false;
+  // Tables of the mixed term's block kernel k_mixed_blk (build_blocks).
+  // As the alpha set: bk_order, the bra of each block; bk_ent, the singles of
+  // bra I and its spectator from s_off[I] + I on, ket | ERI triangle row <<
+  // 32 | spectator << 62 | (sign<0) << 63.  As the beta set:
+  // tasks of up to 16 columns (a column: a string k with one electron less
+  // and its members k + u) over a common list of up to 16 bk_mt orbitals:
+  // task k takes the steps bk_step[k] .. bk_step[k + 1] - 1 (an even number) of
+  // 4 orbitals of the list each; bk_tab[64 step + lane], with v the step's orbital lane /
+  // 16: y holds the member k + v of column lane % 16, string | (sign<0) << 15
+  // (n: none), half m of x the LDS element of (pq|u v) for the list's orbital
+  // u = 16 m + lane % 16 (2 Kt: none); at the
+  // end the accumulators of bk_tp tasks at a time lie in LDS, element (m 16 +
+  // row) 16 + column of each, and string r adds those at bk_col_pos[k] (|
+  // (sign<0) << 15) for bk_col_off[pass (n + 1) + r] <= k < its next.
+  // The singles outside the blocks: sliced ELL of 64 rows (bk_perm: rows by
+  // length, n past the end), bk_len low half groups of 4 entries from group
+  // bk_off on, each group lane-major (word u of lane l at 4 l + u); a word is
+  // ket << bk_pb | widx << 21, widx the triangle index, + Kt when negative
+  // (padding: ket n).  bk_rec: bk_nrec records of 8 halves per row, [slice]
+  // [record][lane]: the row, then the LDS elements of (kk) for the orbitals
+  // in which it differs from bk_ref (+ Kt where the row lacks it; 2 Kt:
+  // none), bk_len high half their number.
+  bool has_blk = false;
+  int bk_pb = 0, bk_mt = 0, bk_ntask = 0, bk_nslice = 0, bk_nrec = 1, bk_tp = 1;
+  int bk_nstep = 0, bk_ngroup = 0;  // steps of all tasks, groups of all slices
+  uint64_t bk_ref = 0;
+  size_t bk_image = 0;  // LDS bytes of one group
+  uint64_t *bk_ent = nullptr;
+  uint16_t *bk_col_pos = nullptr;
+  uint32_t *bk_order = nullptr, *bk_step = nullptr, *bk_col_off = nullptr, *bk_perm = nullptr, *bk_off = nullptr,
+           *bk_len = nullptr, *bk_ell = nullptr;
+  uint2 *bk_tab = nullptr;
+  uint4 *bk_rec = nullptr;
   // Tables of the RDM's mixed term (build_rdm_tables).
   // As the alpha set: the singles with p > q and the identity pairs (I, I)
   // of p == q, grouped by pair index: ra_ent = I | J << 32 | (sign<0) << 63
@@ -162,6 +195,9 @@ struct Context {
   bool eri_rs_sym = false;
   int Kt = 0;                  // L(L+1)/2
   uint16_t *tri_rs = nullptr;  // [Kt]: rs = a*L + b of triangle element a(a+1)/2 + b, a >= b
+  double *eri_tri = nullptr;   // [Kt + 1][Kt]: eri over the triangles, then its sums over B.bk_ref (on first use)
+  int blk_mode = -1;           // FP64 mixed term by k_mixed_blk: undecided, no, yes
+  double *spec = nullptr;      // [na][Kt]: spectator rows of the alpha strings (with eri_tri)
   double *h1 = nullptr;    // [K] spatial one-body
   SpinTables A, B;
   double *hii = nullptr;   // [N]
@@ -330,6 +366,7 @@ void check_launch(const char *what);
 void build_spin_tables(Context &c, SpinTables &t, const std::vector<uint64_t> &strs);
 void build_singles_ell(Context &c, SpinTables &t);
 void build_singles_ell_parts(Context &c, SpinTables &t, int nparts);
+void build_blocks(Context &c);
 void build_rdm_tables(Context &c, SpinTables &t, const std::vector<uint64_t> &strs, bool as_alpha, bool as_beta);
 void compute_diag(Context &c);
 void sign_convert(Context &c, const double *in, double *out);      // out = S*in

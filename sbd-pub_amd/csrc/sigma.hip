@@ -585,6 +585,405 @@ __global__ void __launch_bounds__(1024) k_mixed_sw(int nb, int K, int L, int Kt,
   }
 }
 
+// ---- mixed term by blocks of beta singles (FP64, general form)
+// Tables of one beta set (SpinTables::bk_*) and the launch geometry.
+struct BlkArgs {
+  int nb, Kt, nslice, nrec, ntask, task0, nwg, nmw, ng;
+  uint32_t img, xbase;  // bytes of one group's LDS image, and of its ERI part
+  uint32_t dump;        // byte offset of the accumulators' area in it at the end
+  int tp, per;          // tasks per pass through that area; per matrix wave
+  const uint64_t *a_off, *a_ent;
+  const uint32_t *order;  // bra of each block
+  const double *eri, *spec;
+  const uint32_t *step0;
+  const uint2 *tab;
+  const uint32_t *col_off;
+  const uint16_t *col_pos;
+  const uint32_t *perm;
+  const uint4 *rec;
+  const uint32_t *off, *len, *ell;
+};
+// a table value at a wave-uniform index, through the scalar cache
+template <typename U> __device__ __forceinline__ U sload(const U *p, size_t i) {
+  return ((const __attribute__((address_space(4))) U *)p)[i];
+}
+// alpha entries of the block kernel: ket | ERI triangle row << 32 | spectator
+// << 62 | (sign<0) << 63
+constexpr uint64_t kSpectator = 1ull << 62;
+
+// Mixed term y[I,:] += sum over the alpha singles (J, pq, s_a) of I of
+// s_a sum over the beta singles (j, rs, s_b) of r of s_b (pq|rs) x[J, j],
+// with both dressings, for one bra I per block.
+//
+// Beta singles come in blocks (SpinTables::bk_*): the strings k + u sharing a
+// string k with one electron less are all singles of each other, so over
+// the columns k and orbitals u the sum is a matrix product,
+//   y[k + u] += s_u sum_v (pq|uv) s_v x[J, k + v],
+// done on the FP64 matrix cores (16x16x4): a task is up to 16 columns over a
+// common list of at most 16 MT orbitals; the ERI operand is the same for all
+// columns of a task, the ket operand is gathered from the staged row x[J,:]
+// through a table of string numbers and signs, and the accumulators stay in
+// registers over all alpha singles of I.  The singles outside the blocks are
+// walked entry by entry from a sliced-ELL table as in k_mixed_sw: the staged
+// ERI row is kept over the triangle r >= s twice, with both signs, so an
+// entry is one mask, one shift and two LDS reads.  Some waves of a block do
+// the one (nmw of nwg), the rest the other, so each kind's registers hold
+// its own sums only.
+//
+// A round stages EB alpha singles of I, interleaved as EB-wide LDS elements:
+// 2 Kt + 1 signed ERI values (the last a zero) and nb + 1 ket values (the
+// last a zero).  The last pair of a bra is the spectator, sum_{k in alpha(I)}
+// (kk|..) with x[I,:], which dresses the beta singles; the dressing of an
+// alpha single, x[J,r] sum_{k in beta(r)} s_a (pq|kk), is that sum over a
+// reference string (one number per pair) corrected on the orbitals in which
+// r differs from it.  The block's waves form ng groups of nwg waves with an
+// LDS image each; group g takes rounds g, g + ng, ..
+// The sums meet in LDS at the end in a fixed order (the entries' sums, then
+// the blocks' tasks, then the groups), so results repeat bitwise.
+//
+// Bound by the matrix cores and LDS together: at 8000 x 8000 strings in 36
+// orbitals a round is 1600 matrix instructions (25600 cycles of a CU), some
+// 27000 cycles of LDS reads and 128 KB of ket rows from the caches, 31000
+// cycles in all; one entry at a time, two LDS reads and two FMA each, it was
+// 44000.  The entry waves alone stage, with a round's ket values held in
+// registers from the round before (with half of them loaded in place it was
+// 43 ms instead of 31, as fast as the form without blocks); the matrix waves
+// read their operands one step ahead of the instructions that use them.
+template <int EB, int MT, int NT, int TPW>
+__global__ void __launch_bounds__(1024) k_mixed_blk(BlkArgs g, const double *__restrict__ x, double *__restrict__ y) {
+  typedef double T;
+  typedef typename Pack<T, EB>::V V;
+  typedef double C __attribute__((ext_vector_type(4)));
+  constexpr int PB = sizeof(V) == 16 ? 4 : 3;  // log2 of an LDS element
+  constexpr uint32_t xmask = 0x1ffffu & ~((1u << PB) - 1u);
+  // the kernel has no static LDS, so the dynamic array starts at LDS
+  // address 0 (checked by the launcher) and an offset is an address
+  typedef __attribute__((address_space(3))) V lds_v;
+  typedef __attribute__((address_space(3))) T lds_t;
+  auto at = [](uint32_t o) -> V { return *reinterpret_cast<const lds_v *>((size_t)o); };
+  auto put = [](uint32_t o, V v) { *reinterpret_cast<lds_v *>((size_t)o) = v; };
+  auto val = [](uint32_t base, uint32_t i) { return reinterpret_cast<lds_t *>((size_t)(base + i * 8u)); };
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int grp = wave / g.nwg, wl = wave % g.nwg;
+  const int gsz = g.nwg * 64, gt = wl * 64 + lane;  // threads of a group
+  const uint32_t wb = grp * g.img, xb = wb + g.xbase;
+  const int nb = g.nb, Kt = g.Kt;
+  const int I = (int)sload(g.order, blockIdx.x);
+  // the bra's entries: its singles and the spectator
+  const uint64_t e0 = sload(g.a_off, I) + I, e1 = sload(g.a_off, I + 1) + I + 1;
+  const int part = (wl + (g.nwg < 4 ? 0 : grp)) % g.nwg;  // parts rotate, so that SIMDs share them evenly
+  // every round of this group in an entry wave: stage, then body(the
+  // reference's dressing).  Two barriers per round in every wave, whatever
+  // its part; then one more, after which the images are free.
+  const int et = (part - g.nmw) * 64 + lane, esz = (g.nwg - g.nmw) * 64;  // threads of the entry waves
+  auto rounds = [&](auto body) {
+    if (et == 0) {
+      V z;
+#pragma unroll
+      for (int q = 0; q < EB; q++) lane_of<T, EB>(z, q) = T(0);
+      put(wb + ((uint32_t)(2 * Kt) << PB), z);
+      put(xb + ((uint32_t)nb << PB), z);
+    }
+    const T *xs[EB], *vs[EB];
+    uint32_t neg[EB];
+    T cr[EB];
+    bool some[EB];
+    auto source = [&](uint64_t e) {
+#pragma unroll
+      for (int q = 0; q < EB; q++) {
+        some[q] = e + q < e1;
+        const uint64_t ent = sload(g.a_ent, some[q] ? e + q : e1 - 1);
+        const uint32_t t = (uint32_t)(ent >> 32) & 0xffffu;
+        const bool sp = (ent & kSpectator) != 0;
+        neg[q] = (uint32_t)(ent >> 63) << 31;
+        xs[q] = x + (size_t)(uint32_t)ent * nb;
+        vs[q] = sp ? g.spec + (size_t)I * Kt : g.eri + (size_t)t * Kt;
+        cr[q] = sp || !some[q] ? T(0) : flip_sign(sload(g.eri, (size_t)Kt * Kt + t), neg[q]);
+      }
+    };
+    // the first CH chunks of the ket values (all of them up to 24 slices a
+    // wave) and the first ERI value of a round load while the previous round
+    // is worked on
+    constexpr int CH = NT < (EB == 2 ? 8 : 16) ? NT : (EB == 2 ? 8 : 16);
+    V xv[CH], wv;
+    auto load_x = [&](int i0) {
+      asm volatile("" : "+v"(i0));  // as below: no offset kept over a round
+#pragma unroll
+      for (int k = 0; k < CH; k++) {
+        const int i = i0 + k * esz;
+        const int ic = i < nb ? i : nb - 1;  // every load in bounds, none behind a branch
+#pragma unroll
+        for (int q = 0; q < EB; q++) lane_of<T, EB>(xv[k], q) = xs[q][ic];
+      }
+    };
+    auto store_x = [&](int i0) {
+      asm volatile("" : "+v"(i0));
+#pragma unroll
+      for (int k = 0; k < CH; k++) {
+        const int i = i0 + k * esz;
+#pragma unroll
+        for (int q = 0; q < EB; q++)
+          if (!some[q]) lane_of<T, EB>(xv[k], q) = T(0);  // an empty pair has read some row
+        if (i < nb) put(xb + ((uint32_t)i << PB), xv[k]);
+      }
+    };
+    auto load_w = [&](int i) {
+#pragma unroll
+      for (int q = 0; q < EB; q++) lane_of<T, EB>(wv, q) = vs[q][i];
+    };
+    auto store_w = [&](int i) {
+      V w, wn;
+#pragma unroll
+      for (int q = 0; q < EB; q++) {
+        const T v = some[q] ? flip_sign(lane_c<T, EB>(wv, q), neg[q]) : T(0);
+        lane_of<T, EB>(w, q) = v;
+        lane_of<T, EB>(wn, q) = -v;
+      }
+      put(wb + ((uint32_t)i << PB), w);
+      put(wb + ((uint32_t)(Kt + i) << PB), wn);
+    };
+    source(e0 + (uint64_t)EB * grp);
+    load_x(et);
+    load_w(et < Kt ? et : Kt - 1);
+#pragma clang loop unroll(disable)
+    for (uint64_t er = e0; er < e1; er += (uint64_t)EB * g.ng) {
+      const bool live = some[0];  // uniform per group
+      __syncthreads();            // the previous round's reads
+      if (live) {
+        store_x(et);
+        if (et < Kt) store_w(et);
+#pragma clang loop unroll(disable)
+        for (int i0 = et + CH * esz; i0 - lane < nb; i0 += CH * esz) {
+          load_x(i0);
+          store_x(i0);
+        }
+#pragma clang loop unroll(disable)
+        for (int i = et + esz; i < Kt; i += esz) {
+          load_w(i);
+          store_w(i);
+        }
+      }
+      V cref;
+#pragma unroll
+      for (int q = 0; q < EB; q++) lane_of<T, EB>(cref, q) = cr[q];
+      source(er + (uint64_t)EB * (g.ng + grp));
+      __syncthreads();
+      load_x(et);
+      load_w(et < Kt ? et : Kt - 1);
+      if (live) body(cref);
+    }
+    __syncthreads();
+  };
+  // at the end: string r's sum at val(wb, r); the accumulators of tp tasks at
+  // a time behind them, from where r's thread adds its own (col_pos)
+  auto add_columns = [&](int pass) {
+    const uint32_t *co = g.col_off + (size_t)pass * (nb + 1);
+    for (int r = gt; r < nb; r += gsz) {
+      T v = T(0);
+      for (uint32_t k = co[r]; k < co[r + 1]; k++) {
+        const uint32_t p = g.col_pos[k];
+        v += flip_sign(*val(wb + g.dump, p & 0x7fffu), (p & 0x8000u) << 16);
+      }
+      *val(wb, r) += v;
+    }
+  };
+  const int pass0 = g.task0 / g.tp, pass1 = (g.ntask + g.tp - 1) / g.tp;
+  if (part < g.nmw) {
+    // ---- matrix waves
+    C acc[TPW][MT];
+#pragma unroll
+    for (int q = 0; q < TPW; q++)
+#pragma unroll
+      for (int m = 0; m < MT; m++) acc[q][m] = C{T(0), T(0), T(0), T(0)};
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    typedef __attribute__((address_space(1))) const u32x2 gl_u2;
+    const int t0 = g.task0 + part * g.per;  // this wave's tasks
+    uint32_t end[TPW];                      // the step after each
+#pragma unroll
+    for (int q = 0; q < TPW; q++) end[q] = sload(g.step0, q < g.per && t0 + q < g.ntask ? t0 + q + 1 : 0);
+    const uint32_t first = sload(g.step0, t0 < g.ntask ? t0 : 0);
+    for (uint64_t er = e0; er < e1; er += (uint64_t)EB * g.ng) {
+      __syncthreads();
+      __syncthreads();
+      if (er + (uint64_t)EB * grp >= e1 || t0 >= g.ntask) continue;
+      // (an opaque lane index, an empty asm statement without instruction,
+      // keeps the compiler from holding table words over all rounds)
+      int ln = lane;
+      asm volatile("" : "+v"(ln));
+      gl_u2 *p = (gl_u2 *)g.tab + (size_t)first * 64 + ln;
+      // operands are read from LDS one step ahead, table words three (past
+      // the last step: the next task or the table's padding, not used)
+      u32x2 a = p[0], b = p[64];
+      V xa, xc, wa[MT], wc[MT];
+      auto fetch = [&](u32x2 w, V &xq, V (&wq)[MT]) {
+        xq = flip_sign<T, EB>(at(xb + ((w.y & 0x7fffu) << PB)), (w.y & 0x8000u) << 16);
+#pragma unroll
+        for (int m = 0; m < MT; m++) wq[m] = at(wb + (((w.x >> (16 * m)) & 0xffffu) << PB));
+      };
+      fetch(a, xa, wa);
+      a = p[128];
+      uint32_t s = first;
+#pragma unroll
+      for (int q = 0; q < TPW; q++) {
+#pragma clang loop unroll(disable)
+        for (; s < end[q]; s += 2) {
+          fetch(b, xc, wc);
+          p += 128;
+          asm volatile("" : "+v"(p));
+          b = p[64];
+#pragma unroll
+          for (int qq = 0; qq < EB; qq++)
+#pragma unroll
+            for (int m = 0; m < MT; m++)
+              acc[q][m] = __builtin_amdgcn_mfma_f64_16x16x4f64(lane_c<T, EB>(wa[m], qq), lane_c<T, EB>(xa, qq),
+                                                               acc[q][m], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          fetch(a, xa, wa);
+          a = p[128];
+#pragma unroll
+          for (int qq = 0; qq < EB; qq++)
+#pragma unroll
+            for (int m = 0; m < MT; m++)
+              acc[q][m] = __builtin_amdgcn_mfma_f64_16x16x4f64(lane_c<T, EB>(wc[m], qq), lane_c<T, EB>(xc, qq),
+                                                               acc[q][m], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+    __syncthreads();
+    for (int pass = pass0; pass < pass1; pass++) {
+#pragma unroll
+      for (int q = 0; q < TPW; q++) {
+        const int task = t0 + q, k = task - pass * g.tp;
+        if (q < g.per && task < g.ntask && k >= 0 && k < g.tp) {
+#pragma unroll
+          for (int m = 0; m < MT; m++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)  // accumulator r of lane l: row 4 r + l / 16, column l % 16
+              *val(wb + g.dump, (k * MT + m) * 256 + 64 * r + lane) = acc[q][m][r];
+        }
+      }
+      __syncthreads();
+      add_columns(pass);
+      __syncthreads();
+    }
+  } else {
+    // ---- entry waves
+    T ae[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) ae[t] = T(0);
+    const int w0 = __builtin_amdgcn_readfirstlane(part - g.nmw), nw = g.nwg - g.nmw;
+    rounds([&](V cref) {
+      typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+      typedef __attribute__((address_space(1))) const u32x4 gl_u4;
+      int ln = lane, s0 = __builtin_amdgcn_readfirstlane(w0);
+      asm volatile("" : "+v"(ln), "+s"(s0));
+      auto row = [&](int sl) { return sl < g.nslice ? sl : 0; };
+      auto rec_at = [&](int sl) { return ((gl_u4 *)g.rec)[(size_t)row(sl) * 64 * g.nrec + ln]; };
+      auto ell_at = [&](int sl) { return (gl_u4 *)g.ell + (size_t)sload(g.off, row(sl)) * 64 + ln; };
+      // the row record and the first two groups of entries are loaded one
+      // slice ahead
+      u32x4 rec = rec_at(s0);
+      gl_u4 *p = ell_at(s0);
+      u32x4 ga = p[0], gb = p[64];
+#pragma unroll
+      for (int t = 0; t < NT; t++) {
+        const int sl = s0 + t * nw;
+        if (sl < g.nslice) {
+          const uint32_t ld = sload(g.len, sl), ng4 = ld & 0xffffu, nd = ld >> 16;
+          const u32x4 rc = rec, g0 = ga, g1 = gb;
+          gl_u4 *pc = p;
+          if (t + 1 < NT) {
+            rec = rec_at(sl + nw);
+            p = ell_at(sl + nw);
+            ga = p[0];
+            gb = p[64];
+          }
+          // dressing: + the orbitals of the row outside the reference, - those it lacks
+          const V xr = at(xb + ((rc.x & 0xffffu) << PB));
+          V dr = (cref + at(wb + ((rc.x >> 16) << PB))) + at(wb + ((rc.y & 0xffffu) << PB));
+          dr += at(wb + ((rc.y >> 16) << PB)) + at(wb + ((rc.z & 0xffffu) << PB));
+          if (nd > 4) {
+            dr += at(wb + ((rc.z >> 16) << PB)) + (at(wb + ((rc.w & 0xffffu) << PB)) + at(wb + ((rc.w >> 16) << PB)));
+            for (uint32_t k = 1; 8 * k - 1 < nd; k++) {  // further records of 8
+              const u32x4 r2 = ((gl_u4 *)g.rec)[((size_t)sl * g.nrec + k) * 64 + ln];
+#pragma unroll
+              for (int u = 0; u < 4; u++)
+                dr += at(wb + ((r2[u] & 0xffffu) << PB)) + at(wb + ((r2[u] >> 16) << PB));
+            }
+          }
+          T s[2] = {T(0), T(0)};
+#pragma unroll
+          for (int qq = 0; qq < EB; qq++) s[0] = fma(lane_c<T, EB>(dr, qq), lane_c<T, EB>(xr, qq), s[0]);
+          auto group = [&](const u32x4 &w) {
+            constexpr int H = 4 / EB;  // entries read at a time
+#pragma unroll
+            for (int h = 0; h < 4; h += H) {
+              V wq[H], xq[H];
+#pragma unroll
+              for (int u = 0; u < H; u++) {
+                wq[u] = at((w[h + u] >> (21 - PB)) + wb);
+                xq[u] = at((w[h + u] & xmask) + xb);
+              }
+#pragma unroll
+              for (int u = 0; u < H; u++)
+#pragma unroll
+                for (int qq = 0; qq < EB; qq++)
+                  s[u & 1] = fma(lane_c<T, EB>(wq[u], qq), lane_c<T, EB>(xq[u], qq), s[u & 1]);
+              if (H < 4) __builtin_amdgcn_sched_barrier(0);  // the registers of one part at a time
+            }
+          };
+          if (ng4 > 0) group(g0);
+          if (ng4 > 1) group(g1);
+          if (ng4 > 2) {
+            // two buffers in turn, two groups ahead (past the last group:
+            // the next slice or the table's padding, not used)
+            u32x4 b0 = pc[128], b1 = pc[192];
+            pc += 256;
+            uint32_t q = 2;
+            for (; q + 2 <= ng4; q += 2) {
+              asm volatile("" : "+v"(pc));
+              group(b0);
+              b0 = pc[0];
+              group(b1);
+              b1 = pc[64];
+              pc += 128;
+            }
+            if (q < ng4) group(b0);
+          }
+          ae[t] += s[0] + s[1];
+        }
+        // no loads of slices after the next one ahead of this one's sums:
+        // their registers are those of the accumulators
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    });
+    if (g.nslice == 0)  // a launch with further tasks only
+      for (int i = w0 * 64 + lane; i < nb; i += nw * 64) *val(wb, i) = T(0);
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+      const int sl = w0 + t * nw;
+      if (sl < g.nslice) {
+        const uint32_t r = g.perm[sl * 64 + lane];
+        if (r < (uint32_t)nb) *val(wb, r) = ae[t];
+      }
+    }
+    for (int pass = pass0; pass < pass1; pass++) {
+      __syncthreads();
+      add_columns(pass);
+      __syncthreads();
+    }
+  }
+  if (pass0 >= pass1) __syncthreads();  // uniform per launch
+  for (int i = threadIdx.x; i < nb; i += blockDim.x) {
+    T v = *val(0u, i);
+    for (int k = 1; k < g.ng; k++) v += *val(k * g.img, i);
+    const size_t o = (size_t)I * nb + i;
+    y[o] += v;
+  }
+}
+
 // Mixed term for KV vectors at once (x_v = x + v*N): one ERI row and the KV
 // ket rows x_v[J,:] staged per alpha single (then the spectator pair), so
 // each sliced-ELL entry costs one table load and 1 + KV LDS reads for KV
@@ -1162,6 +1561,7 @@ static bool mixed_ell_dispatch(Context &c, int nt, const T *eri, const T *x, T *
 // Staging width code of the signed-triangle kernel in the autotuner's
 // (width, slots) choice: 16-byte pairs, 4 FP32 or 2 FP64 values.
 constexpr int kEbSigned = 16;
+constexpr int kEbBlocks = 32;  // the width reported for k_mixed_blk
 
 template <typename T, int NT, bool SYM>
 static void launch_mixed_sw(Context &c, const T *eri, const T *x, T *y, size_t lds) {
@@ -1192,6 +1592,199 @@ static bool mixed_sw_dispatch(Context &c, int nt, const T *eri, const T *x, T *y
   else if (nt <= 4) launch_mixed_sw<T, 4, SYM>(c, eri, x, y, lds);
   else launch_mixed_sw<T, 8, SYM>(c, eri, x, y, lds);
   return true;
+}
+
+// ---- the block kernel's ERI tables and launches
+// (pq|rs) over the triangles pq and rs: out[i * Kt + j], i and j triangle
+// indices (tri_rs: triangle index to pair index), and behind it for every i
+// the sum over the orbitals k of ref of (pq|kk)
+__global__ void __launch_bounds__(256) k_eri_tri(int Kt, int K, int L, uint64_t ref,
+                                                 const uint16_t *__restrict__ tri_rs,
+                                                 const double *__restrict__ eri, double *__restrict__ out) {
+  const size_t n = (size_t)Kt * Kt;
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n + Kt; i += (size_t)gridDim.x * 256) {
+    if (i < n) {
+      out[i] = eri[(size_t)tri_rs[i / Kt] * K + tri_rs[i % Kt]];
+    } else {
+      double v = 0.0;
+      for (uint64_t o = ref; o; o &= o - 1) v += eri[(size_t)tri_rs[i - n] * K + __builtin_ctzll(o) * (L + 1)];
+      out[i] = v;
+    }
+  }
+}
+// Spectator rows: out[I * Kt + j] = sum_{k in alpha(I)} (kk|j), zero on the
+// diagonal j = (rr); one block per string
+__global__ void __launch_bounds__(256) k_spectator(int Kt, int L, const uint64_t *__restrict__ str,
+                                                   const uint16_t *__restrict__ tri_rs,
+                                                   const double *__restrict__ eri_tri, double *__restrict__ out) {
+  const uint64_t s = str[blockIdx.x];
+  for (int j = threadIdx.x; j < Kt; j += 256) {
+    double v = 0.0;
+    if (tri_rs[j] % (L + 1) != 0)
+      for (uint64_t o = s; o; o &= o - 1) {
+        const int k = __builtin_ctzll(o);
+        v += eri_tri[(size_t)(k * (k + 3) / 2) * Kt + j];
+      }
+    out[(size_t)blockIdx.x * Kt + j] = v;
+  }
+}
+static void blk_tables(Context &c) {
+  if (c.eri_tri) return;
+  double *e = (double *)dalloc(c, sizeof(double) * (size_t)c.Kt * (c.Kt + 1));
+  hipLaunchKernelGGL(k_eri_tri, dim3(std::min<unsigned>(cdiv((size_t)c.Kt * (c.Kt + 1), 256), 4096)), dim3(256), 0,
+                     c.stream, c.Kt, c.K, c.L, c.B.bk_ref, (const uint16_t *)c.tri_rs, (const double *)c.eri, e);
+  check_launch("k_eri_tri");
+  c.spec = (double *)dalloc(c, sizeof(double) * (size_t)c.Kt * c.na);
+  hipLaunchKernelGGL(k_spectator, dim3((unsigned)c.na), dim3(256), 0, c.stream, c.Kt, c.L,
+                     (const uint64_t *)c.A.str, (const uint16_t *)c.tri_rs, (const double *)e, c.spec);
+  check_launch("k_spectator");
+  c.eri_tri = e;
+}
+
+// Geometry of k_mixed_blk for this context: waves per group, matrix waves
+// among them, groups per block, slices per entry wave.
+struct BlkGeom {
+  int nwg, nmw, ng, nt;
+};
+constexpr int blk_tpw(int mt) { return mt == 1 ? 8 : 5; }  // tasks per matrix wave
+static BlkGeom blk_geom(const Context &c) {
+  const SpinTables &t = c.B;
+  BlkGeom g{};
+  const int nt_max = 24, tpw = blk_tpw(t.bk_mt), eb = t.bk_pb == 4 ? 2 : 1;
+  // Cycles of a round: a step of a task is eb bk_mt matrix instructions of 64
+  // cycles, done task by task in a wave and on four SIMDs for all groups of
+  // a CU together (a wave alone on its SIMD reaches some 80 % of that: 8 of
+  // 16 waves instead of 4 took the product of 8000 x 8000 strings in 36
+  // orbitals from 33.8 to 30.7 ms); a slice some 400 cycles and 150 per
+  // group of entries (latencies of its loads from L2 and LDS, partly
+  // overlapped).  The split with the least cycles per round of a CU that
+  // holds all slices is taken, of the smallest groups among equal ones; with
+  // more tasks than 16 waves hold, further launches follow.
+  const double mat = (double)t.bk_nstep * eb * t.bk_mt * 64.0;
+  double best = 0.0;
+  g.nwg = 16;
+  g.nmw = -1;
+  for (int n = 4; n <= 16; n *= 2) {
+    const int unit = n / 4;
+    const double grp = (double)std::min<size_t>(16 / n, std::max<size_t>(1, c.lds_limit / t.bk_image));
+    for (int m = t.bk_ntask ? unit : 0; m <= (t.bk_ntask ? n - unit : 0); m += unit) {
+      const int w = n - m;
+      if ((t.bk_nslice + w - 1) / w > nt_max || (n < 16 && m * tpw < t.bk_ntask)) continue;
+      double cost = (400.0 * t.bk_nslice + 150.0 * t.bk_ngroup) / w;
+      if (m) cost = std::max({cost, mat * ((t.bk_ntask + m - 1) / m) / t.bk_ntask, mat * grp / 4.0 * (m * grp > 4 ? 1.0 : 1.25)});
+      cost /= grp;
+      if (g.nmw < 0 || cost < 0.99 * best) best = cost, g.nmw = m, g.nwg = n;
+    }
+  }
+  const int w = std::max(1, g.nwg - g.nmw), per = (t.bk_nslice + w - 1) / w;
+  g.nt = per <= 4 ? 4 : per <= 12 ? 12 : per <= 16 ? 16 : 24;
+  // groups: one where the bras fill the chip twice over with blocks of one
+  // group (blocks then overlap each other's staging), else up to 16 waves,
+  // as far as they fit in LDS and have a round each
+  const size_t rounds = (c.A.max_s + 1 + eb - 1) / eb;
+  g.ng = 1;
+  while (g.nwg * g.ng * 2 <= 16 && t.bk_image * g.ng * 2 <= c.lds_limit && (size_t)g.ng * 2 <= rounds &&
+         c.na < (size_t)2 * c.n_cu * (16 / (g.nwg * g.ng)))
+    g.ng *= 2;
+  return g;
+}
+
+template <int EB, int MT, int NT>
+static void launch_mixed_blk(Context &c, const BlkGeom &q, const double *x, double *y) {
+  auto fn = k_mixed_blk<EB, MT, NT, blk_tpw(MT)>;
+  static bool lds_base_checked = false;
+  if (!lds_base_checked) {
+    hipFuncAttributes attr;
+    SBDX_HIP(hipFuncGetAttributes(&attr, (const void *)fn));
+    if (attr.sharedSizeBytes != 0) throw Error(2, "k_mixed_blk: static LDS would offset the dynamic array");
+    lds_base_checked = true;
+  }
+  const SpinTables &t = c.B;
+  const size_t lds = t.bk_image * q.ng;
+  SBDX_HIP(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  BlkArgs g{};
+  g.nb = (int)c.nb;
+  g.Kt = c.Kt;
+  g.nrec = t.bk_nrec;
+  g.nwg = q.nwg;
+  g.nmw = q.nmw;
+  g.ng = q.ng;
+  g.img = (uint32_t)t.bk_image;
+  g.xbase = (uint32_t)(((size_t)2 * c.Kt + 1) << t.bk_pb);
+  g.dump = (uint32_t)(8 * c.nb);
+  g.tp = t.bk_tp;
+  g.a_off = c.A.s_off;
+  g.a_ent = c.A.bk_ent;
+  g.order = c.A.bk_order;
+  g.eri = c.eri_tri;
+  g.spec = c.spec;
+  g.step0 = t.bk_step;
+  g.tab = t.bk_tab;
+  g.col_off = t.bk_col_off;
+  g.col_pos = t.bk_col_pos;
+  g.perm = t.bk_perm;
+  g.rec = t.bk_rec;
+  g.off = t.bk_off;
+  g.len = t.bk_len;
+  g.ell = t.bk_ell;
+  // further launches for the tasks that the matrix waves cannot hold (whole
+  // passes of tp tasks each)
+  int most = blk_tpw(MT) * std::max(1, q.nmw);
+  if (most < t.bk_ntask) most = std::max(1, most / t.bk_tp) * t.bk_tp;
+  for (int t0 = 0; t0 == 0 || t0 < t.bk_ntask; t0 += most) {
+    g.task0 = t0;
+    g.ntask = std::min(t.bk_ntask, t0 + most);
+    g.per = (g.ntask - t0 + std::max(1, q.nmw) - 1) / std::max(1, q.nmw);
+    g.nslice = t0 == 0 ? t.bk_nslice : 0;
+    hipLaunchKernelGGL(fn, dim3((unsigned)c.na), dim3(64 * q.nwg * q.ng), lds, c.stream, g, x, y);
+    check_launch("k_mixed_blk");
+  }
+}
+
+static void mixed_blk(Context &c, const double *x, double *y) {
+  const SpinTables &t = c.B;
+  const BlkGeom q = blk_geom(c);
+  auto go = [&](auto eb, auto mt) {
+    constexpr int EB = decltype(eb)::value, MT = decltype(mt)::value;
+    if (q.nt == 4) launch_mixed_blk<EB, MT, 4>(c, q, x, y);
+    else if (q.nt == 12) launch_mixed_blk<EB, MT, 12>(c, q, x, y);
+    else if (q.nt == 16) launch_mixed_blk<EB, MT, 16>(c, q, x, y);
+    else launch_mixed_blk<EB, MT, 24>(c, q, x, y);
+  };
+  using std::integral_constant;
+  if (t.bk_pb == 4) {
+    if (t.bk_mt == 1) go(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+    else go(integral_constant<int, 2>{}, integral_constant<int, 2>{});
+  } else {
+    if (t.bk_mt == 1) go(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+    else go(integral_constant<int, 1>{}, integral_constant<int, 2>{});
+  }
+}
+
+// Whether the block kernel computes the FP64 mixed term of the general form,
+// decided on a context's first FP64 product: wherever its tables hold the
+// set (ERIs symmetric in rs, at most 44 orbitals, an LDS image of the beta
+// strings, spectator rows of at most 1 GiB).  Its time against the fastest
+// form without blocks, of one product's mixed term: 60 x 60 strings 14 : 22
+// us, 275 x 239 38 : 72 us, 1543 x 1387 0.73 : 1.24 ms, 8000 x 8000 30.7 :
+// 43.5 ms, 11003 x 11003 111 : 180 ms.  SBDX_MIXED_EB or SBDX_MIXED_NT fix
+// one of the other kernels.
+static bool use_blk(Context &c) {
+  if (c.blk_mode < 0) {
+    bool on = c.mixed_eb[0] == 0 && !std::getenv("SBDX_MIXED_EB") && !std::getenv("SBDX_MIXED_NT") &&
+              sizeof(double) * (size_t)c.Kt * c.na <= ((size_t)1 << 30);
+    try {
+      if (on) build_blocks(c);
+      on = on && c.B.has_blk && blk_geom(c).nmw >= 0;
+      if (on) blk_tables(c);
+    } catch (const Error &e) {
+      if (e.code != 4) throw;  // SBDX_ERR_ALLOC
+      on = false;  // no room for the tables: the other kernels need none
+    }
+    if (on) c.mixed_eb[0] = kEbBlocks, c.mixed_nt[0] = blk_geom(c).nt;
+    c.blk_mode = on ? 1 : 0;
+  }
+  return c.blk_mode == 1;
 }
 
 template <typename T, int NT>
@@ -1296,16 +1889,16 @@ static bool mixed_parts_dispatch(Context &c, const T *eri, const T *x, T *y) {
 template <bool SYM = false>
 static bool mixed_ell_cfg(Context &c, int eb, int nt, const double *eri, const double *x, double *y) {
   return eb == kEbSigned ? mixed_sw_dispatch<double, SYM>(c, nt, eri, x, y)
-       : eb == 4 ? mixed_ell_dispatch<double, 4, SYM>(c, nt, eri, x, y)
-       : eb == 2 ? mixed_ell_dispatch<double, 2, SYM>(c, nt, eri, x, y)
-                 : mixed_ell_dispatch<double, 1, SYM>(c, nt, eri, x, y);
+         : eb == 4 ? mixed_ell_dispatch<double, 4, SYM>(c, nt, eri, x, y)
+         : eb == 2 ? mixed_ell_dispatch<double, 2, SYM>(c, nt, eri, x, y)
+                   : mixed_ell_dispatch<double, 1, SYM>(c, nt, eri, x, y);
 }
 template <bool SYM = false>
 static bool mixed_ell_cfg(Context &c, int eb, int nt, const float *eri, const float *x, float *y) {
   return eb == kEbSigned ? mixed_sw_dispatch<float, SYM>(c, nt, eri, x, y)
-       : eb == 4 ? mixed_ell_dispatch<float, 4, SYM>(c, nt, eri, x, y)
-       : eb == 2 ? mixed_ell_dispatch<float, 2, SYM>(c, nt, eri, x, y)
-                 : mixed_ell_dispatch<float, 1, SYM>(c, nt, eri, x, y);
+         : eb == 4 ? mixed_ell_dispatch<float, 4, SYM>(c, nt, eri, x, y)
+         : eb == 2 ? mixed_ell_dispatch<float, 2, SYM>(c, nt, eri, x, y)
+                   : mixed_ell_dispatch<float, 1, SYM>(c, nt, eri, x, y);
 }
 // Autotuner for the sliced-ELL mixed kernel: every (staging width EB in
 // {1, 2, 4, kEbSigned (k_mixed_sw)}, slots per thread NT in {1, 2, 4, 8})
@@ -1385,6 +1978,8 @@ static void sigma_mixed(Context &c, const T *eri, const T *x, T *y) {
   if (c.B.has_ell) {
     // tuned staging width and slots per thread, then row parts
     const int pi = sizeof(T) == 4 ? 1 : 0;
+    if constexpr (sizeof(T) == 8)
+      if (use_blk(c)) return mixed_blk(c, x, y);
     const int eb = mixed_cfg<T>(c, eri, x);
     if (eb > 0 && mixed_ell_cfg(c, eb, c.mixed_nt[pi], eri, x, y)) return check_launch("k_mixed_ell");
     if (mixed_parts_dispatch<T>(c, eri, x, y)) return check_launch("k_mixed_parts");

@@ -782,6 +782,289 @@ inline uint64_t bit_reverse(uint64_t v) {
 inline bool odd_below(uint64_t key, int orb) { return __builtin_popcountll(key & ((1ull << orb) - 1ull)) & 1; }
 }  // namespace
 
+// Tables of the mixed term's block kernel (SpinTables::bk_*).  Columns are
+// the particle blocks of the note above, sorted by the bit-reversed string
+// (the lowest orbitals, the hole pattern, first), so that consecutive
+// columns have nearly the same orbitals; 16 of them make a task over the 16
+// bk_mt orbitals most of their members use, and a member outside that list
+// keeps its singles in the entry table.  A column costs tiles x steps matrix
+// instructions per 16 columns and alpha single (4 cycles of a CU per tile,
+// step and column in FP64); an ordered pair in the entry table some 0.15.
+// They run on different units at the same time, so the line is drawn at
+// kColWorth pairs per tile and step.
+namespace {
+constexpr int kColWorth = 4;
+}
+
+// The alpha set's tables: bk_order, bk_ent.
+static void build_blocks_bra(Context &c, SpinTables &t, const std::vector<uint64_t> &strs) {
+  const int n = t.n, L = c.L;
+  auto put = [&](const void *src, size_t bytes) {
+    void *dst = dalloc(c, bytes);
+    if (bytes) SBDX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c.stream));
+    return dst;
+  };
+  std::vector<uint64_t> off, ent;
+  download_singles(c, t, off, ent);
+  // order of the bras: those with more than twice the average singles
+  // first (the last blocks of a launch are then short), the rest by the
+  // bit-reversed string, so that bras that run together share ket rows;
+  // the 32 blocks that run on one XCD at a time get neighbours
+  std::vector<uint32_t> ord(n);
+  for (int i = 0; i < n; i++) ord[i] = (uint32_t)i;
+  const double heavy = 2.0 * (double)t.ns / n;
+  std::vector<uint64_t> rev(n);
+  for (int i = 0; i < n; i++) rev[i] = bit_reverse(strs[i]);
+  std::stable_sort(ord.begin(), ord.end(), [&](uint32_t a, uint32_t b) {
+    const uint64_t la = off[a + 1] - off[a], lb = off[b + 1] - off[b];
+    const bool ha = (double)la > heavy, hb = (double)lb > heavy;
+    if (ha != hb) return ha;
+    return ha ? la > lb : rev[a] < rev[b];
+  });
+  std::vector<uint32_t> blk(ord);
+  for (int w = 0; w + 256 <= n; w += 256)
+    for (int b = 0; b < 256; b++) blk[w + b] = ord[w + (b & 7) * 32 + (b >> 3)];
+  t.bk_order = (uint32_t *)put(blk.data(), sizeof(uint32_t) * n);
+  std::vector<uint64_t> e2(t.ns + n);
+  for (int r = 0; r < n; r++) {
+    uint64_t *o = e2.data() + off[r] + r;
+    for (uint64_t k = off[r]; k < off[r + 1]; k++) {
+      const uint32_t pq = (uint32_t)((ent[k] >> 32) & 0x7fffffffull), a = pq / L, b = pq % L;
+      const uint64_t tri = a > b ? a * (a + 1) / 2 + b : b * (b + 1) / 2 + a;
+      *o++ = (ent[k] & 0xffffffffull) | (tri << 32) | (ent[k] & (1ull << 63));
+    }
+    *o = (uint64_t)r | (1ull << 62);
+  }
+  t.bk_ent = (uint64_t *)put(e2.data(), sizeof(uint64_t) * e2.size());
+  SBDX_HIP(hipStreamSynchronize(c.stream));
+}
+
+// The beta set's tables; has_blk where the form holds them.
+static void build_blocks_ket(Context &c, SpinTables &t, const std::vector<uint64_t> &strs) {
+  const int n = t.n, L = c.L, Kt = c.Kt;
+  auto put = [&](const void *src, size_t bytes) {
+    void *dst = dalloc(c, bytes);
+    if (bytes) SBDX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c.stream));
+    return dst;
+  };
+  t.has_blk = false;
+  if (!c.eri_rs_sym || 2 * Kt + 1 > 2048) return;
+  auto image = [&](int pb) { return ((size_t)2 * Kt + 1 + n + 1) << pb; };
+  if (n < 8192 && image(4) <= c.lds_limit) t.bk_pb = 4;
+  else if (n < 16384 && image(3) <= c.lds_limit) t.bk_pb = 3;
+  else return;
+  t.bk_mt = L <= 16 ? 1 : 2;
+  const int MT = t.bk_mt;
+  std::vector<uint64_t> off, ent;
+  download_singles(c, t, off, ent);
+  // ---- columns
+  std::vector<Member> pm;
+  pm.reserve((size_t)n * 16);
+  for (int r = 0; r < n; r++)
+    for (uint64_t o = strs[r]; o; o &= o - 1) {
+      const int u = __builtin_ctzll(o);
+      pm.push_back({strs[r] ^ (1ull << u), (uint32_t)r, (uint8_t)u});
+    }
+  std::sort(pm.begin(), pm.end(), [](const Member &a, const Member &b) {
+    return a.key < b.key || (a.key == b.key && a.orb < b.orb);
+  });
+  auto worth = [&](int m) { return m > 1 && m * (m - 1) >= kColWorth * MT * 4 * MT; };
+  struct Col {
+    uint64_t rev;
+    uint32_t first, m;
+  };
+  std::vector<Col> cols;
+  for (size_t i = 0; i < pm.size();) {
+    size_t j = i;
+    while (j < pm.size() && pm[j].key == pm[i].key) j++;
+    if (worth((int)(j - i))) cols.push_back({bit_reverse(pm[i].key), (uint32_t)i, (uint32_t)(j - i)});
+    i = j;
+  }
+  std::sort(cols.begin(), cols.end(), [](const Col &a, const Col &b) { return a.rev < b.rev; });
+  // ---- tasks
+  const int ntask = (int)((cols.size() + 15) / 16);
+  auto tri = [](int a, int b) { return a > b ? a * (a + 1) / 2 + b : b * (b + 1) / 2 + a; };
+  std::vector<uint32_t> step(1, 0u);
+  std::vector<uint2> tab;
+  const uint2 none = make_uint2((uint32_t)(2 * Kt) * 0x00010001u, (uint32_t)n);
+  // column of string r with the electron in u removed, where it is a member
+  std::vector<int32_t> col_of((size_t)n * L, -1);
+  // every string's accumulators: task, element | sign << 15
+  std::vector<std::vector<std::pair<int, uint16_t>>> pos_of(n);
+  for (int k = 0; k < ntask; k++) {
+    const size_t c0 = (size_t)16 * k, c1 = std::min(cols.size(), c0 + 16);
+    int use[64] = {};
+    for (size_t q = c0; q < c1; q++)
+      for (uint32_t i = 0; i < cols[q].m; i++) use[pm[cols[q].first + i].orb]++;
+    std::vector<int> list;
+    for (int u = 0; u < L; u++)
+      if (use[u]) list.push_back(u);
+    std::stable_sort(list.begin(), list.end(), [&](int a, int b) { return use[a] > use[b]; });
+    if ((int)list.size() > 16 * MT) list.resize(16 * MT);
+    std::sort(list.begin(), list.end());
+    int pos[64];
+    std::fill(pos, pos + 64, -1);
+    for (size_t i = 0; i < list.size(); i++) pos[list[i]] = (int)i;
+    const int nu = (int)list.size();
+    const size_t s0 = tab.size() / 64;
+    const int ns = 2 * ((nu + 7) / 8);  // the kernel takes two at a time
+    step.push_back((uint32_t)(s0 + ns));
+    tab.resize(tab.size() + (size_t)64 * ns, none);
+    for (int iv = 0; iv < nu; iv++)
+      for (int iu = 0; iu < nu; iu++) {
+        if (iu == iv) continue;
+        uint32_t &w = tab[(s0 + iv / 4) * 64 + 16 * (iv % 4) + iu % 16].x;
+        const int sh = 16 * (iu / 16);
+        w = (w & ~(0xffffu << sh)) | ((uint32_t)tri(list[iu], list[iv]) << sh);
+      }
+    for (size_t q = c0; q < c1; q++)
+      for (uint32_t i = 0; i < cols[q].m; i++) {
+        const Member &mb = pm[cols[q].first + i];
+        const int p = pos[mb.orb], cc = (int)(q - c0);
+        if (p < 0) continue;
+        const uint32_t v = mb.str | (odd_below(mb.key, mb.orb) ? 0x8000u : 0u);
+        tab[(s0 + p / 4) * 64 + 16 * (p % 4) + cc].y = v;
+        pos_of[mb.str].push_back({k, (uint16_t)(p * 16 + cc + ((v & 0x8000u) ? 0x8000u : 0u))});
+        col_of[(size_t)mb.str * L + mb.orb] = (int32_t)q;
+      }
+  }
+  t.bk_ntask = ntask;
+  // at the end a group's LDS holds a sum per string and, behind them, the
+  // accumulators of as many tasks at a time as its image has room for (more
+  // room is taken where one block fills a CU's LDS anyway)
+  const size_t unit = (size_t)MT * 256 * 8, sums = (size_t)8 * n;
+  size_t room = image(t.bk_pb);
+  if (room * 2 > c.lds_limit) room = c.lds_limit;
+  room = std::max(room, sums + unit);
+  t.bk_tp = (int)std::max<size_t>(1, std::min<size_t>({(room - sums) / unit, (size_t)std::max(ntask, 1), size_t{20}}));
+  t.bk_image = (std::max(image(t.bk_pb), sums + t.bk_tp * unit) + 15) / 16 * 16;
+  if (t.bk_image > c.lds_limit) return;
+  const int npass = (ntask + t.bk_tp - 1) / t.bk_tp;
+  std::vector<uint32_t> col_off;
+  std::vector<uint16_t> col_pos;
+  for (int q = 0; q < npass; q++) {
+    for (int r = 0; r < n; r++) {
+      col_off.push_back((uint32_t)col_pos.size());
+      for (const auto &v : pos_of[r])
+        if (v.first / t.bk_tp == q)
+          col_pos.push_back((uint16_t)(v.second + (v.first % t.bk_tp) * MT * 256));
+    }
+    col_off.push_back((uint32_t)col_pos.size());
+  }
+  t.bk_col_off = (uint32_t *)put(col_off.data(), sizeof(uint32_t) * col_off.size());
+  t.bk_col_pos = (uint16_t *)put(col_pos.data(), sizeof(uint16_t) * col_pos.size());
+  t.bk_nstep = (int)step.back();
+  tab.resize(tab.size() + 6 * 64, none);  // the kernel loads up to four steps ahead
+  t.bk_step = (uint32_t *)put(step.data(), sizeof(uint32_t) * step.size());
+  t.bk_tab = (uint2 *)put(tab.data(), sizeof(uint2) * tab.size());
+  // ---- the rest, entry by entry
+  auto covered = [&](int r, uint64_t e) {
+    const uint32_t pq = (uint32_t)((e >> 32) & 0x7fffffffull);
+    const int32_t a = col_of[(size_t)r * L + pq / L];
+    return a >= 0 && a == col_of[(e & 0xffffffffull) * L + pq % L];
+  };
+  std::vector<uint32_t> cnt(n, 0);
+  for (int r = 0; r < n; r++)
+    for (uint64_t k = off[r]; k < off[r + 1]; k++) cnt[r] += covered(r, ent[k]) ? 0 : 1;
+  // the reference string, when the rows differ from it in fewer orbitals
+  // than they have electrons
+  size_t nd = 0, ne = 0;
+  for (int r = 0; r < n; r++) {
+    nd += __builtin_popcountll(strs[r] ^ strs[0]);
+    ne += __builtin_popcountll(strs[r]);
+  }
+  t.bk_ref = nd < ne ? strs[0] : 0ull;
+  std::vector<uint32_t> order(n);
+  for (int i = 0; i < n; i++) order[i] = (uint32_t)i;
+  std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) {
+    const uint32_t ga = (cnt[a] + 3) / 4, gb = (cnt[b] + 3) / 4;
+    if (ga != gb) return ga > gb;
+    return __builtin_popcountll(strs[a] ^ t.bk_ref) > __builtin_popcountll(strs[b] ^ t.bk_ref);
+  });
+  const int nsl = (n + 63) / 64;
+  std::vector<uint32_t> perm((size_t)nsl * 64, (uint32_t)n), soff(nsl), len(nsl);
+  int most = 0;  // orbitals in which a row differs from the reference
+  for (int r = 0; r < n; r++) most = std::max(most, __builtin_popcountll(strs[r] ^ t.bk_ref));
+  t.bk_nrec = (most + 8) / 8;
+  std::vector<uint16_t> rec((size_t)nsl * t.bk_nrec * 64 * 8, (uint16_t)(2 * Kt));
+  uint32_t tot = 0;
+  for (int sl = 0; sl < nsl; sl++) {
+    uint32_t mx = 0, md = 0;
+    for (int l = 0; l < 64; l++) rec[((size_t)sl * t.bk_nrec * 64 + l) * 8] = (uint16_t)n;
+    for (int l = 0; l < 64 && sl * 64 + l < n; l++) {
+      const uint32_t r = order[(size_t)sl * 64 + l];
+      perm[(size_t)sl * 64 + l] = r;
+      mx = std::max(mx, (cnt[r] + 3) / 4);
+      rec[((size_t)sl * t.bk_nrec * 64 + l) * 8] = (uint16_t)r;
+      uint32_t q = 1;
+      for (uint64_t o = strs[r] ^ t.bk_ref; o; o &= o - 1, q++) {
+        const int k = __builtin_ctzll(o);
+        rec[(((size_t)sl * t.bk_nrec + q / 8) * 64 + l) * 8 + q % 8] =
+            (uint16_t)(k * (k + 3) / 2 + (((t.bk_ref >> k) & 1ull) ? Kt : 0));
+      }
+      md = std::max(md, q - 1);
+    }
+    soff[sl] = tot;
+    len[sl] = mx | (md << 16);
+    tot += mx;
+  }
+  // dealt in the word layout of schedule_slice_packed, whose fields hold LDS
+  // elements: the ket's 2 Kt + 1 + ket, the ERI value's triangle index
+  const uint32_t xe = 2u * (uint32_t)Kt + 1u;
+  std::vector<uint32_t> ell((size_t)(tot + 4) * 256);
+  const uint32_t pad = (xe + (uint32_t)n) << 4;
+  std::fill(ell.begin(), ell.end(), (uint32_t)n << t.bk_pb);
+  const int nthr = (int)std::max(1u, std::min({16u, std::thread::hardware_concurrency(), (unsigned)(nsl + 7) / 8}));
+  std::atomic<int> next{0};
+  auto worker = [&]() {
+    std::vector<uint32_t> rows[64], dealt;
+    for (int sl = next++; sl < nsl; sl = next++) {
+      uint32_t longest = 0;
+      for (int l = 0; l < 64; l++) {
+        rows[l].clear();
+        const uint32_t r = perm[(size_t)sl * 64 + l];
+        if (r == (uint32_t)n) continue;
+        for (uint64_t k = off[r]; k < off[r + 1]; k++) {
+          if (covered((int)r, ent[k])) continue;
+          const uint32_t pq = (uint32_t)((ent[k] >> 32) & 0x7fffffffull);
+          const uint32_t w = (uint32_t)tri((int)(pq / L), (int)(pq % L)) + ((ent[k] >> 63) ? (uint32_t)Kt : 0u);
+          rows[l].push_back(((xe + (uint32_t)(ent[k] & 0xffffffffull)) << 4) | (w << 19));
+        }
+        longest = std::max(longest, (uint32_t)rows[l].size());
+      }
+      const uint32_t ng4 = len[sl] & 0xffffu;
+      dealt.assign((size_t)ng4 * 4 * 64, pad);
+      schedule_slice_packed(rows, longest, pad, dealt.data(), t.bk_pb == 4);
+      uint32_t *o = ell.data() + (size_t)soff[sl] * 256;
+      for (uint32_t k = 0; k < 4 * ng4; k++)
+        for (int l = 0; l < 64; l++) {
+          const uint32_t w = dealt[(size_t)64 * k + l];
+          o[256 * (k / 4) + 4 * l + (k % 4)] = ((((w >> 4) & 0x7fffu) - xe) << t.bk_pb) | ((w >> 19) << 21);
+        }
+    }
+  };
+  std::vector<std::thread> pool;
+  for (int i = 1; i < nthr; i++) pool.emplace_back(worker);
+  worker();
+  for (auto &th : pool) th.join();
+  t.bk_nslice = nsl;
+  t.bk_ngroup = (int)tot;
+  t.bk_perm = (uint32_t *)put(perm.data(), sizeof(uint32_t) * perm.size());
+  t.bk_rec = (uint4 *)put(rec.data(), sizeof(uint16_t) * rec.size());
+  t.bk_off = (uint32_t *)put(soff.data(), sizeof(uint32_t) * nsl);
+  t.bk_len = (uint32_t *)put(len.data(), sizeof(uint32_t) * nsl);
+  t.bk_ell = (uint32_t *)put(ell.data(), sizeof(uint32_t) * ell.size());
+  SBDX_HIP(hipStreamSynchronize(c.stream));
+  t.has_blk = true;
+}
+
+// On a context's first FP64 product: one for FP32 or symmetric products,
+// density matrices or the diagonal needs none of this.
+void build_blocks(Context &c) {
+  build_blocks_ket(c, c.B, c.h_bstr);
+  if (c.B.has_blk) build_blocks_bra(c, c.A, c.h_astr);
+}
+
 void build_rdm_tables(Context &c, SpinTables &t, const std::vector<uint64_t> &strs, bool as_alpha, bool as_beta) {
   const int n = t.n, L = c.L;
   const size_t K = (size_t)c.K;
