@@ -8,13 +8,49 @@
 // masked popcount give each match its slot, so the order is ascending
 // without sorting.
 #include <algorithm>
-#include <array>
 #include <atomic>
+#include <exception>
+#include <mutex>
 #include <thread>
 
 #include "common.h"
 
+// host code only: the population count as an instruction
+#ifdef __HIP_DEVICE_COMPILE__
+#define SBDX_POPCNT
+#else
+#define SBDX_POPCNT __attribute__((target("popcnt")))
+#endif
+
 namespace sbdx {
+
+// fn(i) for i in [0, n) on up to 16 host threads (work independent per i);
+// an exception of any of them is rethrown here once all have ended.
+template <typename F>
+static void parallel_for(int n, const F &fn) {
+  const int nthr = std::max(1, std::min({16, (int)std::thread::hardware_concurrency(), n}));
+  std::atomic<int> next{0};
+  std::exception_ptr err;
+  std::mutex mu;
+  auto worker = [&]() {
+    try {
+      for (int i = next++; i < n; i = next++) fn(i);
+    } catch (...) {
+      std::lock_guard<std::mutex> lock(mu);
+      if (!err) err = std::current_exception();
+      next = n;
+    }
+  };
+  std::vector<std::thread> pool;
+  pool.reserve(nthr);
+  try {
+    for (int i = 1; i < nthr; i++) pool.emplace_back(worker);
+  } catch (...) {  // no more threads: those that run and this one do the work
+  }
+  worker();
+  for (auto &th : pool) th.join();
+  if (err) std::rethrow_exception(err);
+}
 
 __device__ __forceinline__ double parity1(uint64_t s, int a, int b) {
   // Reference parity rule (chemistry/basic/determinants.h:230-281) on one
@@ -290,12 +326,11 @@ static void schedule_slice(std::vector<uint32_t> *rows, uint32_t len, uint32_t p
   }
 }
 
-// Sliced-ELL layout of the singles of t with rows taken in `order`
-// (64 rows per slice); results in host vectors.
-static void ell_layout(Context &c, const SpinTables &t, const std::vector<uint64_t> &off,
-                       const std::vector<uint64_t> &ent, const std::vector<uint32_t> &order,
-                       std::vector<uint32_t> &perm, std::vector<uint32_t> &sl_len,
-                       std::vector<uint64_t> &sl_off, std::vector<uint32_t> &ell) {
+// Slices of the sliced-ELL layout with the rows of t taken in `order` (64
+// rows per slice); results in host vectors, returns the number of entries.
+static uint64_t ell_slices(const SpinTables &t, const std::vector<uint64_t> &off,
+                           const std::vector<uint32_t> &order, std::vector<uint32_t> &perm,
+                           std::vector<uint32_t> &sl_len, std::vector<uint64_t> &sl_off) {
   const int n = t.n;
   const int nsl = (n + 63) / 64;
   perm.assign((size_t)nsl * 64, 0xffffffffu);
@@ -313,26 +348,7 @@ static void ell_layout(Context &c, const SpinTables &t, const std::vector<uint64
     sl_off[s] = total;
     total += (uint64_t)mx * 64;
   }
-  const uint32_t pad = (uint32_t)c.K << 16;
-  // 4 x 64 padding entries past the end: the mixed kernel prefetches the
-  // next 4 positions of a slice unconditionally (past a slice's end it
-  // reads the next slice's entries or these, and never uses them)
-  ell.assign(total + 4 * 64 + 1, pad);
-  std::vector<uint32_t> rows[64];
-  for (int s = 0; s < nsl; s++) {
-    for (int l = 0; l < 64; l++) {
-      rows[l].clear();
-      const uint32_t r = perm[(size_t)s * 64 + l];
-      if (r == 0xffffffffu) continue;
-      for (uint64_t k = 0; k < off[r + 1] - off[r]; k++) {
-        const uint64_t e = ent[off[r] + k];
-        const uint32_t ket = (uint32_t)(e & 0xffffffffull);
-        const uint32_t pq = (uint32_t)((e >> 32) & 0x7fffffffull);
-        rows[l].push_back(ket | (pq << 16) | ((e >> 63) ? 0x80000000u : 0u));
-      }
-    }
-    schedule_slice(rows, sl_len[s], (uint32_t)c.K, (uint32_t)n, ell.data() + sl_off[s]);
-  }
+  return total;
 }
 
 // Packed entries of the staged mixed kernel (SpinTables::ell2): bits 4..18
@@ -364,12 +380,13 @@ static void ell_layout(Context &c, const SpinTables &t, const std::vector<uint64
 // grouping) to 5.2 (4 without conflicts).  4- and 8-byte reads follow
 // another rule (schedule_slice_packed), dealt by the same search.
 namespace qsched {
-// NL lanes per group, NR residues (a power of two, <= 32; NL == NR here)
+// NL lanes per group, NR residues (16 or 32; NL == NR here)
 template <int NR>
 struct Lane {
+  static constexpr int W = NR * NR / 64;
   std::vector<uint32_t> ent;
   uint16_t cnt[NR * NR];  // entries per (x, w) residue pair
-  uint32_t xw[NR];        // bit w of xw[x]: some entry has residues (x, w)
+  uint64_t have[W];       // bit x NR + w: some entry has residues (x, w)
 };
 template <int NR>
 static inline int rx(uint32_t w) { return (w >> 4) & (NR - 1); }
@@ -377,6 +394,7 @@ template <int NR>
 static inline int rw(uint32_t w) { return (w >> 19) & (NR - 1); }
 template <int NL, int NR>
 struct Search {
+  static constexpr int W = NR * NR / 64, XW = 64 / NR;  // residues x per word of a pair set
   Lane<NR> *L;
   int remx[NR], remw[NR];
   uint8_t ux[NR], uw[NR];
@@ -387,44 +405,43 @@ struct Search {
   int pick[NL];  // pair index x*NR+w, or -1 idle
   bool need[NL], done[NL];
   bool fits(int x, int w) const { return ux[x] < cx && uw[w] < cw; }
-  int options(int l, uint32_t wfree) const {
-    int n = 0;
-    for (int x = 0; x < NR; x++)
-      if (ux[x] < cx) n += __builtin_popcount(L[l].xw[x] & wfree);
-    return n;
-  }
-  uint32_t wfree_mask() const {
-    uint32_t m = 0;
-    for (int w = 0; w < NR; w++) if (uw[w] < cw) m |= 1u << w;
-    return m;
-  }
-  bool dfs(int depth) {
+  SBDX_POPCNT bool dfs(int depth) {
     if (depth == NL) return true;
     if (++nodes > limit) return false;
+    // the pairs whose residues are both below their bounds
+    uint64_t open[W], wf = 0;
+    for (int w = 0; w < NR; w++)
+      if (uw[w] < cw) wf |= 1ull << w;
+    for (int i = 0; i < W; i++) {
+      open[i] = 0;
+      for (int q = 0; q < XW; q++)
+        if (ux[i * XW + q] < cx) open[i] |= wf << (q * NR);
+    }
     int bl = -1, bn = 1 << 30;
-    const uint32_t wf = wfree_mask();
     for (int l = 0; l < NL; l++) {
       if (done[l]) continue;
-      int n = options(l, wf) + (need[l] ? 0 : 1);
+      int n = need[l] ? 0 : 1;
+      for (int i = 0; i < W; i++) n += __builtin_popcountll(L[l].have[i] & open[i]);
       if (n < bn) { bn = n; bl = l; }
     }
     if (bn == 0) return false;
     const int l = bl;
     done[l] = true;
-    std::array<std::pair<int, int>, NR * NR> cand;
+    // its candidates, the most loaded residues first (then the lowest pair);
+    // most searches take the first, so the order is found as it is needed
+    uint32_t cand[NR * NR];
     int nc = 0;
-    for (int x = 0; x < NR; x++) {
-      if (ux[x] >= cx) continue;
-      uint32_t m = L[l].xw[x] & wf;
-      while (m) {
-        const int w = __builtin_ctz(m);
-        m &= m - 1;
-        cand[nc++] = {-(remx[x] + remw[w]), x * NR + w};
+    for (int i = 0; i < W; i++)
+      for (uint64_t m = L[l].have[i] & open[i]; m; m &= m - 1) {
+        const int p = 64 * i + __builtin_ctzll(m);
+        cand[nc++] = ((uint32_t)(remx[p / NR] + remw[p % NR]) << 10) | (uint32_t)(NR * NR - 1 - p);
       }
-    }
-    std::sort(cand.begin(), cand.begin() + nc);
     for (int i = 0; i < nc; i++) {
-      const int p = cand[i].second, x = p / NR, w = p % NR;
+      int best = i;
+      for (int j = i + 1; j < nc; j++)
+        if (cand[j] > cand[best]) best = j;
+      std::swap(cand[i], cand[best]);
+      const int p = NR * NR - 1 - (int)(cand[i] & (NR * NR - 1)), x = p / NR, w = p % NR;
       ux[x]++; uw[w]++;
       pick[l] = p;
       if (dfs(depth + 1)) return true;
@@ -444,24 +461,26 @@ struct Search {
     return false;
   }
 };
-// rows[lanes[i]]: the NL lanes' entries (consumed); out[64*k + lanes[i]]
-template <int NL, int NR>
-static void deal_group(std::vector<uint32_t> *rows, const int *lanes, uint32_t len, uint32_t pad, uint32_t *out,
-                       long limit) {
+// rows(lane, v): puts lane's entries into v.  Entry k of lane l goes to
+// out[256 (k / 4) + 4 l + k % 4]: groups of 4 positions, each lane-major.
+template <int NL, int NR, typename F>
+static void deal_group(const F &rows, const int *lanes, uint32_t len, uint32_t pad, uint32_t *out, long limit) {
+  static_assert(NR * NR <= 1024, "a pair index takes 10 bits");
   std::vector<Lane<NR>> L(NL);
   Search<NL, NR> s;
   s.L = L.data();
   std::fill(s.remx, s.remx + NR, 0);
   std::fill(s.remw, s.remw + NR, 0);
   for (int l = 0; l < NL; l++) {
-    L[l].ent = rows[lanes[l]];
+    rows(lanes[l], L[l].ent);
     std::fill(L[l].cnt, L[l].cnt + NR * NR, 0);
-    std::fill(L[l].xw, L[l].xw + NR, 0);
+    std::fill(L[l].have, L[l].have + Lane<NR>::W, 0ull);
     for (uint32_t w : L[l].ent) {
-      L[l].cnt[rx<NR>(w) * NR + rw<NR>(w)]++;
-      L[l].xw[rx<NR>(w)] |= 1u << rw<NR>(w);
-      s.remx[rx<NR>(w)]++;
-      s.remw[rw<NR>(w)]++;
+      const int p = rx<NR>(w) * NR + rw<NR>(w);
+      L[l].cnt[p]++;
+      L[l].have[p / 64] |= 1ull << (p % 64);
+      s.remx[p / NR]++;
+      s.remw[p % NR]++;
     }
   }
   s.padx = rx<NR>(pad);
@@ -515,37 +534,34 @@ static void deal_group(std::vector<uint32_t> *rows, const int *lanes, uint32_t l
         auto &E = L[l].ent;
         for (size_t i = 0; i < E.size(); i++)
           if (rx<NR>(E[i]) * NR + rw<NR>(E[i]) == p) { w = E[i]; E[i] = E.back(); E.pop_back(); break; }
-        if (--L[l].cnt[p] == 0) L[l].xw[p / NR] &= ~(1u << (p % NR));
+        if (--L[l].cnt[p] == 0) L[l].have[p / 64] &= ~(1ull << (p % 64));
         s.remx[p / NR]--;
         s.remw[p % NR]--;
       }
-      out[(size_t)64 * k + lanes[l]] = w;
+      out[256 * (size_t)(k / 4) + 4 * lanes[l] + k % 4] = w;
     }
   }
 }
 }  // namespace qsched
 
-// The packed entries of one slice (rows: the 64 lanes' entries, consumed),
-// group by group: for 16-byte reads the 4 measured lane groups of 16 lanes
-// with residues mod 16; for 4- and 8-byte reads the two half-waves with
-// residues mod 32 (measured with the same probe: lanes of different
+// The packed entries of lane group g of one slice (rows(lane, v): a lane's
+// entries): for 16-byte reads one of the 4 measured lane groups of 16 lanes
+// with residues mod 16; for 4- and 8-byte reads one of the two half-waves
+// with residues mod 32 (measured with the same probe: lanes of different
 // half-waves never conflict, and two distinct addresses of one half-wave
 // conflict when their element indices agree mod 32).
-static void schedule_slice_packed(std::vector<uint32_t> *rows, uint32_t len, uint32_t pad, uint32_t *out,
-                                  bool wide) {
+static int lane_groups(bool wide) { return wide ? 4 : 2; }
+template <typename F>
+static void schedule_slice_packed(const F &rows, int g, uint32_t len, uint32_t pad, uint32_t *out, bool wide) {
   if (wide) {
-    for (int c = 0; c < 4; c++) {
-      int lanes[16], n = 0;
-      for (int l = 0; l < 64; l++)
-        if (((l >> 5) & 1) * 2 + (((l >> 4) ^ (l >> 3) ^ (l >> 2)) & 1) == c) lanes[n++] = l;
-      qsched::deal_group<16, 16>(rows, lanes, len, pad, out, 200);
-    }
+    int lanes[16], n = 0;
+    for (int l = 0; l < 64; l++)
+      if (((l >> 5) & 1) * 2 + (((l >> 4) ^ (l >> 3) ^ (l >> 2)) & 1) == g) lanes[n++] = l;
+    qsched::deal_group<16, 16>(rows, lanes, len, pad, out, 200);
   } else {
-    for (int c = 0; c < 2; c++) {
-      int lanes[32];
-      for (int l = 0; l < 32; l++) lanes[l] = 32 * c + l;
-      qsched::deal_group<32, 32>(rows, lanes, len, pad, out, 200);
-    }
+    int lanes[32];
+    for (int l = 0; l < 32; l++) lanes[l] = 32 * g + l;
+    qsched::deal_group<32, 32>(rows, lanes, len, pad, out, 200);
   }
 }
 
@@ -569,25 +585,18 @@ void build_singles_ell(Context &c, SpinTables &t) {
   std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) {
     return (off[a + 1] - off[a]) > (off[b + 1] - off[b]);
   });
-  std::vector<uint32_t> perm, sl_len, ell;
+  std::vector<uint32_t> perm, sl_len;
   std::vector<uint64_t> sl_off;
-  ell_layout(c, t, off, ent, order, perm, sl_len, sl_off, ell);
+  const uint64_t total = ell_slices(t, off, order, perm, sl_len, sl_off);
   const int nsl = (int)sl_len.size();
-  t.nslice = nsl;
-  t.ell = (uint32_t *)dalloc(c, sizeof(uint32_t) * ell.size());
-  t.perm = (uint32_t *)dalloc(c, sizeof(uint32_t) * perm.size());
-  t.sl_off = (uint64_t *)dalloc(c, sizeof(uint64_t) * nsl);
-  t.sl_len = (uint32_t *)dalloc(c, sizeof(uint32_t) * nsl);
-  SBDX_HIP(hipMemcpyAsync(t.ell, ell.data(), sizeof(uint32_t) * ell.size(), hipMemcpyHostToDevice, c.stream));
-  SBDX_HIP(hipMemcpyAsync(t.perm, perm.data(), sizeof(uint32_t) * perm.size(), hipMemcpyHostToDevice, c.stream));
-  SBDX_HIP(hipMemcpyAsync(t.sl_off, sl_off.data(), sizeof(uint64_t) * nsl, hipMemcpyHostToDevice, c.stream));
-  SBDX_HIP(hipMemcpyAsync(t.sl_len, sl_len.data(), sizeof(uint32_t) * nsl, hipMemcpyHostToDevice, c.stream));
-  SBDX_HIP(hipStreamSynchronize(c.stream));
-  t.has_ell = true;
+  // 4 x 64 padding entries past the end: the mixed kernel prefetches the
+  // next 4 positions of a slice unconditionally (past a slice's end it
+  // reads the next slice's entries or these, and never uses them)
+  std::vector<uint32_t> ell(total + 4 * 64 + 1, (uint32_t)c.K << 16);
   // the packed form for k_mixed_ell (same rows, slices and lengths)
   t.has_ell2 = false;
   t.has_ell3 = false;
-  if (c.K > 4096 || (size_t)c.K + (size_t)n > 32767) return;
+  const bool packed = c.K <= 4096 && (size_t)c.K + (size_t)n <= 32767;
   const uint32_t pad2 = ((uint32_t)(c.K + n)) << 4;
   // the reads the kernel will make: 16-byte values when four FP32 pairs fit
   // in LDS (the autotuner's choice whenever they do), else 4- or 8-byte ones
@@ -603,76 +612,78 @@ void build_singles_ell(Context &c, SpinTables &t) {
     sl_off2[sl] = total2;
     total2 += (uint64_t)sl_len2[sl] * 64;
   }
-  // deal every slice's entries (word_of: the packed word of one singles
-  // entry, pad the padding word) into the group layout; slices are
-  // independent and dealt on up to 16 host threads
-  auto deal_all = [&](auto word_of, uint32_t pad, std::vector<uint32_t> &dst) {
-    dst.assign(total2 + 2 * 256, pad);
-    const int nthr = (int)std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
-    std::atomic<int> next{0};
-    auto worker = [&]() {
-      std::vector<uint32_t> rows[64];
-      std::vector<uint32_t> dealt;
-      for (int sl = next++; sl < nsl; sl = next++) {
-        for (int l = 0; l < 64; l++) {
-          rows[l].clear();
-          const uint32_t r = perm[(size_t)sl * 64 + l];
-          if (r == 0xffffffffu) continue;
-          for (uint64_t k = off[r]; k < off[r + 1]; k++) rows[l].push_back(word_of(ent[k]));
-        }
-        const uint32_t len2 = sl_len2[sl];
-        dealt.assign((size_t)len2 * 64, pad);
-        schedule_slice_packed(rows, sl_len[sl], pad, dealt.data(), wide);
-        uint32_t *o = dst.data() + sl_off2[sl];
-        for (uint32_t k = 0; k < len2; k++)
-          for (int l = 0; l < 64; l++) o[256 * (k / 4) + 4 * l + (k % 4)] = dealt[(size_t)64 * k + l];
-      }
-    };
-    std::vector<std::thread> pool;
-    for (int i = 1; i < nthr; i++) pool.emplace_back(worker);
-    worker();
-    for (auto &th : pool) th.join();
-  };
-  std::vector<uint32_t> ell2;
-  deal_all(
-      [&](uint64_t e) {
-        const uint32_t ket = (uint32_t)(e & 0xffffffffull);
-        const uint32_t pq = (uint32_t)((e >> 32) & 0x7fffffffull);
-        return ((uint32_t)(c.K + ket) << 4) | (pq << 19) | ((e >> 63) ? 0x80000000u : 0u);
-      },
-      pad2, ell2);
   // the signed-triangle form: dealt in the ell2 word layout with the ket
   // element at 2048 + ket (the kernel's ket rows start at byte 32768 = 2048
   // 16-byte elements, so residues match the LDS addresses) and the signed
   // triangle index in the pq field, then repacked
-  if (c.eri_rs_sym && c.Kt <= 1024 && n < 8192 && wide) {
-    const uint32_t Kt = (uint32_t)c.Kt;
-    const int L = c.L;
-    std::vector<uint32_t> ell3;
-    deal_all(
-        [&](uint64_t e) {
-          const uint32_t ket = (uint32_t)(e & 0xffffffffull);
-          const uint32_t pq = (uint32_t)((e >> 32) & 0x7fffffffull);
-          const uint32_t a = pq / L, b = pq % L, hi = a > b ? a : b, lo = a > b ? b : a;
-          const uint32_t widx = hi * (hi + 1) / 2 + lo + ((e >> 63) ? Kt : 0u);
-          return ((2048u + ket) << 4) | (widx << 19);
-        },
-        (2048u + (uint32_t)n) << 4, ell3);
+  const bool triangle = packed && c.eri_rs_sym && c.Kt <= 1024 && n < 8192 && wide;
+  const uint32_t pad3 = (2048u + (uint32_t)n) << 4;
+  std::vector<uint32_t> ell2, ell3;
+  if (packed) ell2.assign(total2 + 2 * 256, pad2);
+  if (triangle) ell3.assign(total2 + 2 * 256, pad3);
+  // One item deals a slice's entries for `ell` or one lane group of a slice
+  // for a packed form; all are independent and run on the host's threads.
+  // The searches take nearly all of the build's time: for 2583 strings of 29
+  // orbitals (one thread for `ell`, one thread per slice for each packed form
+  // in turn) that was 37 of 49 ms; with this split and the searches' pair sets
+  // as bits the whole build takes 22 ms.
+  const int ng = lane_groups(wide), forms = 1 + (packed ? ng : 0) + (triangle ? ng : 0);
+  parallel_for(nsl * forms, [&](int item) {
+    const int sl = item / forms, f = item % forms;
+    auto each = [&](int l, auto take) {
+      const uint32_t r = perm[(size_t)sl * 64 + l];
+      if (r != 0xffffffffu)
+        for (uint64_t k = off[r]; k < off[r + 1]; k++)
+          take((uint32_t)(ent[k] & 0xffffffffull), (uint32_t)((ent[k] >> 32) & 0x7fffffffull), (uint32_t)(ent[k] >> 63));
+    };
+    if (f == 0) {
+      std::vector<uint32_t> rows[64];
+      for (int l = 0; l < 64; l++)
+        each(l, [&](uint32_t ket, uint32_t pq, uint32_t neg) { rows[l].push_back(ket | (pq << 16) | (neg << 31)); });
+      schedule_slice(rows, sl_len[sl], (uint32_t)c.K, (uint32_t)n, ell.data() + sl_off[sl]);
+    } else if (f <= ng) {
+      schedule_slice_packed(
+          [&](int l, std::vector<uint32_t> &v) {
+            each(l, [&](uint32_t ket, uint32_t pq, uint32_t neg) {
+              v.push_back((((uint32_t)c.K + ket) << 4) | (pq << 19) | (neg << 31));
+            });
+          },
+          f - 1, sl_len[sl], pad2, ell2.data() + sl_off2[sl], wide);
+    } else {
+      const uint32_t L = (uint32_t)c.L, Kt = (uint32_t)c.Kt;
+      schedule_slice_packed(
+          [&](int l, std::vector<uint32_t> &v) {
+            each(l, [&](uint32_t ket, uint32_t pq, uint32_t neg) {
+              const uint32_t a = pq / L, b = pq % L, hi = a > b ? a : b, lo = a > b ? b : a;
+              v.push_back(((2048u + ket) << 4) | ((hi * (hi + 1) / 2 + lo + (neg ? Kt : 0u)) << 19));
+            });
+          },
+          f - 1 - ng, sl_len[sl], pad3, ell3.data() + sl_off2[sl], wide);
+    }
+  });
+  auto put = [&](const void *src, size_t bytes) {
+    void *dst = dalloc(c, bytes);
+    SBDX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c.stream));
+    return dst;
+  };
+  t.nslice = nsl;
+  t.ell = (uint32_t *)put(ell.data(), sizeof(uint32_t) * ell.size());
+  t.perm = (uint32_t *)put(perm.data(), sizeof(uint32_t) * perm.size());
+  t.sl_off = (uint64_t *)put(sl_off.data(), sizeof(uint64_t) * nsl);
+  t.sl_len = (uint32_t *)put(sl_len.data(), sizeof(uint32_t) * nsl);
+  if (triangle) {
     for (uint32_t &w : ell3) w = ((((w >> 4) & 0x7fffu) - 2048u) << 4) | (((w >> 19) & 0xfffu) << 21);
-    t.ell3 = (uint32_t *)dalloc(c, sizeof(uint32_t) * ell3.size());
-    SBDX_HIP(hipMemcpyAsync(t.ell3, ell3.data(), sizeof(uint32_t) * ell3.size(), hipMemcpyHostToDevice,
-                            c.stream));
-    SBDX_HIP(hipStreamSynchronize(c.stream));
-    t.has_ell3 = true;
+    t.ell3 = (uint32_t *)put(ell3.data(), sizeof(uint32_t) * ell3.size());
   }
-  t.ell2 = (uint32_t *)dalloc(c, sizeof(uint32_t) * ell2.size());
-  t.sl_off2 = (uint64_t *)dalloc(c, sizeof(uint64_t) * nsl);
-  t.sl_len2 = (uint32_t *)dalloc(c, sizeof(uint32_t) * nsl);
-  SBDX_HIP(hipMemcpyAsync(t.ell2, ell2.data(), sizeof(uint32_t) * ell2.size(), hipMemcpyHostToDevice, c.stream));
-  SBDX_HIP(hipMemcpyAsync(t.sl_off2, sl_off2.data(), sizeof(uint64_t) * nsl, hipMemcpyHostToDevice, c.stream));
-  SBDX_HIP(hipMemcpyAsync(t.sl_len2, sl_len2.data(), sizeof(uint32_t) * nsl, hipMemcpyHostToDevice, c.stream));
+  if (packed) {
+    t.ell2 = (uint32_t *)put(ell2.data(), sizeof(uint32_t) * ell2.size());
+    t.sl_off2 = (uint64_t *)put(sl_off2.data(), sizeof(uint64_t) * nsl);
+    t.sl_len2 = (uint32_t *)put(sl_len2.data(), sizeof(uint32_t) * nsl);
+  }
   SBDX_HIP(hipStreamSynchronize(c.stream));
-  t.has_ell2 = true;
+  t.has_ell = true;
+  t.has_ell2 = packed;
+  t.has_ell3 = triangle;
 }
 
 // Ket-range parts of the sliced-ELL singles (SpinTables::pell): part p holds
@@ -1014,39 +1025,33 @@ static void build_blocks_ket(Context &c, SpinTables &t, const std::vector<uint64
   std::vector<uint32_t> ell((size_t)(tot + 4) * 256);
   const uint32_t pad = (xe + (uint32_t)n) << 4;
   std::fill(ell.begin(), ell.end(), (uint32_t)n << t.bk_pb);
-  const int nthr = (int)std::max(1u, std::min({16u, std::thread::hardware_concurrency(), (unsigned)(nsl + 7) / 8}));
-  std::atomic<int> next{0};
-  auto worker = [&]() {
-    std::vector<uint32_t> rows[64], dealt;
-    for (int sl = next++; sl < nsl; sl = next++) {
-      uint32_t longest = 0;
-      for (int l = 0; l < 64; l++) {
-        rows[l].clear();
-        const uint32_t r = perm[(size_t)sl * 64 + l];
-        if (r == (uint32_t)n) continue;
-        for (uint64_t k = off[r]; k < off[r + 1]; k++) {
-          if (covered((int)r, ent[k])) continue;
-          const uint32_t pq = (uint32_t)((ent[k] >> 32) & 0x7fffffffull);
-          const uint32_t w = (uint32_t)tri((int)(pq / L), (int)(pq % L)) + ((ent[k] >> 63) ? (uint32_t)Kt : 0u);
-          rows[l].push_back(((xe + (uint32_t)(ent[k] & 0xffffffffull)) << 4) | (w << 19));
-        }
-        longest = std::max(longest, (uint32_t)rows[l].size());
+  const bool wide = t.bk_pb == 4;
+  const int ng = lane_groups(wide);
+  parallel_for(nsl * ng, [&](int item) {
+    const int sl = item / ng;
+    const size_t words = (size_t)(len[sl] & 0xffffu) * 256;
+    std::vector<uint32_t> dealt(words, pad);
+    uint32_t longest = 0;
+    auto rows = [&](int l, std::vector<uint32_t> &v) {
+      const uint32_t r = perm[(size_t)sl * 64 + l];
+      if (r == (uint32_t)n) return;
+      for (uint64_t k = off[r]; k < off[r + 1]; k++) {
+        if (covered((int)r, ent[k])) continue;
+        const uint32_t pq = (uint32_t)((ent[k] >> 32) & 0x7fffffffull);
+        const uint32_t w = (uint32_t)tri((int)(pq / L), (int)(pq % L)) + ((ent[k] >> 63) ? (uint32_t)Kt : 0u);
+        v.push_back(((xe + (uint32_t)(ent[k] & 0xffffffffull)) << 4) | (w << 19));
       }
-      const uint32_t ng4 = len[sl] & 0xffffu;
-      dealt.assign((size_t)ng4 * 4 * 64, pad);
-      schedule_slice_packed(rows, longest, pad, dealt.data(), t.bk_pb == 4);
-      uint32_t *o = ell.data() + (size_t)soff[sl] * 256;
-      for (uint32_t k = 0; k < 4 * ng4; k++)
-        for (int l = 0; l < 64; l++) {
-          const uint32_t w = dealt[(size_t)64 * k + l];
-          o[256 * (k / 4) + 4 * l + (k % 4)] = ((((w >> 4) & 0x7fffu) - xe) << t.bk_pb) | ((w >> 19) << 21);
-        }
+    };
+    for (int l = 0; l < 64; l++) {
+      const uint32_t r = perm[(size_t)sl * 64 + l];
+      if (r != (uint32_t)n) longest = std::max(longest, cnt[r]);
     }
-  };
-  std::vector<std::thread> pool;
-  for (int i = 1; i < nthr; i++) pool.emplace_back(worker);
-  worker();
-  for (auto &th : pool) th.join();
+    schedule_slice_packed(rows, item % ng, longest, pad, dealt.data(), wide);
+    // repacked lane by lane: a padding word stays as `ell` was filled
+    uint32_t *o = ell.data() + (size_t)soff[sl] * 256;
+    for (size_t i = 0; i < words; i++)
+      if (dealt[i] != pad) o[i] = ((((dealt[i] >> 4) & 0x7fffu) - xe) << t.bk_pb) | ((dealt[i] >> 19) << 21);
+  });
   t.bk_nslice = nsl;
   t.bk_ngroup = (int)tot;
   t.bk_perm = (uint32_t *)put(perm.data(), sizeof(uint32_t) * perm.size());
