@@ -169,10 +169,11 @@ int sbdx_set_restart(sbdx_handle_t h, int keep);
 
 /* Form of the same-spin terms chosen for precision 0 (FP64) or 1 (FP32) (no
  * counterpart in the reference): -1 not chosen yet (no sigma of that
- * precision so far), 0 sparse row kernels, 1 dense GEMMs over the same-spin
- * blocks.  The choice is made on the first sigma of each precision by timing
+ * precision so far), 0 sparse row kernels, 1 matrix products over the
+ * same-spin blocks.  The choice is made on the first sigma of each precision:
+ * FP64 by the sets' sizes and numbers of singles and doubles, FP32 by timing
  * both forms; ms_* receive those timings (0 when a form was not timed, e.g.
- * when SBDX_SAME_SPIN=sparse|dense in the environment fixed it). */
+ * in FP64 or when SBDX_SAME_SPIN=sparse|dense in the environment fixed it). */
 int sbdx_same_spin_form(sbdx_handle_t h, int precision, int *form, float *ms_sparse,
                         float *ms_dense);
 

@@ -153,6 +153,15 @@ struct SpinTables {
   std::vector<uint32_t *> psl_len;
 };
 
+// One spin's same-spin block as tiles of `tm` rows, each over the list of the
+// kets that its rows meet (same.hip).  rows: [ntile * tm] strings (>= n past
+// the end); list and val of tile t from base[t] on (multiples of a stage).
+struct SameTiles {
+  int tm = 0, ntile = 0;
+  uint32_t *rows = nullptr, *base = nullptr, *list = nullptr;
+  double *val = nullptr;
+};
+
 struct ProfSlot {
   std::vector<std::pair<hipEvent_t, hipEvent_t>> ev;
   long launches = 0;
@@ -205,11 +214,14 @@ struct Context {
   // Same-spin blocks as dense symmetric matrices for the GEMM form of the
   // same-spin terms (row-major n x n; the beta block aliases the alpha one
   // when the string sets are equal), FP64 and FP32, built on first use.
+  // (FP64: only for small sets; larger ones as tiles.)
   double *Hd_a = nullptr, *Hd_b = nullptr;
+  SameTiles tiles_a, tiles_b;
   float *Hf_a = nullptr, *Hf_b = nullptr;
   void *blas = nullptr;  // rocblas_handle bound to `stream`
   // Same-spin form per precision [0 FP64, 1 FP32]: -1 not chosen yet,
-  // 0 sparse row kernels, 1 dense GEMM; the timings that decided it (ms).
+  // 0 sparse row kernels, 1 matrix products; for FP32 the timings that
+  // decided it (ms).
   int same_mode[2] = {-1, -1};
   float same_ms[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
   // Sliced-ELL mixed kernel configuration per form (0 FP64, 1 FP32 general;
@@ -398,6 +410,16 @@ void host_syev(int n, double *A, double *Q, double *E);
 // dimension ld: S-orthonormal eigenvectors Y (n x n, ld n), E ascending
 void host_sygv(int n, const double *H, const double *S, int ld, double *Y, double *E);
 void transpose_into(Context &c, const double *in, double *out, int R, int Cc);  // out = in^T
+void transpose_add(Context &c, const double *in, double *out, int R, int Cc);   // out += in^T
+void dense_blocks(Context &c, double *&Ha, double *&Hb);  // the same-spin blocks, dense, built on first use
+
+// same.hip
+constexpr size_t kSameSmall = 1200;  // na + nb up to which both same-spin terms are one launch
+size_t same_mm_bytes(const Context &c);  // at most, for what is not built yet
+bool same_mm_fits(const Context &c);
+bool same_mm_worth(const Context &c);
+void same_mm(Context &c, const double *x, double *y, double *xt, double *yt);
+void same_mm_alpha(Context &c, const double *x, double *G);
 
 // davidson.hip
 int davidson_solve(Context &c, int max_it, int nb, double eps, double max_time, double *energy,

@@ -7,10 +7,9 @@
 // spin so every product is a coalesced row operation and no atomics are
 // needed:
 //   same-spin         y = hii*x + H_a X + X H_b with X the na x nb vector:
-//                     either two dense GEMMs (the same-spin blocks H_a, H_b
-//                     are symmetric and, at selected-CI sizes, ~5-15% full
-//                     with no empty tiles) or sparse row kernels (x and its
-//                     transpose); the faster is picked on first use
+//                     either matrix products (FP64: tiles over lists of kets,
+//                     same.hip; FP32: two dense GEMMs) or sparse row kernels
+//                     (x and its transpose); see same_mode
 //   mixed alpha-beta  y[I,:] += sum_{J in S_a(I)} s_a V_pq * x[J,:] gathered
 //                     through the beta-singles table, with x[J,:] and the
 //                     ERI row V_pq staged in LDS.
@@ -1525,6 +1524,10 @@ void transpose_into(Context &c, const double *in, double *out, int R, int Cc) {
   transpose<double>(c, in, out, R, Cc, false);
 }
 
+void transpose_add(Context &c, const double *in, double *out, int R, int Cc) {
+  transpose<double>(c, in, out, R, Cc, true);
+}
+
 // Rows of the mixed term are split over ceil(slots / (1024*NT)) blocks.
 template <typename T, int NT, int EB, bool SYM>
 static void launch_mixed_ell(Context &c, const T *eri, const T *x, T *y, size_t lds) {
@@ -2116,7 +2119,7 @@ static T *densify(Context &c, const SpinTables &t) {
   return H;
 }
 
-static void dense_blocks(Context &c, double *&Ha, double *&Hb) {
+void dense_blocks(Context &c, double *&Ha, double *&Hb) {
   if (!c.Hd_a) {
     c.Hd_a = densify<double>(c, c.A);
     c.Hd_b = c.B.alias ? c.Hd_a : densify<double>(c, c.B);
@@ -2146,17 +2149,21 @@ static rocblas_status gemm(rocblas_handle h, int m, int n, int k, const float *A
                        ldb, &beta, C, ldc);
 }
 
-// y = hii*x + H_a X + X H_b.  Column-major, the na x nb row-major X is the
+// y = hii*x + H_a X + X H_b: FP64 on tiles (same.hip), FP32 as GEMMs over the
+// dense blocks.  Column-major, the na x nb row-major X is the
 // nb x na matrix X^T, so with symmetric H_a, H_b:
 //   (H_a X)^T = X^T H_a   -> gemm(nb, na, na, X^T, H_a)
 //   (X H_b)^T = H_b X^T   -> gemm(nb, na, nb, H_b, X^T)
-template <typename T>
-static void same_dense(Context &c, const T *hii, const T *x, T *y) {
-  T *Ha, *Hb;
+static void same_dense(Context &c, const SigmaOperands<double> &o, const double *x, double *y) {
+  same_mm(c, x, y, o.T1, o.T2);
+}
+static void same_dense(Context &c, const SigmaOperands<float> &o, const float *x, float *y) {
+  const float *hii = o.hii;
+  float *Ha, *Hb;
   dense_blocks(c, Ha, Hb);
   const int na = (int)c.na, nb = (int)c.nb;
   const unsigned g = (unsigned)std::min<size_t>(cdiv(c.N, 256), 65536);
-  hipLaunchKernelGGL((k_diag_mul<T>), dim3(g), dim3(256), 0, c.stream, c.N, hii, x, y);
+  hipLaunchKernelGGL((k_diag_mul<float>), dim3(g), dim3(256), 0, c.stream, c.N, hii, x, y);
   check_launch("k_diag_mul");
   rocblas_handle h = blas(c);
   if (gemm(h, nb, na, na, x, nb, Ha, na, y, nb) != rocblas_status_success)
@@ -2165,13 +2172,6 @@ static void same_dense(Context &c, const T *hii, const T *x, T *y) {
     throw Error(3, "same-spin beta GEMM failed");
 }
 
-static rocblas_status gemm_batched(rocblas_handle h, int m, int n, int k, const double *A, int lda,
-                                   rocblas_stride sa, const double *B, int ldb, rocblas_stride sb,
-                                   double *C, int ldc, rocblas_stride sc, int batch) {
-  const double one = 1.0;
-  return rocblas_dgemm_strided_batched(h, rocblas_operation_none, rocblas_operation_none, m, n, k,
-                                       &one, A, lda, sa, B, ldb, sb, &one, C, ldc, sc, batch);
-}
 static rocblas_status gemm_batched(rocblas_handle h, int m, int n, int k, const float *A, int lda,
                                    rocblas_stride sa, const float *B, int ldb, rocblas_stride sb,
                                    float *C, int ldc, rocblas_stride sc, int batch) {
@@ -2180,19 +2180,23 @@ static rocblas_status gemm_batched(rocblas_handle h, int m, int n, int k, const 
                                        &one, A, lda, sa, B, ldb, sb, &one, C, ldc, sc, batch);
 }
 
-// Dense form for k contiguous vectors: the alpha term as a strided batch
+static void same_dense_block(Context &c, const SigmaOperands<double> &o, int k, const double *x, double *y) {
+  for (int v = 0; v < k; v++) same_mm(c, x + v * c.N, y + v * c.N, o.T1, o.T2);
+}
+
+// FP32 dense form for k contiguous vectors: the alpha term as a strided batch
 // over the vectors (shared H_a), the beta term as one GEMM over all k*na
 // columns of the side-by-side X^T blocks.
-template <typename T>
-static void same_dense_block(Context &c, const T *hii, int k, const T *x, T *y) {
-  T *Ha, *Hb;
+static void same_dense_block(Context &c, const SigmaOperands<float> &o, int k, const float *x, float *y) {
+  const float *hii = o.hii;
+  float *Ha, *Hb;
   dense_blocks(c, Ha, Hb);
   const int na = (int)c.na, nb = (int)c.nb;
   const size_t N = c.N;
   if ((size_t)k * na >= (1ull << 31)) throw Error(3, "block sigma: too many columns for one GEMM");
   const unsigned g = (unsigned)std::min<size_t>(cdiv(N, 256), 65536);
   for (int v = 0; v < k; v++) {
-    hipLaunchKernelGGL((k_diag_mul<T>), dim3(g), dim3(256), 0, c.stream, N, hii, x + v * N, y + v * N);
+    hipLaunchKernelGGL((k_diag_mul<float>), dim3(g), dim3(256), 0, c.stream, N, hii, x + v * N, y + v * N);
     check_launch("k_diag_mul");
   }
   rocblas_handle h = blas(c);
@@ -2225,28 +2229,30 @@ static void same_sparse(Context &c, const SigmaOperands<T> &o, const T *x, T *y)
   }
 }
 
-// Autotuner for the same-spin form: when the dense blocks fit (below a
-// quarter of free device memory, 32-bit GEMM dimensions), time both forms
-// on this x (second of two runs each, HIP events on the handle's stream;
-// both overwrite y, which the caller's real pass overwrites again) and keep
-// the faster for this precision.  SBDX_SAME_SPIN=sparse|dense overrides.
+// The same-spin form: row kernels unless the matrix form's operands fit
+// (below a quarter of free device memory, 32-bit dimensions).  FP64 goes by
+// same_mm_worth.  FP32: time both forms on this x (second of two runs each,
+// HIP events on the handle's stream; both overwrite y, which the caller's
+// real pass overwrites again) and keep the faster.
+// SBDX_SAME_SPIN=sparse|dense overrides.
 template <typename T>
 static int same_mode(Context &c, const SigmaOperands<T> &o, const T *x, T *y) {
   const int pi = sizeof(T) == 4 ? 1 : 0;
   if (c.same_mode[pi] >= 0) return c.same_mode[pi];
   const char *env = std::getenv("SBDX_SAME_SPIN");
   const size_t na = c.na, nb = c.nb;
-  const size_t bytes = sizeof(T) * (na * na + (c.B.alias ? 0 : nb * nb));
+  const size_t bytes = sizeof(T) == 8 ? same_mm_bytes(c) : sizeof(T) * (na * na + (c.B.alias ? 0 : nb * nb));
   size_t free_b = 0, total_b = 0;
   SBDX_HIP(hipMemGetInfo(&free_b, &total_b));
   const bool fits = na < (1u << 31) && nb < (1u << 31) && na * nb < (1ull << 31) &&
-                    bytes < free_b / 4;
+                    bytes < free_b / 4 && (sizeof(T) == 4 || same_mm_fits(c));
   if (env && std::string(env) == "sparse") return c.same_mode[pi] = 0;
   if (env && std::string(env) == "dense") {
     if (!fits) throw Error(3, "SBDX_SAME_SPIN=dense: same-spin blocks do not fit");
     return c.same_mode[pi] = 1;
   }
   if (!fits) return c.same_mode[pi] = 0;
+  if (sizeof(T) == 8) return c.same_mode[pi] = same_mm_worth(c) ? 1 : 0;
   hipEvent_t e0, e1;
   SBDX_HIP(hipEventCreate(&e0));
   SBDX_HIP(hipEventCreate(&e1));
@@ -2257,7 +2263,7 @@ static int same_mode(Context &c, const SigmaOperands<T> &o, const T *x, T *y) {
       if (mode == 0)
         same_sparse<T>(c, o, x, y);
       else
-        same_dense<T>(c, o.hii, x, y);
+        same_dense(c, o, x, y);
       SBDX_HIP(hipEventRecord(e1, c.stream));
       SBDX_HIP(hipEventSynchronize(e1));
       SBDX_HIP(hipEventElapsedTime(&ms[mode], e0, e1));
@@ -2275,7 +2281,7 @@ static void sigma_impl(Context &c, const T *x, T *y) {
   const bool f32 = sizeof(T) == 4;
   if (same_mode<T>(c, o, x, y) == 1) {
     ProfScope ps(c, f32 ? "same_gemm_f32" : "same_gemm");
-    same_dense<T>(c, o.hii, x, y);
+    same_dense(c, o, x, y);
   } else {
     same_sparse<T>(c, o, x, y);
   }
@@ -2345,14 +2351,20 @@ static void sym_same_split(Context &c, const float *hii, const float *x, float *
   check_launch("k_sym_combine");
 }
 
-// The symmetric same-spin term with the GEMM in the element type itself.
+static void sym_product(Context &c, const double *x, double *G) { same_mm_alpha(c, x, G); }
+static void sym_product(Context &c, const float *x, float *G) {
+  const int n = (int)c.na;
+  float *Ha, *Hb;
+  dense_blocks(c, Ha, Hb);
+  if (gemm(blas(c), n, n, n, x, n, Ha, n, G, n, 0.0f) != rocblas_status_success)
+    throw Error(3, "symmetric same-spin GEMM failed");
+}
+
+// The symmetric same-spin term with the product in the element type itself.
 template <typename T>
 static void sym_same_gemm(Context &c, const SigmaOperands<T> &o, const T *x, T *y) {
   const int n = (int)c.na;
-  T *Ha, *Hb;
-  dense_blocks(c, Ha, Hb);
-  if (gemm(blas(c), n, n, n, x, n, Ha, n, o.T1, n, T(0)) != rocblas_status_success)
-    throw Error(3, "symmetric same-spin GEMM failed");
+  sym_product(c, x, o.T1);
   hipLaunchKernelGGL((k_sym_combine<T>), dim3(cdiv(n, 64), cdiv(n, 64)), dim3(256), 0, c.stream, n, o.hii, x,
                      (const T *)o.T1, y, (const float *)nullptr, c.sym_par < 0 ? 1 : 0);
   check_launch("k_sym_combine");
@@ -2624,9 +2636,9 @@ static bool sym_ok(Context &c) {
   if (!c.B.alias || !c.B.has_ell || c.na != c.nb) return false;
   size_t free_b = 0, total_b = 0;
   SBDX_HIP(hipMemGetInfo(&free_b, &total_b));
-  const size_t bytes = (c.Hd_a ? 0 : sizeof(double) * c.na * c.na) +
+  const size_t bytes = same_mm_bytes(c) +
                        (c.f32.ready && !c.Hf_a ? sizeof(float) * c.na * c.na : 0);
-  return c.na < (1u << 31) && c.N < (1ull << 31) && bytes < free_b / 4;
+  return c.na < (1u << 31) && c.N < (1ull << 31) && bytes < free_b / 4 && same_mm_fits(c);
 }
 
 // sigma for a spin-flip symmetric x (x = x^T as an na x na matrix, equal
@@ -2778,7 +2790,7 @@ static void sigma_block_impl(Context &c, int k, const T *x, T *y) {
   const size_t N = c.N;
   if (same_mode<T>(c, o, x, y) == 1) {
     ProfScope ps(c, f32 ? "blk_same_gemm_f32" : "blk_same_gemm");
-    same_dense_block<T>(c, o.hii, k, x, y);
+    same_dense_block(c, o, k, x, y);
   } else {
     for (int v = 0; v < k; v++) same_sparse<T>(c, o, x + v * N, y + v * N);
   }
