@@ -23,6 +23,7 @@
 
 namespace sbdx {
 
+typedef double d4 __attribute__((ext_vector_type(4)));
 static inline unsigned cdiv(size_t a, size_t b) { return (unsigned)((a + b - 1) / b); }
 
 __device__ __forceinline__ double parity1r(uint64_t s, int a, int b) {
@@ -150,9 +151,143 @@ __global__ void __launch_bounds__(256) k_rdm_double_pairs(int n, int M, uint64_t
   }
 }
 
-// The same double pairs from the Gram matrix G = w w^T of this spin's n rows
-// (one library GEMM per spin instead of a dot product per pair):
-// out[e - e0] = sign * G[I, J]
+// The Gram matrix G = w w^T of n rows of M values, its lower triangle (tiles
+// across the diagonal whole).  A wave holds 16 T x 16 T elements over all
+// columns, a block 2 x 2 waves (KS 1); or half the columns, a block two tiles
+// side by side and their sums added in LDS (KS 2: for few rows, where whole
+// tiles would leave SIMDs idle).  Operands come straight from memory into
+// registers, PD - 1 stages of 8 columns ahead: lane group g of both operands
+// takes columns 2 g and 2 g + 1 (a 16-byte load per row) as the k of two
+// matrix steps.  Bound by the matrix instructions (16 of 64 cycles per KB of
+// operands at T = 4).  The library's product does the whole matrix: 8000 rows
+// of 8000 15.5 ms, here 9.3;
+// 2583 of 1387 and the transpose 0.51 ms together, here 0.42; 500 of 500 20 us,
+// here 15.
+template <int T, int KS>
+__global__ void __launch_bounds__(256, T == 4 ? 2 : 4) k_rdm_gram(int n, int M, unsigned total,
+                                                                 const double *__restrict__ w,
+                                                                 double *__restrict__ G) {
+  constexpr int PD = T == 4 ? 2 : 4, D = PD - 1;
+  // blocks of one XCD take neighbouring tiles (tile row by tile row)
+  const unsigned per = (total + 7) / 8, id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if ((blockIdx.x >> 3) >= per || id >= total) return;
+  const unsigned tile = id / KS;
+  int bi = (int)((sqrt(8.0 * tile + 1.0) - 1.0) * 0.5);
+  while ((unsigned)bi * (bi + 1) / 2 > tile) bi--;
+  while ((unsigned)(bi + 1) * (bi + 2) / 2 <= tile) bi++;
+  const int bj = (int)(tile - (unsigned)bi * (bi + 1) / 2);
+  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, q = lane & 15, g = lane >> 4, half = wv >> 1;
+  const int i0 = (2 * bi + (KS == 2 ? (int)(id & 1) : half)) * 16 * T, j0 = (2 * bj + (wv & 1)) * 16 * T;
+  const bool mine = j0 <= i0 && i0 < n;
+  if (KS == 1 && !mine) return;
+  typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));  // rows of odd length: any element
+  const double *pa[T], *pb[T];
+#pragma unroll
+  for (int f = 0; f < T; f++) {
+    pa[f] = w + (size_t)min(i0 + 16 * f + q, n - 1) * M;
+    pb[f] = w + (size_t)min(j0 + 16 * f + q, n - 1) * M;
+  }
+  d4 acc[T][T];
+#pragma unroll
+  for (int f = 0; f < T; f++)
+#pragma unroll
+    for (int j = 0; j < T; j++) acc[f][j] = d4{0.0, 0.0, 0.0, 0.0};
+  struct Ops {
+    d2u a[T], b[T];
+  };
+  auto mac = [&](const Ops &o) {
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int f = 0; f < T; f++)
+#pragma unroll
+        for (int j = 0; j < T; j++)
+          acc[f][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(u ? o.a[f].y : o.a[f].x, u ? o.b[j].y : o.b[j].x,
+                                                           acc[f][j], 0, 0, 0);
+  };
+  const int all = M / 8, first = KS == 2 && half ? all / 2 : 0;
+  const int end = !mine ? 0 : KS == 2 && !half ? all / 2 : all;
+  if (first < end) {
+    auto fetch = [&](int s, Ops &o) {
+      const int k = 8 * min(s, end - 1) + 2 * g;
+#pragma unroll
+      for (int f = 0; f < T; f++) {
+        o.a[f] = *reinterpret_cast<const d2u *>(pa[f] + k);
+        o.b[f] = *reinterpret_cast<const d2u *>(pb[f] + k);
+      }
+    };
+    Ops o[PD];
+#pragma unroll
+    for (int p = 0; p < D; p++) fetch(first + p, o[p]);
+    int s = first;
+    for (; s + PD <= end; s += PD)
+#pragma unroll
+      for (int p = 0; p < PD; p++) {
+        fetch(s + p + D, o[(p + D) % PD]);
+        mac(o[p]);
+        __builtin_amdgcn_sched_barrier(0);  // keep the stages' loads in this order
+      }
+#pragma unroll
+    for (int p = 0; p < D; p++)
+      if (s + p < end) mac(o[p]);
+  }
+  if (M % 8 && mine && (KS == 1 || half)) {  // the columns left over, zeros past them
+    const int k = 8 * all + 2 * g;
+    Ops o;
+#pragma unroll
+    for (int f = 0; f < T; f++) {
+      o.a[f] = d2u{k < M ? pa[f][k] : 0.0, k + 1 < M ? pa[f][k + 1] : 0.0};
+      o.b[f] = d2u{k < M ? pb[f][k] : 0.0, k + 1 < M ? pb[f][k + 1] : 0.0};
+    }
+    mac(o);
+  }
+  if constexpr (KS == 2) {
+    __shared__ d4 other[2][T * T][64];
+    if (half)
+#pragma unroll
+      for (int f = 0; f < T; f++)
+#pragma unroll
+        for (int j = 0; j < T; j++) other[wv & 1][f * T + j][lane] = acc[f][j];
+    __syncthreads();
+    if (half || !mine) return;
+#pragma unroll
+    for (int f = 0; f < T; f++)
+#pragma unroll
+      for (int j = 0; j < T; j++) acc[f][j] += other[wv & 1][f * T + j][lane];
+  }
+#pragma unroll
+  for (int f = 0; f < T; f++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int i = i0 + 16 * f + 4 * r + g;
+      if (i >= n) continue;
+#pragma unroll
+      for (int j = 0; j < T; j++) {
+        const int c = j0 + 16 * j + q;
+        if (c < n) G[(size_t)i * n + c] = acc[f][j][r];
+      }
+    }
+}
+
+// Tiles of 64 x 64 where they give every SIMD two waves, else of 32 x 32.
+static void rdm_gram(Context &c, int n, int M, const double *w, double *G) {
+  auto tiles = [&](int T) {
+    const size_t b = cdiv(n, 32 * T);
+    return b * (b + 1) / 2;
+  };
+  const bool wide = tiles(4) >= 2 * (size_t)c.n_cu;
+  const size_t total = wide ? tiles(4) : 2 * tiles(2);
+  if (total >= (1u << 28)) throw Error(3, "rdm: Gram matrix too large for one launch");
+  const dim3 grid((unsigned)((total + 7) / 8 * 8));
+  if (wide)
+    hipLaunchKernelGGL((k_rdm_gram<4, 1>), grid, dim3(256), 0, c.stream, n, M, (unsigned)total, w, G);
+  else
+    hipLaunchKernelGGL((k_rdm_gram<2, 2>), grid, dim3(256), 0, c.stream, n, M, (unsigned)total, w, G);
+  check_launch("k_rdm_gram");
+}
+
+// The same double pairs from the Gram matrix (its lower triangle) instead of a
+// dot product per pair: out[e - e0] = sign * G[I, J]
 __global__ void __launch_bounds__(256) k_rdm_double_gram(int n, uint64_t e0, uint64_t e1,
                                                          const uint64_t *__restrict__ d_off,
                                                          const uint32_t *__restrict__ d_ket,
@@ -169,7 +304,7 @@ __global__ void __launch_bounds__(256) k_rdm_double_gram(int n, uint64_t e0, uin
   const uint64_t bra = str[I];
   double sg = parity1r(bra, i, a) * parity1r(bra, j, b);
   if (a > j || b < i) sg = -sg;
-  out[e - e0] = sg * G[(size_t)I * n + J];
+  out[e - e0] = sg * G[J < (size_t)I ? (size_t)I * n + J : J * n + I];
 }
 
 // Same-spin OneDiff scatter for the single pairs e0 <= e < e1 of one spin:
@@ -192,7 +327,8 @@ __global__ void k_rdm_single_scatter(int n, int L, int spin, uint64_t e0, uint64
   if (T) {
     t0 = T[e - e0];
   } else {
-    const double g = G[(size_t)I * n + (uint32_t)(ent & 0xffffffffull)];
+    const size_t J = (uint32_t)(ent & 0xffffffffull);
+    const double g = G[J < (size_t)I ? (size_t)I * n + J : J * n + I];
     t0 = (ent >> 63) ? -g : g;
   }
   atomicAdd(&one[spin * L2 + p + (size_t)L * q], t0);
@@ -260,7 +396,6 @@ constexpr int kMmThreads = 512;
 constexpr int kMmWaves = kMmThreads / 64;
 constexpr int kMmRho = 16;  // x y products per thread kept in registers (ROWS): nb <= 8192
 
-typedef double d4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ double signed_by(double v, uint32_t high) {
   return __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, v) ^ ((uint64_t)high << 32));
 }
@@ -610,12 +745,7 @@ static void rdm_run(Context &c, const double *Wp, double *one, double *two, cons
     const bool gram = wk.G != nullptr;
     double *rho = spin ? wk.rho_b : wk.rho_a;
     if (gram) {
-      // G = w w^T: w is n rows of M values, i.e. the column-major M x n
-      // matrix B, and G = B^T B (n x n, symmetric)
-      const double one_d = 1.0, zero_d = 0.0;
-      if (rocblas_dgemm((rocblas_handle)blas_handle(c), rocblas_operation_transpose, rocblas_operation_none, t.n,
-                        t.n, M, &one_d, w, M, w, M, &zero_d, wk.G, t.n) != rocblas_status_success)
-        throw Error(3, "rdm: rocblas_dgemm (Gram matrix) failed");
+      rdm_gram(c, t.n, M, w, wk.G);
     } else {
       hipLaunchKernelGGL(k_rdm_diag_rows, dim3(t.n), dim3(256), 0, c.stream, M, w, rho);
       check_launch("k_rdm_diag_rows");
