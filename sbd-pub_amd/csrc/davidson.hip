@@ -22,7 +22,7 @@
 
 namespace sbdx {
 
-constexpr int kRedBlocks = 1024;
+constexpr int kRedBlocks = 1024;  // at most; see red_blocks
 // FP32 noise level of a product relative to |E0| (1000 x 2^-24): below
 // kFp32Floor |E0| a stalled mixed-precision solve switches to FP64 products
 constexpr double kFp32Floor = 1000.0 * 5.9604644775390625e-8;
@@ -61,6 +61,12 @@ __device__ __forceinline__ double block_sum(double v, double *sh) {
   return r;
 }
 
+// Blocks of a pass over a vector: one element per thread up to kRedBlocks
+// (the blocks past that would add only zeros to the sums that follow).
+static int red_blocks(const Context &c) {
+  return (int)std::min<size_t>(kRedBlocks, std::max<size_t>(1, (c.N + kRedThreads - 1) / kRedThreads));
+}
+
 // part[b*nv + k] = sum over this block's slice of X_k . y.  The vectors go
 // in groups of 8 sharing one read of y (y is read ceil(nv/8) times, each X_k
 // once); every thread sums its elements in index order, then a fixed tree.
@@ -91,25 +97,35 @@ __global__ void __launch_bounds__(kRedThreads) k_dots(VecList X, int nv, const d
   }
 }
 
-// Fixed-order sum of part[b*stride + off] over b < nblk by one whole
-// wavefront: lane l adds b = l, l + 64, ... in order, then a butterfly over
-// the 64 lanes (each step adds a pair of lanes' values in both lanes, so
-// every lane ends with the same total).  A single thread summing the 1024
-// partials one load at a time took ~0.1 ms.
+// Fixed-order sum of part[b*stride + off] over b < nblk <= kRedBlocks by one
+// whole wavefront: lane l adds b = l, l + 64, ... in order, then a butterfly
+// over the 64 lanes (each step adds a pair of lanes' values in both lanes, so
+// every lane ends with the same total).  All of a lane's loads are issued
+// before the first is added: they are most of the time of the small kernels
+// that begin with this sum (6 to 10 us each at 1024 partials with the loads
+// one after the other, 3 to 5 this way).
 __device__ __forceinline__ double wave_sum(const double *part, int nblk, int stride, int off) {
   const int lane = threadIdx.x & 63;
+  double v[kRedBlocks / 64];
+#pragma unroll
+  for (int q = 0; q < kRedBlocks / 64; q++) {
+    const int b = lane + 64 * q;
+    v[q] = b < nblk ? part[(size_t)b * stride + off] : 0.0;
+  }
   double s = 0.0;
-  for (int b = lane; b < nblk; b += 64) s += part[(size_t)b * stride + off];
+#pragma unroll
+  for (int q = 0; q < kRedBlocks / 64; q++) s += v[q];
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
   return s;
 }
-// threads of the one-block finishing kernels (4 wavefronts)
-constexpr int kFinishThreads = 256;
+// threads of the one-block finishing kernels: 16 wavefronts, one per column of
+// most subspaces
+constexpr int kFinishThreads = 1024;
 
 // Fixed-order sum of the partials of column k; written to H[k + ld*col] and
 // H[col + ld*k] (the symmetric subspace matrix, column-major).  Wavefront w
-// sums columns w, w + 4, ...
+// sums columns w, w + 16, ...
 __global__ void __launch_bounds__(kFinishThreads) k_finish_hcol(int nv, int nblk, const double *__restrict__ part,
                                                                 double *H, int ld, int col) {
   for (int k = threadIdx.x >> 6; k < nv; k += kFinishThreads / 64) {
@@ -223,12 +239,19 @@ void host_syev(int n, double *A, double *Q, double *E) {
   std::copy(Qs.begin(), Qs.end(), Q);
 }
 
+// Pinned host staging: the subspace matrix, its eigenvectors twice, the
+// eigenvalues, and values read back (read_pair).
+static double *host_stage(Context &c) {
+  if (!c.hpin) SBDX_HIP(hipHostMalloc((void **)&c.hpin, sizeof(double) * (3 * kNbMax * kNbMax + 3 * kNbMax)));
+  return c.hpin;
+}
+
 // Eigenpairs of the leading n x n block of the device subspace matrix H
 // (column-major, ld): to the host (pinned staging), host_syev, U (ld) and E
-// back to the device.  Synchronous.
+// back to the device in stream order.  The staging of U and E is written
+// again only after a later call's wait for H, which comes after these copies.
 static void subspace_eig(Context &c, int n, int ld, const double *H, double *U, double *E) {
-  if (!c.hpin) SBDX_HIP(hipHostMalloc((void **)&c.hpin, sizeof(double) * (3 * kNbMax * kNbMax + kNbMax)));
-  double *hA = c.hpin, *hQ = c.hpin + kNbMax * kNbMax, *hU = c.hpin + 2 * kNbMax * kNbMax;
+  double *hA = host_stage(c), *hQ = c.hpin + kNbMax * kNbMax, *hU = c.hpin + 2 * kNbMax * kNbMax;
   double *hE = c.hpin + 3 * kNbMax * kNbMax;
   SBDX_HIP(hipMemcpy2DAsync(hA, sizeof(double) * n, H, sizeof(double) * ld, sizeof(double) * n, n,
                             hipMemcpyDeviceToHost, c.stream));
@@ -238,7 +261,18 @@ static void subspace_eig(Context &c, int n, int ld, const double *H, double *U, 
     for (int i = 0; i < ld; i++) hU[i + (size_t)ld * j] = i < n ? hQ[i + (size_t)n * j] : 0.0;
   SBDX_HIP(hipMemcpyAsync(U, hU, sizeof(double) * ld * n, hipMemcpyHostToDevice, c.stream));
   SBDX_HIP(hipMemcpyAsync(E, hE, sizeof(double) * n, hipMemcpyHostToDevice, c.stream));
+}
+
+// a = *d0, b = *d1 (device; d0 < d1, within 2 kNbMax of it): one copy, then a
+// wait for the stream
+static void read_pair(Context &c, const double *d0, const double *d1, double &a, double &b) {
+  double *h = host_stage(c) + 3 * kNbMax * kNbMax + kNbMax;
+  const size_t n = (size_t)(d1 - d0) + 1;
+  if (d1 <= d0 || n > 2 * (size_t)kNbMax) throw Error(3, "davidson: values to read are too far apart");
+  SBDX_HIP(hipMemcpyAsync(h, d0, sizeof(double) * n, hipMemcpyDeviceToHost, c.stream));
   SBDX_HIP(hipStreamSynchronize(c.stream));
+  a = h[0];
+  b = h[n - 1];
 }
 
 // W = sum_k U[k] C_k ; R = -sum_k U[k] HC_k + E0*W ; partial |W|^2, |R|^2.
@@ -430,12 +464,16 @@ __global__ void __launch_bounds__(kRedThreads) k_precond(const double *__restric
   }
 }
 
-// c -= (sum of partials) * x   (one modified Gram-Schmidt projection)
-__global__ void __launch_bounds__(kRedThreads) k_axpy_part(double *__restrict__ c,
-                                                           const double *__restrict__ x, size_t n,
-                                                           const double *__restrict__ part,
-                                                           int nblk) {
+// c -= (sum of partials) * x (one modified Gram-Schmidt projection), and the
+// partials of the dot of the result with `next` (null: with itself).  One pass
+// where a projection and a dot of its own read c twice more and launched
+// twice: the sums are the same bit for bit.
+__global__ void __launch_bounds__(kRedThreads) k_axpy_dot(double *__restrict__ c, const double *__restrict__ x,
+                                                          const double *__restrict__ next, size_t n,
+                                                          const double *__restrict__ part, int nblk,
+                                                          double *__restrict__ out) {
   __shared__ double ol;
+  __shared__ double sh[kRedThreads];
   if (threadIdx.x < 64) {
     const double v = wave_sum(part, nblk, 1, 0);
     if (threadIdx.x == 0) ol = -v;
@@ -443,8 +481,14 @@ __global__ void __launch_bounds__(kRedThreads) k_axpy_part(double *__restrict__ 
   __syncthreads();
   const double o = ol;
   const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
-    c[i] += x[i] * o;
+  double s = 0.0;
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+    const double v = c[i] + x[i] * o;
+    c[i] = v;
+    s += (next ? next[i] : v) * v;
+  }
+  const double t = block_sum(s, sh);
+  if (threadIdx.x == 0) out[blockIdx.x] = t;
 }
 
 // c *= 1/sqrt(sum of partials)
@@ -472,11 +516,11 @@ static void dots(Context &c, const double *const *X, int nv, const double *y, do
                  const int *gate = nullptr) {
   VecList L{};
   for (int k = 0; k < nv; k++) L.p[k] = X[k];
-  hipLaunchKernelGGL(k_dots, dim3(kRedBlocks), dim3(kRedThreads), 0, c.stream, L, nv, y, c.N, part, gate);
+  hipLaunchKernelGGL(k_dots, dim3(red_blocks(c)), dim3(kRedThreads), 0, c.stream, L, nv, y, c.N, part, gate);
   check_launch("k_dots");
 }
 static void dots(Context &c, const VecList &L, int nv, const double *y, double *part) {
-  hipLaunchKernelGGL(k_dots, dim3(kRedBlocks), dim3(kRedThreads), 0, c.stream, L, nv, y, c.N, part,
+  hipLaunchKernelGGL(k_dots, dim3(red_blocks(c)), dim3(kRedThreads), 0, c.stream, L, nv, y, c.N, part,
                      (const int *)nullptr);
   check_launch("k_dots");
 }
@@ -486,7 +530,7 @@ double device_dot(Context &c, const double *x, const double *y, size_t n) {
   const double *X[1] = {x};
   dots(c, X, 1, y, c.part);
   double *scal = c.dsmall + kScalarOffset + 8;
-  hipLaunchKernelGGL(k_finish_scalar, dim3(1), dim3(64), 0, c.stream, kRedBlocks, c.part, scal);
+  hipLaunchKernelGGL(k_finish_scalar, dim3(1), dim3(64), 0, c.stream, red_blocks(c), c.part, scal);
   check_launch("k_finish_scalar");
   double r = 0.0;
   SBDX_HIP(hipMemcpyAsync(&r, scal, sizeof(double), hipMemcpyDeviceToHost, c.stream));
@@ -627,7 +671,8 @@ int davidson_solve(Context &c, int max_it, int nb, double eps, double max_time, 
   double *H = c.dsmall, *U = c.dsmall + ld * ld, *E = c.dsmall + 2 * ld * ld;
   double *scal = c.dsmall + kScalarOffset;
   const size_t N = c.N;
-  const dim3 g(kRedBlocks), b(kRedThreads);
+  const int nblk = red_blocks(c);
+  const dim3 g(nblk), b(kRedThreads);
   c.trace.clear();
   auto t_start = std::chrono::steady_clock::now();
   std::vector<double> step_times;
@@ -657,7 +702,7 @@ int davidson_solve(Context &c, int max_it, int nb, double eps, double max_time, 
           dots(c, c.HC.data(), ib + 1, c.C[ib], c.part);
         else
           dots(c, c.C.data(), ib + 1, c.HC[ib], c.part);
-        hipLaunchKernelGGL(k_finish_hcol, dim3(1), dim3(kFinishThreads), 0, c.stream, ib + 1, kRedBlocks,
+        hipLaunchKernelGGL(k_finish_hcol, dim3(1), dim3(kFinishThreads), 0, c.stream, ib + 1, nblk,
                            c.part, H, ld, ib);
         check_launch("k_finish_hcol");
         subspace_eig(c, ib + 1, ld, H, U, E);
@@ -671,15 +716,11 @@ int davidson_solve(Context &c, int max_it, int nb, double eps, double max_time, 
         }
         hipLaunchKernelGGL(k_ritz, g, b, 0, c.stream, Cv, HCv, ib + 1, U, E, N, c.W, c.R, c.part);
         check_launch("k_ritz");
-        hipLaunchKernelGGL(k_scale2, g, b, 0, c.stream, c.W, c.R, N, c.part, kRedBlocks, scal);
+        hipLaunchKernelGGL(k_scale2, g, b, 0, c.stream, c.W, c.R, N, c.part, nblk, scal);
         check_launch("k_scale2");
       }
-      double hs[2];
-      SBDX_HIP(hipMemcpyAsync(&hs[0], E, sizeof(double), hipMemcpyDeviceToHost, c.stream));
-      SBDX_HIP(hipMemcpyAsync(&hs[1], scal, sizeof(double), hipMemcpyDeviceToHost, c.stream));
-      SBDX_HIP(hipStreamSynchronize(c.stream));
-      E0 = hs[0];
-      const double nr = hs[1];
+      double nr;
+      read_pair(c, E, scal, E0, nr);
       c.trace.push_back(E0);
       c.trace.push_back(nr);
       steps++;
@@ -697,15 +738,17 @@ int davidson_solve(Context &c, int max_it, int nb, double eps, double max_time, 
         double *cn = c.C[ib + 1];
         hipLaunchKernelGGL(k_precond, g, b, 0, c.stream, c.R, c.hii, E, N, eps_reg, cn);
         check_launch("k_precond");
-        for (int kb = 0; kb <= ib; kb++) {
-          const double *X[1] = {c.C[kb]};
-          dots(c, X, 1, cn, c.part);
-          hipLaunchKernelGGL(k_axpy_part, g, b, 0, c.stream, cn, c.C[kb], N, c.part, kRedBlocks);
-          check_launch("k_axpy_part");
-        }
-        const double *X[1] = {cn};
+        // modified Gram-Schmidt; each projection's pass takes the dot with
+        // the next vector, the last one |cn|^2 (partials in turn in two places)
+        const double *X[1] = {c.C[0]};
         dots(c, X, 1, cn, c.part);
-        hipLaunchKernelGGL(k_scale_part, g, b, 0, c.stream, cn, N, c.part, kRedBlocks);
+        auto part = [&](int kb) { return c.part + (size_t)(kb & 1) * kRedBlocks; };
+        for (int kb = 0; kb <= ib; kb++) {
+          hipLaunchKernelGGL(k_axpy_dot, g, b, 0, c.stream, cn, (const double *)c.C[kb],
+                             (const double *)(kb < ib ? c.C[kb + 1] : nullptr), N, part(kb), nblk, part(kb + 1));
+          check_launch("k_axpy_dot");
+        }
+        hipLaunchKernelGGL(k_scale_part, g, b, 0, c.stream, cn, N, part(ib + 1), nblk);
         check_launch("k_scale_part");
       }
       auto s1 = std::chrono::steady_clock::now();
@@ -752,16 +795,12 @@ int davidson_solve_thick(Context &c, int max_steps, int nb, int keep, double eps
   double *H = c.dsmall, *U = c.dsmall + ld * ld, *E = c.dsmall + 2 * ld * ld;
   double *scal = c.dsmall + kScalarOffset;
   const size_t N = c.N;
-  const dim3 g(kRedBlocks), b(kRedThreads);
+  const int nblk = red_blocks(c);
+  const dim3 g(nblk), b(kRedThreads);
   c.trace.clear();
   auto t_start = std::chrono::steady_clock::now();
   auto elapsed = [&]() {
     return std::chrono::duration<double>(std::chrono::steady_clock::now() - t_start).count();
-  };
-  auto host2 = [&](const double *d0, const double *d1, double &a, double &bb) {
-    SBDX_HIP(hipMemcpyAsync(&a, d0, sizeof(double), hipMemcpyDeviceToHost, c.stream));
-    SBDX_HIP(hipMemcpyAsync(&bb, d1, sizeof(double), hipMemcpyDeviceToHost, c.stream));
-    SBDX_HIP(hipStreamSynchronize(c.stream));
   };
   // Column col of the subspace matrix as C[col] . HC[k], k <= col: the
   // older vector's product is used, so the coupling of every later vector to
@@ -784,7 +823,7 @@ int davidson_solve_thick(Context &c, int max_steps, int nb, int keep, double eps
   };
   auto add_column = [&](int col) {
     dots(c, hc_list(col + 1), col + 1, c.C[col], c.part);
-    hipLaunchKernelGGL(k_finish_hcol, dim3(1), dim3(kFinishThreads), 0, c.stream, col + 1, kRedBlocks, c.part,
+    hipLaunchKernelGGL(k_finish_hcol, dim3(1), dim3(kFinishThreads), 0, c.stream, col + 1, nblk, c.part,
                        H, ld, col);
     check_launch("k_finish_hcol");
   };
@@ -876,7 +915,7 @@ int davidson_solve_thick(Context &c, int max_steps, int nb, int keep, double eps
   {
     const double *X[1] = {c.C[0]};
     dots(c, X, 1, c.C[0], c.part);
-    hipLaunchKernelGGL(k_scale_part, g, b, 0, c.stream, c.C[0], N, c.part, kRedBlocks);
+    hipLaunchKernelGGL(k_scale_part, g, b, 0, c.stream, c.C[0], N, c.part, nblk);
     check_launch("k_scale_part");
   }
   // Anchor products (the start and the restarts) are exact so that the
@@ -934,12 +973,12 @@ int davidson_solve_thick(Context &c, int max_steps, int nb, int keep, double eps
         hipLaunchKernelGGL(k_ritz_expand, g, b, 0, c.stream, Cv, HCv, d + 1, U, E, c.hii, eps_reg, N, c.W,
                            c.C[d + 1], c.part, c.part + kPwOffset);
         check_launch("k_ritz_expand");
-        hipLaunchKernelGGL(k_finish_norms, dim3(1), dim3(64), 0, c.stream, kRedBlocks, c.part + kPwOffset, scal);
+        hipLaunchKernelGGL(k_finish_norms, dim3(1), dim3(64), 0, c.stream, nblk, c.part + kPwOffset, scal);
         check_launch("k_finish_norms");
       } else {
         hipLaunchKernelGGL(k_ritz, g, b, 0, c.stream, Cv, HCv, d + 1, U, E, N, c.W, c.R, c.part);
         check_launch("k_ritz");
-        hipLaunchKernelGGL(k_scale2, g, b, 0, c.stream, c.W, c.R, N, c.part, kRedBlocks, scal);
+        hipLaunchKernelGGL(k_scale2, g, b, 0, c.stream, c.W, c.R, N, c.part, nblk, scal);
         check_launch("k_scale2");
       }
     }
@@ -948,7 +987,7 @@ int davidson_solve_thick(Context &c, int max_steps, int nb, int keep, double eps
       hipLaunchKernelGGL(k_scale_by, g, b, 0, c.stream, c.W, N, scal + 1);
       check_launch("k_scale_by");
     };
-    host2(E, scal, E0, nr);
+    read_pair(c, E, scal, E0, nr);
     c.trace.push_back(E0);
     c.trace.push_back(nr);
     if (c.verbose) {
@@ -985,14 +1024,14 @@ int davidson_solve_thick(Context &c, int max_steps, int nb, int keep, double eps
       const double *X[1] = {c.W};
       dots(c, X, 1, HW, c.part);
       double *Eex = scal + 2;
-      hipLaunchKernelGGL(k_exact_resid, g, b, 0, c.stream, c.W, HW, N, c.part, kRedBlocks, c.R,
+      hipLaunchKernelGGL(k_exact_resid, g, b, 0, c.stream, c.W, HW, N, c.part, nblk, c.R,
                          c.part + kRedBlocks, Eex);
       check_launch("k_exact_resid");
-      hipLaunchKernelGGL(k_finish_scalar, dim3(1), dim3(64), 0, c.stream, kRedBlocks,
+      hipLaunchKernelGGL(k_finish_scalar, dim3(1), dim3(64), 0, c.stream, nblk,
                          c.part + kRedBlocks, scal + 3);
       check_launch("k_finish_scalar");
       double e_ex, r2;
-      host2(Eex, scal + 3, e_ex, r2);
+      read_pair(c, Eex, scal + 3, e_ex, r2);
       E0 = e_ex;
       nr = std::sqrt(r2);
       c.trace.push_back(E0);
@@ -1028,7 +1067,7 @@ int davidson_solve_thick(Context &c, int max_steps, int nb, int keep, double eps
       {
         const double *Y[1] = {c.R};
         dots(c, Y, 1, c.R, c.part);
-        hipLaunchKernelGGL(k_scale_part, g, b, 0, c.stream, c.R, N, c.part, kRedBlocks);
+        hipLaunchKernelGGL(k_scale_part, g, b, 0, c.stream, c.R, N, c.part, nblk);
         check_launch("k_scale_part");
       }
       // thick restart basis: W (exact product) + Ritz vectors 1..keep_now-1
@@ -1110,19 +1149,19 @@ int davidson_solve_thick(Context &c, int max_steps, int nb, int keep, double eps
       for (int k = 0; k <= d; k++) Xw[k] = c.C[k];
       Xw[d + 1] = cn;  // d + 2 <= nb <= kNbMax
       if (!have_cn) dots(c, Xw, d + 2, cn, c.part);  // else k_ritz_expand wrote them
-      hipLaunchKernelGGL(k_finish_dgks, dim3(1), dim3(kFinishThreads), 0, c.stream, d + 1, kRedBlocks, c.part, coef, gate);
+      hipLaunchKernelGGL(k_finish_dgks, dim3(1), dim3(kFinishThreads), 0, c.stream, d + 1, nblk, c.part, coef, gate);
       check_launch("k_finish_dgks");
       hipLaunchKernelGGL(k_sub_combo, g, b, 0, c.stream, Cv, d + 1, coef, cn, N, (const int *)nullptr);
       check_launch("k_sub_combo");
       dots(c, c.C.data(), d + 1, cn, c.part, gate);
-      hipLaunchKernelGGL(k_finish_vec, dim3(1), dim3(kFinishThreads), 0, c.stream, d + 1, kRedBlocks, c.part, coef,
+      hipLaunchKernelGGL(k_finish_vec, dim3(1), dim3(kFinishThreads), 0, c.stream, d + 1, nblk, c.part, coef,
                          (const int *)gate);
       check_launch("k_finish_vec");
       hipLaunchKernelGGL(k_sub_combo, g, b, 0, c.stream, Cv, d + 1, coef, cn, N, (const int *)gate);
       check_launch("k_sub_combo");
       const double *X[1] = {cn};
       dots(c, X, 1, cn, c.part);
-      hipLaunchKernelGGL(k_scale_part, g, b, 0, c.stream, cn, N, c.part, kRedBlocks);
+      hipLaunchKernelGGL(k_scale_part, g, b, 0, c.stream, cn, N, c.part, nblk);
       check_launch("k_scale_part");
     }
     if (mixed && sym) {
