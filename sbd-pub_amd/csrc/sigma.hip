@@ -102,19 +102,32 @@ __global__ void __launch_bounds__(256) k_same_xcd(int nrows, int M, int nch, int
   if (live) y[r * Ms + m] = acc;
 }
 
-// out[c][r] (+)= in[r][c] for an R x Cc row-major matrix, 64x64 LDS tiles.
-template <typename T, bool ACC>
+// Tiles of the transposing passes: 64 x 64, or 32 x 32 where the larger ones
+// would be fewer than four blocks per CU (up to some 2000 rows and columns).
+// Such passes are bound by the latency of a block's loads (all of a thread's
+// are in flight at once) and by how many blocks run beside each other:
+// k_sym_combine in FP32 at 500 strings 12.8 us with 64 x 64 tiles, 4.6 with
+// 32 x 32, k_symmetrize at 1001 strings 15.6 and 7.3.
+static bool small_tiles(const Context &c, size_t R, size_t C) {
+  return (size_t)cdiv(R, 64) * cdiv(C, 64) < (size_t)4 * c.n_cu;
+}
+
+// out[c][r] (+)= in[r][c] for an R x Cc row-major matrix, TS x TS LDS tiles.
+template <typename T, bool ACC, int TS>
 __global__ void __launch_bounds__(256) k_transpose(const T *__restrict__ in, T *__restrict__ out,
                                                    int R, int Cc) {
-  __shared__ T tile[64][65];
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  const int c0 = blockIdx.x * 64, r0 = blockIdx.y * 64;
-  for (int k = ty; k < 64; k += 4) {
+  constexpr int ST = 256 / TS;
+  __shared__ T tile[TS][TS + 1];
+  const int tx = threadIdx.x % TS, ty = threadIdx.x / TS;
+  const int c0 = blockIdx.x * TS, r0 = blockIdx.y * TS;
+#pragma unroll
+  for (int q = 0, k = ty; q < TS / ST; q++, k += ST) {
     const int r = r0 + k, cc = c0 + tx;
     if (r < R && cc < Cc) tile[k][tx] = in[(size_t)r * Cc + cc];
   }
   __syncthreads();
-  for (int k = ty; k < 64; k += 4) {
+#pragma unroll
+  for (int q = 0, k = ty; q < TS / ST; q++, k += ST) {
     const int cc = c0 + k, r = r0 + tx;
     if (cc < Cc && r < R) {
       const T v = tile[tx][k];
@@ -1337,26 +1350,29 @@ __global__ void __launch_bounds__(256) k_densify(int n, const uint64_t *__restri
 }
 
 // Spin-flip symmetric form of the same-spin terms for equal string sets:
-// y = hii*x + (G + G^T) with G = H X (n x n row-major), 64x64 tiles, G^T
+// y = hii*x + (G + G^T) with G = H X (n x n row-major), TS x TS tiles, G^T
 // through LDS; for symmetric x the result is bitwise symmetric.  For the
 // odd sector (x = -x^T, odd != 0) X H = -G^T, so y = hii*x + (G - G^T),
 // bitwise antisymmetric with a zero diagonal.
 // gscale (device, may be null): G holds 2^(ex+eh) times the product (the
 // split-FP16 GEMM), and gscale[0] * gscale[1] = 2^-(ex+eh) undoes it exactly.
-template <typename T>
+template <typename T, int TS>
 __global__ void __launch_bounds__(256) k_sym_combine(int n, const T *__restrict__ hii, const T *__restrict__ x,
                                                      const T *__restrict__ G, T *__restrict__ y,
                                                      const float *__restrict__ gscale, int odd) {
+  constexpr int ST = 256 / TS;
   const T s = gscale ? (T)(gscale[0] * gscale[1]) : T(1);
-  __shared__ T tile[64][65];
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  const int c0 = blockIdx.x * 64, r0 = blockIdx.y * 64;
-  for (int k = ty; k < 64; k += 4) {
+  __shared__ T tile[TS][TS + 1];
+  const int tx = threadIdx.x % TS, ty = threadIdx.x / TS;
+  const int c0 = blockIdx.x * TS, r0 = blockIdx.y * TS;
+#pragma unroll
+  for (int q = 0, k = ty; q < TS / ST; q++, k += ST) {
     const int gr = c0 + k, gc = r0 + tx;
     if (gr < n && gc < n) tile[k][tx] = G[(size_t)gr * n + gc];
   }
   __syncthreads();
-  for (int k = ty; k < 64; k += 4) {
+#pragma unroll
+  for (int q = 0, k = ty; q < TS / ST; q++, k += ST) {
     const int r = r0 + k, cc = c0 + tx;
     if (r < n && cc < n) {
       const size_t o = (size_t)r * n + cc;
@@ -1364,6 +1380,18 @@ __global__ void __launch_bounds__(256) k_sym_combine(int n, const T *__restrict_
       y[o] = hii[o] * x[o] + (odd ? G[o] - tile[tx][k] : G[o] + tile[tx][k]) * s;
     }
   }
+}
+
+template <typename T>
+static void sym_combine(Context &c, int n, const T *hii, const T *x, const T *G, T *y, const float *gscale) {
+  const int odd = c.sym_par < 0 ? 1 : 0;
+  if (small_tiles(c, n, n))
+    hipLaunchKernelGGL((k_sym_combine<T, 32>), dim3(cdiv(n, 32), cdiv(n, 32)), dim3(256), 0, c.stream, n, hii, x, G,
+                       y, gscale, odd);
+  else
+    hipLaunchKernelGGL((k_sym_combine<T, 64>), dim3(cdiv(n, 64), cdiv(n, 64)), dim3(256), 0, c.stream, n, hii, x, G,
+                       y, gscale, odd);
+  check_launch("k_sym_combine");
 }
 
 // Split-FP16 operands of the symmetric FP32 same-spin GEMM.  An FP32 array
@@ -1421,17 +1449,21 @@ __global__ void __launch_bounds__(256) k_split_f16(size_t n, const float *__rest
 // v = (v + p v^T)/2 on an n x n row-major matrix, p = +1 (even sector) or
 // -1 (odd sector: the diagonal becomes 0); block (bx, by), bx <= by, owns
 // the tile pair (by, bx) / (bx, by).
+template <int TS>
 __global__ void __launch_bounds__(256) k_symmetrize(int n, double *__restrict__ v, double p) {
   if (blockIdx.x > blockIdx.y) return;
-  __shared__ double A[64][65], B[64][65];
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  const int R0 = blockIdx.y * 64, C0 = blockIdx.x * 64;
-  for (int k = ty; k < 64; k += 4) {
+  constexpr int ST = 256 / TS;
+  __shared__ double A[TS][TS + 1], B[TS][TS + 1];
+  const int tx = threadIdx.x % TS, ty = threadIdx.x / TS;
+  const int R0 = blockIdx.y * TS, C0 = blockIdx.x * TS;
+#pragma unroll
+  for (int q = 0, k = ty; q < TS / ST; q++, k += ST) {
     A[k][tx] = (R0 + k < n && C0 + tx < n) ? v[(size_t)(R0 + k) * n + C0 + tx] : 0.0;
     B[k][tx] = (C0 + k < n && R0 + tx < n) ? v[(size_t)(C0 + k) * n + R0 + tx] : 0.0;
   }
   __syncthreads();
-  for (int k = ty; k < 64; k += 4) {
+#pragma unroll
+  for (int q = 0, k = ty; q < TS / ST; q++, k += ST) {
     if (R0 + k < n && C0 + tx < n) v[(size_t)(R0 + k) * n + C0 + tx] = 0.5 * (A[k][tx] + p * B[tx][k]);
     if (C0 + k < n && R0 + tx < n) v[(size_t)(C0 + k) * n + R0 + tx] = 0.5 * (B[k][tx] + p * A[tx][k]);
   }
@@ -1510,14 +1542,20 @@ static void sigma_same(Context &c, const SpinTables &t, const T *s_val, const T 
   check_launch("k_same_xcd");
 }
 
+template <typename T, bool ACC>
+static void launch_transpose(Context &c, const T *in, T *out, int R, int Cc) {
+  if (small_tiles(c, R, Cc))
+    hipLaunchKernelGGL((k_transpose<T, ACC, 32>), dim3(cdiv(Cc, 32), cdiv(R, 32)), dim3(256), 0, c.stream, in, out,
+                       R, Cc);
+  else
+    hipLaunchKernelGGL((k_transpose<T, ACC, 64>), dim3(cdiv(Cc, 64), cdiv(R, 64)), dim3(256), 0, c.stream, in, out,
+                       R, Cc);
+  check_launch("k_transpose");
+}
 template <typename T>
 static void transpose(Context &c, const T *in, T *out, int R, int Cc, bool acc) {
-  const dim3 grid(cdiv(Cc, 64), cdiv(R, 64));
-  if (acc)
-    hipLaunchKernelGGL((k_transpose<T, true>), grid, dim3(256), 0, c.stream, in, out, R, Cc);
-  else
-    hipLaunchKernelGGL((k_transpose<T, false>), grid, dim3(256), 0, c.stream, in, out, R, Cc);
-  check_launch("k_transpose");
+  if (acc) launch_transpose<T, true>(c, in, out, R, Cc);
+  else launch_transpose<T, false>(c, in, out, R, Cc);
 }
 
 void transpose_into(Context &c, const double *in, double *out, int R, int Cc) {
@@ -2346,9 +2384,7 @@ static void sym_same_split(Context &c, const float *hii, const float *x, float *
                       rocblas_datatype_f32_r, n, G, rocblas_datatype_f32_r, n, rocblas_datatype_f32_r,
                       rocblas_gemm_algo_standard, 0, 0) != rocblas_status_success)
     throw Error(3, "split-FP16 same-spin GEMM failed");
-  hipLaunchKernelGGL((k_sym_combine<float>), dim3(cdiv(n, 64), cdiv(n, 64)), dim3(256), 0, c.stream, n, hii, x,
-                     (const float *)G, y, (const float *)c.split_inv, c.sym_par < 0 ? 1 : 0);
-  check_launch("k_sym_combine");
+  sym_combine<float>(c, n, hii, x, G, y, c.split_inv);
 }
 
 static void sym_product(Context &c, const double *x, double *G) { same_mm_alpha(c, x, G); }
@@ -2365,9 +2401,7 @@ template <typename T>
 static void sym_same_gemm(Context &c, const SigmaOperands<T> &o, const T *x, T *y) {
   const int n = (int)c.na;
   sym_product(c, x, o.T1);
-  hipLaunchKernelGGL((k_sym_combine<T>), dim3(cdiv(n, 64), cdiv(n, 64)), dim3(256), 0, c.stream, n, o.hii, x,
-                     (const T *)o.T1, y, (const float *)nullptr, c.sym_par < 0 ? 1 : 0);
-  check_launch("k_sym_combine");
+  sym_combine<T>(c, n, o.hii, x, o.T1, y, nullptr);
 }
 
 static void sym_same(Context &c, const SigmaOperands<double> &o, const double *x, double *y) {
@@ -2777,8 +2811,12 @@ double sym_defect(Context &c, const double *v, int p) {
 }
 
 void symmetrize(Context &c, double *v, int p) {
-  const unsigned t = cdiv(c.na, 64);
-  hipLaunchKernelGGL(k_symmetrize, dim3(t, t), dim3(256), 0, c.stream, (int)c.na, v, p < 0 ? -1.0 : 1.0);
+  const double s = p < 0 ? -1.0 : 1.0;
+  const unsigned t = cdiv(c.na, small_tiles(c, c.na, c.na) ? 32 : 64);
+  if (small_tiles(c, c.na, c.na))
+    hipLaunchKernelGGL((k_symmetrize<32>), dim3(t, t), dim3(256), 0, c.stream, (int)c.na, v, s);
+  else
+    hipLaunchKernelGGL((k_symmetrize<64>), dim3(t, t), dim3(256), 0, c.stream, (int)c.na, v, s);
   check_launch("k_symmetrize");
 }
 
