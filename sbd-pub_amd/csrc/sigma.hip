@@ -1941,7 +1941,8 @@ static bool mixed_ell_cfg(Context &c, int eb, int nt, const float *eri, const fl
          : eb == 2 ? mixed_ell_dispatch<float, 2, SYM>(c, nt, eri, x, y)
                    : mixed_ell_dispatch<float, 1, SYM>(c, nt, eri, x, y);
 }
-// Autotuner for the sliced-ELL mixed kernel: every (staging width EB in
+// Configuration of the sliced-ELL mixed kernel: by a rule with the
+// signed-triangle table, else timed: every (staging width EB in
 // {1, 2, 4, kEbSigned (k_mixed_sw)}, slots per thread NT in {1, 2, 4, 8})
 // whose LDS footprint fits
 // and that does not cover fewer than half of a row's slots per thread
@@ -1965,7 +1966,33 @@ static int mixed_cfg(Context &c, const T *eri, const T *x) {
   hipEvent_t e0, e1;
   SBDX_HIP(hipEventCreate(&e0));
   SBDX_HIP(hipEventCreate(&e1));
-  // every timed configuration, in the fixed order (the signed-triangle
+  // Where the signed-triangle table exists (up to 8191 strings) the choice is
+  // known: that kernel with the fewest slots per thread that cover a row,
+  // or four pairs a round for symmetric FP64 products of small sets.  Of 27
+  // cases timed (FP32, symmetric FP32 and FP64, 60 to 7000 strings) it was the
+  // fastest in 22 and within 3% in two; in the other three, symmetric FP64,
+  // four pairs took 24 against 28 us at 60 strings, 72 against 86 at 150, 81
+  // against 90 at 275 (at 500: 108 against 104).  Fewer slots than cover a row
+  // took 1.86 against 1.58 ms at 4001.  Timing them all took 15 products
+  // per form of a context's first use, 150 of 320 ms of a first solve at 4001.
+  if (c.B.has_ell3 && !fix_eb && !fix_nt) {
+    int nt = 1;
+    while (nt < nt_max && nt < 8) nt *= 2;
+    const int eb = SYM && sizeof(T) == 8 && c.B.n < 400 ? 4 : kEbSigned;
+    SBDX_HIP(hipEventRecord(e0, c.stream));
+    const bool ok = mixed_ell_cfg<SYM>(c, eb, nt, eri, x, scratch);  // false where it does not fit the LDS
+    SBDX_HIP(hipEventRecord(e1, c.stream));
+    SBDX_HIP(hipEventSynchronize(e1));
+    if (ok) {
+      check_launch("k_mixed_ell");
+      SBDX_HIP(hipEventElapsedTime(&c.mixed_best_ms[pi], e0, e1));
+      SBDX_HIP(hipEventDestroy(e0));
+      SBDX_HIP(hipEventDestroy(e1));
+      c.mixed_nt[pi] = nt;
+      return c.mixed_eb[pi] = eb;
+    }
+  }
+  // else every configuration timed, in the fixed order (the signed-triangle
   // kernel, then eb descending; nt ascending)
   std::vector<std::array<float, 3>> timed;
   for (int eb : {kEbSigned, 4, 2, 1}) {
