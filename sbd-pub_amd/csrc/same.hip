@@ -118,9 +118,10 @@ __global__ void __launch_bounds__(256) k_tiles(int n, int tm, const uint32_t *__
 // one XCD take the row tiles of one column chunk, walking their lists at the
 // same pace, so x's rows come from that XCD's L2.
 // Bound by the matrix instructions: 16 of them, 1024 cycles, per 8 KB of
-// operands at 64 x 64.  One term of 4001 x 4001 strings 1.44 ms (1.09 at the
-// instructions' rate), as a dense library product 1.86; of 2583 x 2583 0.42 ms
-// at 32 x 32 (the halved lists: 0.46); both terms at 1000 x 900 0.10 ms with
+// operands at 64 x 64.  One term of 8000 x 8000 strings 8.8 ms (7.4 at the
+// instructions' rate over the tiles), as a dense library product 14.3; of 4001 x
+// 4001 1.44 ms (1.09), as a dense library product 1.86; of 2583 x 2583 0.42 ms
+// at 32 x 32 (with whole lists 0.46); both terms at 1000 x 900 0.10 ms with
 // their transposes, in the small form below 0.19.
 template <int MT, int NT, int KS, bool DIAG>
 __global__ void __launch_bounds__(256, MT == 4 ? 2 : 4)
