@@ -383,11 +383,12 @@ bool same_mm_fits(const Context &c) {
 // Where the sets have few singles and doubles (random strings), the row
 // kernels over them are faster than tiles that are nearly all zeros: at 60
 // multiply-adds of the matrix cores per entry (the rates of the two forms,
-// 70 and 1.3 TFLOP/s at 8000 x 8000 strings).
+// 70 and 1.3 TFLOP/s at 8000 x 8000 strings); and a single row or column of a
+// large set would read its whole dense block.
 bool same_mm_worth(const Context &c) {
   const double work = (double)c.N * ((double)c.na + (double)c.nb);
   const double ent = (double)(c.A.ns + c.A.nd) * (double)c.nb + (double)(c.B.ns + c.B.nd) * (double)c.na;
-  return small(c) || work <= 60.0 * ent;
+  return c.na + c.nb <= kSameSmall || (!small(c) && work <= 60.0 * ent);
 }
 
 // y = hii*x + H_a X + X H_b; xt and yt: N doubles each
