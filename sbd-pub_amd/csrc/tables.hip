@@ -768,7 +768,9 @@ void build_singles_ell_parts(Context &c, SpinTables &t, int nparts) {
 // all left over, grown greedily from the member with the most partners; the
 // rest goes to the entry table.  On a set of the Hartree-Fock string, its
 // singles and doubles the first kind covers the moves of a particle, the
-// second those of a hole.
+// second those of a hole.  A set may list a string more than once (rows that
+// are alike but do not couple); its copies would share an orbital's place in
+// a column, so blocks that hold such a pair stay in the entry table.
 namespace {
 constexpr int kBlockWorth = 12;
 
@@ -887,8 +889,9 @@ static void build_blocks_ket(Context &c, SpinTables &t, const std::vector<uint64
   std::vector<Col> cols;
   for (size_t i = 0; i < pm.size();) {
     size_t j = i;
-    while (j < pm.size() && pm[j].key == pm[i].key) j++;
-    if (worth((int)(j - i))) cols.push_back({bit_reverse(pm[i].key), (uint32_t)i, (uint32_t)(j - i)});
+    bool twice = false;  // two members at one orbital
+    for (; j < pm.size() && pm[j].key == pm[i].key; j++) twice |= j > i && pm[j].orb == pm[j - 1].orb;
+    if (!twice && worth((int)(j - i))) cols.push_back({bit_reverse(pm[i].key), (uint32_t)i, (uint32_t)(j - i)});
     i = j;
   }
   std::sort(cols.begin(), cols.end(), [](const Col &a, const Col &b) { return a.rev < b.rev; });
@@ -1147,8 +1150,12 @@ void build_rdm_tables(Context &c, SpinTables &t, const std::vector<uint64_t> &st
   for (size_t i = 0; i < pm.size();) {
     size_t j = i;
     uint32_t tiles = 0;
-    for (; j < pm.size() && pm[j].key == pm[i].key; j++) tiles |= 1u << (pm[j].orb >> 4);
-    if (worth((int)(j - i), tile_of(tiles))) {
+    bool twice = false;
+    for (; j < pm.size() && pm[j].key == pm[i].key; j++) {
+      tiles |= 1u << (pm[j].orb >> 4);
+      twice |= j > i && pm[j].orb == pm[j - 1].orb;
+    }
+    if (!twice && worth((int)(j - i), tile_of(tiles))) {
       for (size_t k = i; k < j; k++) big[pm[k].str] |= 1ull << pm[k].orb;
       cols.push_back({pm[i].key, (uint32_t)i, (uint16_t)(j - i), (int8_t)tile_of(tiles), 0});
     }
@@ -1177,11 +1184,15 @@ void build_rdm_tables(Context &c, SpinTables &t, const std::vector<uint64_t> &st
     size_t j = i;
     uint64_t adj[64] = {}, verts = 0;
     uint32_t who[64] = {};
+    bool twice = false;
     for (; j < left.size() && left[j].key == left[i].key; j++) {
-      adj[left[j].miss] |= 1ull << left[j].add;
-      verts |= 1ull << left[j].miss;
-      who[left[j].miss] = left[j].str;
+      const int v = left[j].miss;
+      twice |= ((verts >> v) & 1ull) && who[v] != left[j].str;
+      adj[v] |= 1ull << left[j].add;
+      verts |= 1ull << v;
+      who[v] = left[j].str;
     }
+    if (twice) verts = 0;
     int cls[64];
     std::fill(cls, cls + 64, -1);
     for (int nc = 0;; nc++) {
