@@ -41,6 +41,8 @@ void dfree_all(Context &c) {
   c.allocs.clear();
 }
 
+StreamWait::~StreamWait() { (void)hipStreamSynchronize(c.stream); }
+
 TmpBuf::TmpBuf(size_t bytes) {
   hipError_t e = hipMalloc(&p, bytes ? bytes : 8);
   if (e != hipSuccess) {

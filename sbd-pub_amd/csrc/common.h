@@ -355,6 +355,17 @@ Context *make_sub_context(const Context &c, size_t m);  // first m strings of ea
 void destroy_context(Context *c);
 void *blas_handle(Context &c);     // rocblas_handle bound to the stream
 
+// Waits for the stream at scope exit.  Declared after the host arrays that
+// asynchronous copies read or write, it keeps them until the copies have
+// ended, also where an exception leaves the scope.
+struct StreamWait {
+  Context &c;
+  explicit StreamWait(Context &cx) : c(cx) {}
+  ~StreamWait();
+  StreamWait(const StreamWait &) = delete;
+  StreamWait &operator=(const StreamWait &) = delete;
+};
+
 // Device scratch released at scope exit (callers synchronize first).
 struct TmpBuf {
   void *p = nullptr;

@@ -310,7 +310,9 @@ void build_tiles(Context &c, const SpinTables &t, const std::vector<uint64_t> &s
     SBDX_HIP(hipMemcpyAsync(p, v.data(), sizeof(uint32_t) * v.size(), hipMemcpyHostToDevice, c.stream));
     return p;
   };
+  std::vector<uint32_t> cnt(o.ntile), base(o.ntile + 1, 0), by(o.ntile), rows(order.size());
   TmpBuf tord(sizeof(uint32_t) * order.size()), tpos(sizeof(uint32_t) * n), tcnt(sizeof(uint32_t) * o.ntile);
+  const StreamWait wait(c);
   SBDX_HIP(hipMemcpyAsync(tord.p, order.data(), sizeof(uint32_t) * order.size(), hipMemcpyHostToDevice, c.stream));
   SBDX_HIP(hipMemcpyAsync(tpos.p, pos.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice, c.stream));
   const uint32_t *dord = (const uint32_t *)tord.p, *dpos = (const uint32_t *)tpos.p;
@@ -319,7 +321,6 @@ void build_tiles(Context &c, const SpinTables &t, const std::vector<uint64_t> &s
                      t.s_off, t.s_ent, t.s_val, t.d_off, t.d_ket, t.d_val, (uint32_t *)tcnt.p,
                      (const uint32_t *)nullptr, (uint32_t *)nullptr, (double *)nullptr);
   check_launch("k_tiles");
-  std::vector<uint32_t> cnt(o.ntile), base(o.ntile + 1, 0), by(o.ntile), rows(order.size());
   SBDX_HIP(hipMemcpyAsync(cnt.data(), tcnt.p, sizeof(uint32_t) * o.ntile, hipMemcpyDeviceToHost, c.stream));
   SBDX_HIP(hipStreamSynchronize(c.stream));
   // the tiles with the longest lists first (those of the reference string and

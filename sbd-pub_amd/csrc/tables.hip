@@ -661,6 +661,7 @@ void build_singles_ell(Context &c, SpinTables &t) {
           f - 1 - ng, sl_len[sl], pad3, ell3.data() + sl_off2[sl], wide);
     }
   });
+  const StreamWait wait(c);
   auto put = [&](const void *src, size_t bytes) {
     void *dst = dalloc(c, bytes);
     SBDX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c.stream));
@@ -812,11 +813,6 @@ constexpr int kColWorth = 4;
 // The alpha set's tables: bk_order, bk_ent.
 static void build_blocks_bra(Context &c, SpinTables &t, const std::vector<uint64_t> &strs) {
   const int n = t.n, L = c.L;
-  auto put = [&](const void *src, size_t bytes) {
-    void *dst = dalloc(c, bytes);
-    if (bytes) SBDX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c.stream));
-    return dst;
-  };
   std::vector<uint64_t> off, ent;
   download_singles(c, t, off, ent);
   // order of the bras: those with more than twice the average singles
@@ -837,7 +833,6 @@ static void build_blocks_bra(Context &c, SpinTables &t, const std::vector<uint64
   std::vector<uint32_t> blk(ord);
   for (int w = 0; w + 256 <= n; w += 256)
     for (int b = 0; b < 256; b++) blk[w + b] = ord[w + (b & 7) * 32 + (b >> 3)];
-  t.bk_order = (uint32_t *)put(blk.data(), sizeof(uint32_t) * n);
   std::vector<uint64_t> e2(t.ns + n);
   for (int r = 0; r < n; r++) {
     uint64_t *o = e2.data() + off[r] + r;
@@ -848,6 +843,13 @@ static void build_blocks_bra(Context &c, SpinTables &t, const std::vector<uint64
     }
     *o = (uint64_t)r | (1ull << 62);
   }
+  const StreamWait wait(c);
+  auto put = [&](const void *src, size_t bytes) {
+    void *dst = dalloc(c, bytes);
+    if (bytes) SBDX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c.stream));
+    return dst;
+  };
+  t.bk_order = (uint32_t *)put(blk.data(), sizeof(uint32_t) * n);
   t.bk_ent = (uint64_t *)put(e2.data(), sizeof(uint64_t) * e2.size());
   SBDX_HIP(hipStreamSynchronize(c.stream));
 }
@@ -855,11 +857,6 @@ static void build_blocks_bra(Context &c, SpinTables &t, const std::vector<uint64
 // The beta set's tables; has_blk where the form holds them.
 static void build_blocks_ket(Context &c, SpinTables &t, const std::vector<uint64_t> &strs) {
   const int n = t.n, L = c.L, Kt = c.Kt;
-  auto put = [&](const void *src, size_t bytes) {
-    void *dst = dalloc(c, bytes);
-    if (bytes) SBDX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c.stream));
-    return dst;
-  };
   t.has_blk = false;
   if (!c.eri_rs_sym || 2 * Kt + 1 > 2048) return;
   auto image = [&](int pb) { return ((size_t)2 * Kt + 1 + n + 1) << pb; };
@@ -965,12 +962,8 @@ static void build_blocks_ket(Context &c, SpinTables &t, const std::vector<uint64
     }
     col_off.push_back((uint32_t)col_pos.size());
   }
-  t.bk_col_off = (uint32_t *)put(col_off.data(), sizeof(uint32_t) * col_off.size());
-  t.bk_col_pos = (uint16_t *)put(col_pos.data(), sizeof(uint16_t) * col_pos.size());
   t.bk_nstep = (int)step.back();
   tab.resize(tab.size() + 6 * 64, none);  // the kernel loads up to four steps ahead
-  t.bk_step = (uint32_t *)put(step.data(), sizeof(uint32_t) * step.size());
-  t.bk_tab = (uint2 *)put(tab.data(), sizeof(uint2) * tab.size());
   // ---- the rest, entry by entry
   auto covered = [&](int r, uint64_t e) {
     const uint32_t pq = (uint32_t)((e >> 32) & 0x7fffffffull);
@@ -1057,6 +1050,16 @@ static void build_blocks_ket(Context &c, SpinTables &t, const std::vector<uint64
   });
   t.bk_nslice = nsl;
   t.bk_ngroup = (int)tot;
+  const StreamWait wait(c);
+  auto put = [&](const void *src, size_t bytes) {
+    void *dst = dalloc(c, bytes);
+    if (bytes) SBDX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c.stream));
+    return dst;
+  };
+  t.bk_col_off = (uint32_t *)put(col_off.data(), sizeof(uint32_t) * col_off.size());
+  t.bk_col_pos = (uint16_t *)put(col_pos.data(), sizeof(uint16_t) * col_pos.size());
+  t.bk_step = (uint32_t *)put(step.data(), sizeof(uint32_t) * step.size());
+  t.bk_tab = (uint2 *)put(tab.data(), sizeof(uint2) * tab.size());
   t.bk_perm = (uint32_t *)put(perm.data(), sizeof(uint32_t) * perm.size());
   t.bk_rec = (uint4 *)put(rec.data(), sizeof(uint16_t) * rec.size());
   t.bk_off = (uint32_t *)put(soff.data(), sizeof(uint32_t) * nsl);
@@ -1084,6 +1087,7 @@ void build_rdm_tables(Context &c, SpinTables &t, const std::vector<uint64_t> &st
   };
   std::vector<uint64_t> aent;
   std::vector<uint4> items;
+  const StreamWait wait_a(c);
   if (as_alpha) {
     std::vector<size_t> cnt(K + 1, 0);
     auto kept = [&](uint64_t e) {
@@ -1254,9 +1258,6 @@ void build_rdm_tables(Context &c, SpinTables &t, const std::vector<uint64_t> &st
     t.rc_range[t.rc_nrange++] = make_int4(s0, s0 + ns, cols[i].tile, cols[i].hole);
     i = j;
   }
-  void *p;
-  put(p, tab.data(), sizeof(uint64_t) * tab.size());
-  t.rc_tab = (uint64_t *)p;
   // the entry table of the rest: every pair's entries in runs of at most
   // `run`, the shortest for which 8 slices (one per wavefront) hold all runs
   std::vector<std::vector<uint32_t>> bin(K);
@@ -1297,6 +1298,10 @@ void build_rdm_tables(Context &c, SpinTables &t, const std::vector<uint64_t> &st
     perm[i] = runs[i].pair;
     for (uint32_t k = 0; k < runs[i].len; k++) pb[soff[i / 64] + 64 * k + i % 64] = bin[runs[i].pair][runs[i].first + k];
   }
+  const StreamWait wait_b(c);
+  void *p;
+  put(p, tab.data(), sizeof(uint64_t) * tab.size());
+  t.rc_tab = (uint64_t *)p;
   put(p, pb.data(), sizeof(uint32_t) * pb.size());
   t.pb = (uint32_t *)p;
   put(p, soff.data(), sizeof(uint64_t) * nsl);
