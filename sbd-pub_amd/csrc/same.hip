@@ -357,14 +357,23 @@ void tile_mm(Context &c, const SameTiles &o, int n, int M, const double *x, cons
   check_launch("k_tile_mm");
 }
 
-const SameTiles &tiles_a(Context &c) {
-  if (!c.tiles_a.val) build_tiles(c, c.A, c.h_astr, c.nb, c.tiles_a);
-  return c.tiles_a;
+// The tiles, built on first use: all of their tables or none, so that a call
+// after a failed one starts anew.
+const SameTiles &tiles_of(Context &c, const SpinTables &t, const std::vector<uint64_t> &strs, size_t cols,
+                          SameTiles &o) {
+  if (o.val) return o;
+  SameTiles n;
+  try {
+    build_tiles(c, t, strs, cols, n);
+  } catch (...) {
+    dfree(c, n.rows), dfree(c, n.base), dfree(c, n.list), dfree(c, n.val);
+    throw;
+  }
+  return o = n;
 }
+const SameTiles &tiles_a(Context &c) { return tiles_of(c, c.A, c.h_astr, c.nb, c.tiles_a); }
 const SameTiles &tiles_b(Context &c) {
-  if (c.B.alias) return tiles_a(c);
-  if (!c.tiles_b.val) build_tiles(c, c.B, c.h_bstr, c.na, c.tiles_b);
-  return c.tiles_b;
+  return c.B.alias ? tiles_a(c) : tiles_of(c, c.B, c.h_bstr, c.na, c.tiles_b);
 }
 
 }  // namespace
