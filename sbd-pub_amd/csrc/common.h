@@ -390,6 +390,7 @@ void build_spin_tables(Context &c, SpinTables &t, const std::vector<uint64_t> &s
 void build_singles_ell(Context &c, SpinTables &t);
 void build_singles_ell_parts(Context &c, SpinTables &t, int nparts);
 void build_blocks(Context &c);
+void release_blocks(Context &c);
 void build_rdm_tables(Context &c, SpinTables &t, const std::vector<uint64_t> &strs, bool as_alpha, bool as_beta);
 void compute_diag(Context &c);
 void sign_convert(Context &c, const double *in, double *out);      // out = S*in

@@ -1670,8 +1670,7 @@ __global__ void __launch_bounds__(256) k_spectator(int Kt, int L, const uint64_t
   }
 }
 static void blk_tables(Context &c) {
-  if (c.eri_tri) return;
-  double *e = (double *)dalloc(c, sizeof(double) * (size_t)c.Kt * (c.Kt + 1));
+  double *e = c.eri_tri = (double *)dalloc(c, sizeof(double) * (size_t)c.Kt * (c.Kt + 1));
   hipLaunchKernelGGL(k_eri_tri, dim3(std::min<unsigned>(cdiv((size_t)c.Kt * (c.Kt + 1), 256), 4096)), dim3(256), 0,
                      c.stream, c.Kt, c.K, c.L, c.B.bk_ref, (const uint16_t *)c.tri_rs, (const double *)c.eri, e);
   check_launch("k_eri_tri");
@@ -1679,7 +1678,6 @@ static void blk_tables(Context &c) {
   hipLaunchKernelGGL(k_spectator, dim3((unsigned)c.na), dim3(256), 0, c.stream, c.Kt, c.L,
                      (const uint64_t *)c.A.str, (const uint16_t *)c.tri_rs, (const double *)e, c.spec);
   check_launch("k_spectator");
-  c.eri_tri = e;
 }
 
 // Geometry of k_mixed_blk for this context: waves per group, matrix waves
@@ -1805,7 +1803,8 @@ static void mixed_blk(Context &c, const double *x, double *y) {
 // Whether the block kernel computes the FP64 mixed term of the general form,
 // decided on a context's first FP64 product: wherever its tables hold the
 // set (ERIs symmetric in rs, at most 44 orbitals, an LDS image of the beta
-// strings, spectator rows of at most 1 GiB).  Its time against the fastest
+// strings, spectator rows of at most 1 GiB, all tables in a quarter of free
+// memory).  Its time against the fastest
 // form without blocks, of one product's mixed term: 60 x 60 strings 14 : 22
 // us, 275 x 239 38 : 72 us, 1543 x 1387 0.73 : 1.24 ms, 8000 x 8000 30.7 :
 // 43.5 ms, 11003 x 11003 111 : 180 ms.  SBDX_MIXED_EB or SBDX_MIXED_NT fix
@@ -1814,14 +1813,25 @@ static bool use_blk(Context &c) {
   if (c.blk_mode < 0) {
     bool on = c.mixed_eb[0] == 0 && !std::getenv("SBDX_MIXED_EB") && !std::getenv("SBDX_MIXED_NT") &&
               sizeof(double) * (size_t)c.Kt * c.na <= ((size_t)1 << 30);
+    auto give_back = [&]() {
+      release_blocks(c);
+      dfree(c, c.eri_tri);
+      dfree(c, c.spec);
+      c.eri_tri = c.spec = nullptr;
+    };
     try {
       if (on) build_blocks(c);
       on = on && c.B.has_blk && blk_geom(c).nmw >= 0;
       if (on) blk_tables(c);
     } catch (const Error &e) {
+      give_back();
       if (e.code != 4) throw;  // SBDX_ERR_ALLOC
       on = false;  // no room for the tables: the other kernels need none
+    } catch (...) {
+      give_back();
+      throw;
     }
+    if (!on) give_back();
     if (on) c.mixed_eb[0] = kEbBlocks, c.mixed_nt[0] = blk_geom(c).nt;
     c.blk_mode = on ? 1 : 0;
   }
@@ -2184,19 +2194,25 @@ static T *densify(Context &c, const SpinTables &t) {
   return H;
 }
 
-void dense_blocks(Context &c, double *&Ha, double *&Hb) {
-  if (!c.Hd_a) {
-    c.Hd_a = densify<double>(c, c.A);
-    c.Hd_b = c.B.alias ? c.Hd_a : densify<double>(c, c.B);
+// Both blocks or neither, so that a call after a failed one starts anew.
+template <typename T>
+static void densify_both(Context &c, T *&Ha, T *&Hb) {
+  T *a = densify<T>(c, c.A), *b = a;
+  try {
+    if (!c.B.alias) b = densify<T>(c, c.B);
+  } catch (...) {
+    dfree(c, a);
+    throw;
   }
+  Ha = a, Hb = b;
+}
+void dense_blocks(Context &c, double *&Ha, double *&Hb) {
+  if (!c.Hd_a) densify_both(c, c.Hd_a, c.Hd_b);
   Ha = c.Hd_a;
   Hb = c.Hd_b;
 }
 static void dense_blocks(Context &c, float *&Ha, float *&Hb) {
-  if (!c.Hf_a) {
-    c.Hf_a = densify<float>(c, c.A);
-    c.Hf_b = c.B.alias ? c.Hf_a : densify<float>(c, c.B);
-  }
+  if (!c.Hf_a) densify_both(c, c.Hf_a, c.Hf_b);
   Ha = c.Hf_a;
   Hb = c.Hf_b;
 }

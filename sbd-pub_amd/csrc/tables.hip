@@ -1015,6 +1015,14 @@ static void build_blocks_ket(Context &c, SpinTables &t, const std::vector<uint64
     len[sl] = mx | (md << 16);
     tot += mx;
   }
+  // all tables of the form, the bras' and those of blk_tables among them
+  const size_t bytes = sizeof(uint32_t) * (col_off.size() + step.size() + perm.size() + 2 * (size_t)nsl + c.na +
+                                           (size_t)(tot + 4) * 256) +
+                       sizeof(uint16_t) * (col_pos.size() + rec.size()) + sizeof(uint2) * tab.size() +
+                       sizeof(uint64_t) * (c.A.ns + c.na) + sizeof(double) * Kt * ((size_t)Kt + 1 + c.na);
+  size_t free_b = 0, total_b = 0;
+  SBDX_HIP(hipMemGetInfo(&free_b, &total_b));
+  if (bytes >= free_b / 4) return;  // the room may be wanted for a solver's basis
   // dealt in the word layout of schedule_slice_packed, whose fields hold LDS
   // elements: the ket's 2 Kt + 1 + ket, the ERI value's triangle index
   const uint32_t xe = 2u * (uint32_t)Kt + 1u;
@@ -1074,6 +1082,20 @@ static void build_blocks_ket(Context &c, SpinTables &t, const std::vector<uint64
 void build_blocks(Context &c) {
   build_blocks_ket(c, c.B, c.h_bstr);
   if (c.B.has_blk) build_blocks_bra(c, c.A, c.h_astr);
+}
+
+// Gives back what build_blocks has laid down.
+void release_blocks(Context &c) {
+  auto drop = [&](auto *&p) {
+    dfree(c, p);
+    p = nullptr;
+  };
+  c.B.has_blk = false;
+  for (SpinTables *t : {&c.A, &c.B}) {
+    drop(t->bk_ent), drop(t->bk_order);
+    drop(t->bk_col_off), drop(t->bk_col_pos), drop(t->bk_step), drop(t->bk_tab);
+    drop(t->bk_perm), drop(t->bk_rec), drop(t->bk_off), drop(t->bk_len), drop(t->bk_ell);
+  }
 }
 
 void build_rdm_tables(Context &c, SpinTables &t, const std::vector<uint64_t> &strs, bool as_alpha, bool as_beta) {
