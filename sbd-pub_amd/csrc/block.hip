@@ -240,18 +240,20 @@ __device__ __forceinline__ void sum_parts(const double *part, int nblk, double *
 }
 
 // v -= (x . v)/|x|^2 x with x . v in p_in and |x|^2 in *n2 (0: x was
-// dropped, v stays), and the next projection's share of next . v to p_out.
+// dropped, v stays, whatever x holds), and the next projection's share of
+// next . v to p_out.
 __global__ void __launch_bounds__(kBT) k_mgs_step(const double *__restrict__ x, const double *next, double *v,
                                                   size_t n, const double *__restrict__ p_in, int nblk,
                                                   const double *__restrict__ n2, double *__restrict__ p_out) {
   __shared__ double sh[4], dot;
   sum_parts(p_in, nblk, &dot);
   __syncthreads();
-  const double o = *n2 > 0.0 ? dot / *n2 : 0.0;
+  const bool kept = *n2 > 0.0;
+  const double o = kept ? dot / *n2 : 0.0;
   const size_t stride = (size_t)gridDim.x * blockDim.x;
   double s = 0.0;
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const double t = v[i] - o * x[i];
+    const double t = kept ? v[i] - o * x[i] : v[i];
     v[i] = t;
     s += (next == v ? t : next[i]) * t;
   }
@@ -261,13 +263,13 @@ __global__ void __launch_bounds__(kBT) k_mgs_step(const double *__restrict__ x, 
 }
 
 // *n2 = |v|^2 from the partials, or 0 when it has fallen to 1e-20 of *ref
-// or is not positive (the vector is dropped).
+// or is not positive and finite (the vector is dropped).
 __global__ void __launch_bounds__(64) k_mgs_norm(const double *__restrict__ part, int nblk,
                                                  const double *__restrict__ ref, double *__restrict__ n2) {
   __shared__ double s;
   sum_parts(part, nblk, &s);
   __syncthreads();
-  if (threadIdx.x == 0) *n2 = (s > 1e-20 * *ref && s > 0.0) ? s : 0.0;
+  if (threadIdx.x == 0) *n2 = (s > 1e-20 * *ref && s > 0.0 && isfinite(s)) ? s : 0.0;
 }
 
 // out_j = sum_k U[k + ld*j] in_k for j < nout <= kOutMax.  In place is
