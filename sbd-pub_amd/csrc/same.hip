@@ -394,11 +394,17 @@ bool same_mm_fits(const Context &c) {
 // kernels over them are faster than tiles that are nearly all zeros: at 60
 // multiply-adds of the matrix cores per entry (the rates of the two forms,
 // 70 and 1.3 TFLOP/s at 8000 x 8000 strings); and a single row or column of a
-// large set would read its whole dense block.
+// large set would read its whole dense block.  Up to kSameSmall the one
+// launch saves 9 us of launches and takes 0.092 us per 1e6 multiply-adds, the
+// row kernels 1.4 us per 1e6 entries: a product of random strings over 40
+// orbitals takes 32 us with the dense blocks and 38 with the rows at 250 x
+// 250, 58 and 46 at 500 x 500, 85 and 60 at 600 x 600; over 24 orbitals 85
+// and 80 at 600 x 600 (18e6 entries), 90 and 102 at 600 x 590 (33e6).
 bool same_mm_worth(const Context &c) {
   const double work = (double)c.N * ((double)c.na + (double)c.nb);
   const double ent = (double)(c.A.ns + c.A.nd) * (double)c.nb + (double)(c.B.ns + c.B.nd) * (double)c.na;
-  return c.na + c.nb <= kSameSmall || (!small(c) && work <= 60.0 * ent);
+  if (c.na + c.nb <= kSameSmall) return work <= 1e8 + 15.0 * ent;
+  return !small(c) && work <= 60.0 * ent;
 }
 
 // y = hii*x + H_a X + X H_b; xt and yt: N doubles each
