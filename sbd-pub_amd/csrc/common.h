@@ -398,6 +398,7 @@ void sign_convert_noprof(Context &c, const double *in, double *out);  // out = S
 void sign_convert_add(Context &c, const double *in, double *out);  // out += S*in
 
 // sigma.hip
+bool blk_worth(const Context &c, size_t covered);
 void sigma_alpha_first(Context &c, const double *x, double *y);  // y = H' x (overwrite)
 void sigma_alpha_first_f32(Context &c, const double *x, double *y);  // same, FP32 arithmetic
 void ensure_f32(Context &c);

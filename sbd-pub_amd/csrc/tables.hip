@@ -971,8 +971,11 @@ static void build_blocks_ket(Context &c, SpinTables &t, const std::vector<uint64
     return a >= 0 && a == col_of[(e & 0xffffffffull) * L + pq % L];
   };
   std::vector<uint32_t> cnt(n, 0);
-  for (int r = 0; r < n; r++)
+  size_t nrest = 0;
+  for (int r = 0; r < n; r++) {
     for (uint64_t k = off[r]; k < off[r + 1]; k++) cnt[r] += covered(r, ent[k]) ? 0 : 1;
+    nrest += cnt[r];
+  }
   // the reference string, when the rows differ from it in fewer orbitals
   // than they have electrons
   size_t nd = 0, ne = 0;
@@ -1015,6 +1018,9 @@ static void build_blocks_ket(Context &c, SpinTables &t, const std::vector<uint64
     len[sl] = mx | (md << 16);
     tot += mx;
   }
+  t.bk_nslice = nsl;
+  t.bk_ngroup = (int)tot;
+  if (!blk_worth(c, t.ns - nrest)) return;
   // all tables of the form, the bras' and those of blk_tables among them
   const size_t bytes = sizeof(uint32_t) * (col_off.size() + step.size() + perm.size() + 2 * (size_t)nsl + c.na +
                                            (size_t)(tot + 4) * 256) +
@@ -1056,8 +1062,6 @@ static void build_blocks_ket(Context &c, SpinTables &t, const std::vector<uint64
     for (size_t i = 0; i < words; i++)
       if (dealt[i] != pad) o[i] = ((((dealt[i] >> 4) & 0x7fffu) - xe) << t.bk_pb) | ((dealt[i] >> 19) << 21);
   });
-  t.bk_nslice = nsl;
-  t.bk_ngroup = (int)tot;
   const StreamWait wait(c);
   auto put = [&](const void *src, size_t bytes) {
     void *dst = dalloc(c, bytes);
