@@ -18,6 +18,7 @@
 #include <map>
 #include <stdexcept>
 #include <string>
+#include <thread>
 #include <vector>
 
 namespace sbdx {
@@ -162,6 +163,17 @@ struct SameTiles {
   double *val = nullptr;
 };
 
+// Threads of a context's host work that may still have to end; joined when
+// there are many and with the context.
+struct HostThreads {
+  std::vector<std::thread> t;
+  void join() {
+    for (auto &x : t) x.join();
+    t.clear();
+  }
+  ~HostThreads() { join(); }
+};
+
 struct ProfSlot {
   std::vector<std::pair<hipEvent_t, hipEvent_t>> ev;
   long launches = 0;
@@ -208,6 +220,7 @@ struct Context {
   int blk_mode = -1;           // FP64 mixed term by k_mixed_blk: undecided, no, yes
   double *spec = nullptr;      // [na][Kt]: spectator rows of the alpha strings (with eri_tri)
   double *h1 = nullptr;    // [K] spatial one-body
+  HostThreads helpers;
   SpinTables A, B;
   double *hii = nullptr;   // [N]
   F32Operands f32;

@@ -9,9 +9,10 @@
 // without sorting.
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <exception>
+#include <memory>
 #include <mutex>
-#include <thread>
 
 #include "common.h"
 
@@ -25,31 +26,51 @@
 namespace sbdx {
 
 // fn(i) for i in [0, n) on up to 16 host threads (work independent per i);
-// an exception of any of them is rethrown here once all have ended.
+// an exception of any of them is rethrown here once all have ended.  The call
+// ends with the last item, not with the last thread: a thread that the
+// system starts late, on a busy host a scheduler's tick of 3 ms later, finds
+// nothing left, and the context joins it afterwards (waiting for it here, the
+// first product of 300 x 289 strings took 3.8 ms beside a BLAS library's
+// spinning threads, 0.6 this way).  Such a thread touches the shared counters
+// alone; fn lives as long as any item is worked on.
 template <typename F>
-static void parallel_for(int n, const F &fn) {
-  const int nthr = std::max(1, std::min({16, (int)std::thread::hardware_concurrency(), n}));
-  std::atomic<int> next{0};
-  std::exception_ptr err;
-  std::mutex mu;
-  auto worker = [&]() {
-    try {
-      for (int i = next++; i < n; i = next++) fn(i);
-    } catch (...) {
-      std::lock_guard<std::mutex> lock(mu);
-      if (!err) err = std::current_exception();
-      next = n;
+static void parallel_for(Context &c, int n, const F &fn) {
+  struct Shared {
+    std::atomic<int> next{0};
+    std::mutex mu;
+    std::condition_variable ended;
+    int done = 0;
+    std::exception_ptr err;
+  };
+  if (n <= 0) return;
+  auto sh = std::make_shared<Shared>();
+  auto worker = [sh, n, f = &fn]() {
+    for (int i = sh->next++; i < n; i = sh->next++) {
+      std::exception_ptr e;
+      try {
+        (*f)(i);
+      } catch (...) {
+        e = std::current_exception();
+      }
+      std::lock_guard<std::mutex> lock(sh->mu);
+      if (e && !sh->err) {
+        sh->err = e;
+        const int first = sh->next.exchange(n);  // nobody takes the rest
+        if (first < n) sh->done += n - first;
+      }
+      if (++sh->done == n) sh->ended.notify_all();
     }
   };
-  std::vector<std::thread> pool;
-  pool.reserve(nthr);
+  if (c.helpers.t.size() >= 32) c.helpers.join();
+  const int nthr = std::max(1, std::min({16, (int)std::thread::hardware_concurrency(), n}));
   try {
-    for (int i = 1; i < nthr; i++) pool.emplace_back(worker);
+    for (int i = 1; i < nthr; i++) c.helpers.t.emplace_back(worker);
   } catch (...) {  // no more threads: those that run and this one do the work
   }
   worker();
-  for (auto &th : pool) th.join();
-  if (err) std::rethrow_exception(err);
+  std::unique_lock<std::mutex> lock(sh->mu);
+  sh->ended.wait(lock, [&]() { return sh->done == n; });
+  if (sh->err) std::rethrow_exception(sh->err);
 }
 
 __device__ __forceinline__ double parity1(uint64_t s, int a, int b) {
@@ -628,7 +649,7 @@ void build_singles_ell(Context &c, SpinTables &t) {
   // in turn) that was 37 of 49 ms; with this split and the searches' pair sets
   // as bits the whole build takes 22 ms.
   const int ng = lane_groups(wide), forms = 1 + (packed ? ng : 0) + (triangle ? ng : 0);
-  parallel_for(nsl * forms, [&](int item) {
+  parallel_for(c, nsl * forms, [&](int item) {
     const int sl = item / forms, f = item % forms;
     auto each = [&](int l, auto take) {
       const uint32_t r = perm[(size_t)sl * 64 + l];
@@ -1037,7 +1058,7 @@ static void build_blocks_ket(Context &c, SpinTables &t, const std::vector<uint64
   std::fill(ell.begin(), ell.end(), (uint32_t)n << t.bk_pb);
   const bool wide = t.bk_pb == 4;
   const int ng = lane_groups(wide);
-  parallel_for(nsl * ng, [&](int item) {
+  parallel_for(c, nsl * ng, [&](int item) {
     const int sl = item / ng;
     const size_t words = (size_t)(len[sl] & 0xffffu) * 256;
     std::vector<uint32_t> dealt(words, pad);
