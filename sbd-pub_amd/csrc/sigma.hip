@@ -2030,10 +2030,27 @@ static int mixed_cfg(Context &c, const T *eri, const T *x) {
   // against 90 at 275 (at 500: 108 against 104).  Fewer slots than cover a row
   // took 1.86 against 1.58 ms at 4001.  Timing them all took 15 products
   // per form of a context's first use, 150 of 320 ms of a first solve at 4001.
+  // Of 300 more cases (sets of the Hartree-Fock string's excitations and drawn
+  // ones, 60 to 4000 strings, 16 to 40 orbitals) two kinds were slower by more
+  // than 6% than another choice:
+  //  - rows of 1025 strings and more where one bra's rounds last longer than
+  //    the shares of all others on their CUs (`shares` of them): half the
+  //    slots, so that two blocks share a bra, from 2.4 shares on in the
+  //    symmetric form, where a long row's work is uneven (1100 strings in 28
+  //    orbitals, 2.8 shares: 506 -> 414 us FP64, 305 -> 254 FP32; 2000 in 36,
+  //    2.8: 1.25 -> 1.08 ms; a drawn set of 2.3 shares 182 -> 200 us in FP32), from 1.8
+  //    with four slots (2400 in 36, 2.1: 1.64 -> 1.33 ms; 3000 in 40, 1.9:
+  //    2.21 -> 1.88), and from 4.2 in the
+  //    general form (1600 in 40, 4.3: 831 -> 749 us; 3.8: 668 -> 679);
+  //  - four pairs a round where hardly a bra has as many (at most one single:
+  //    14.0 -> 11.3 us at 275 random strings in 36 orbitals).
   if (c.B.has_ell3 && !fix_eb && !fix_nt) {
     int nt = 1;
     while (nt < nt_max && nt < 8) nt *= 2;
-    const int eb = SYM && sizeof(T) == 8 && c.B.n < 400 ? 4 : kEbSigned;
+    const size_t per_cu = std::min<size_t>(2, std::max<size_t>(1, c.lds_limit / (kSwKetBase + 16 * (c.nb + 1))));
+    const double shares = (double)(c.A.max_s * c.n_cu * per_cu) / (double)std::max<size_t>(c.A.ns, 1);
+    if (nt > 1 && shares >= (SYM ? (nt > 2 ? 1.8 : 2.4) : 4.2)) nt /= 2;
+    const int eb = SYM && sizeof(T) == 8 && c.B.n < 400 && c.A.max_s > 1 ? 4 : kEbSigned;
     SBDX_HIP(hipEventRecord(e0, c.stream));
     const bool ok = mixed_ell_cfg<SYM>(c, eb, nt, eri, x, scratch);  // false where it does not fit the LDS
     SBDX_HIP(hipEventRecord(e1, c.stream));
