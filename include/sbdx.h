@@ -179,20 +179,20 @@ int sbdx_same_spin_form(sbdx_handle_t h, int precision, int *form, float *ms_spa
 
 /* Configuration of the mixed-term kernel chosen for `precision` 0 (FP64) or
  * 1 (FP32) of the general sigma, or 2 (FP64) or 3 (FP32) of the spin-flip
- * symmetric sigma, on the first product of that form: by the number of
- * strings up to 8191 of them (with integrals (pq|rs) = (pq|sr)), else by
- * timing every staging width (alpha singles staged in LDS per round: 1, 2, 4, or 16 for
+ * symmetric sigma, on the first product of that form: by the numbers of
+ * strings and singles up to 8191 strings (with integrals (pq|rs) = (pq|sr)),
+ * else by timing every staging width (alpha singles staged in LDS per round: 1, 2, 4, or 16 for
  * the signed-triangle kernel, whose LDS elements are 16-byte pairs: 4 FP32
  * or 2 FP64 values, and whose staged ERI rows hold the r >= s triangle with
  * both signs) and slots per thread (1, 2, 4, 8; a row's slots are split
  * over blocks accordingly) that fit (no counterpart in the reference):
  * *width 0 before that, -1 when no width fits in LDS (row parts or the
  * CSR/global variants run), 32 for the block kernel of the general FP64 sigma
- * (taken without timing wherever its tables hold the string sets;
- * *slots_per_thread is then the slices of 64 strings per wave it is built
- * for and *ms 0), else 1, 2, 4 or 16; *slots_per_thread, *ms the
- * chosen and its time (with width -1: the row-parts kernel's slots per
- * thread, timed the same way on its first use; SBDX_PARTS_NT fixes it);
+ * (by the blocks of singles that the sets hold; *slots_per_thread is then the
+ * slices of 64 strings per wave it is built for), else 1, 2, 4 or 16;
+ * *slots_per_thread, *ms the chosen and its time, 0 where it was not timed
+ * (with width -1: the row-parts kernel's slots per thread, timed the same way
+ * on its first use; SBDX_PARTS_NT fixes it);
  * *multi (forms 0
  * and 1) whether block products use the multi-vector kernel (1) or
  * per-vector launches (0), decided by timing on the first block product

@@ -1588,10 +1588,14 @@ static void launch_mixed_ell(Context &c, const T *eri, const T *x, T *y, size_t 
 
 // EB pairs staged per round, NT slots per thread (1, 2, 4 or 8); false when
 // the staging does not fit in LDS.
+template <typename T>
+static size_t mixed_ell_lds(const Context &c, int eb) { return sizeof(T) * eb * ((size_t)c.nb + c.K + 1); }
+template <typename T>
+static bool mixed_ell_fits(const Context &c, int eb) { return mixed_ell_lds<T>(c, eb) <= c.lds_limit && c.B.has_ell2; }
 template <typename T, int EB, bool SYM = false>
 static bool mixed_ell_dispatch(Context &c, int nt, const T *eri, const T *x, T *y) {
-  const size_t lds = sizeof(T) * EB * ((size_t)c.nb + c.K + 1);
-  if (lds > c.lds_limit || !c.B.has_ell2) return false;
+  if (!mixed_ell_fits<T>(c, EB)) return false;
+  const size_t lds = mixed_ell_lds<T>(c, EB);
   if (nt <= 1) launch_mixed_ell<T, 1, EB, SYM>(c, eri, x, y, lds);
   else if (nt <= 2) launch_mixed_ell<T, 2, EB, SYM>(c, eri, x, y, lds);
   else if (nt <= 4) launch_mixed_ell<T, 4, EB, SYM>(c, eri, x, y, lds);
@@ -1624,10 +1628,14 @@ static void launch_mixed_sw(Context &c, const T *eri, const T *x, T *y, size_t l
 
 // The signed-triangle kernel, NT slots per thread; false when its table was
 // not built or its LDS image does not fit.
+static size_t mixed_sw_lds(const Context &c) { return kSwKetBase + (size_t)16 * ((size_t)c.nb + 1); }
+static bool mixed_sw_fits(const Context &c) {
+  return c.B.has_ell3 && (size_t)32 * c.Kt <= kSwKetBase && c.nb + 1 <= 8192 && mixed_sw_lds(c) <= c.lds_limit;
+}
 template <typename T, bool SYM = false>
 static bool mixed_sw_dispatch(Context &c, int nt, const T *eri, const T *x, T *y) {
-  const size_t lds = kSwKetBase + (size_t)16 * ((size_t)c.nb + 1);
-  if (!c.B.has_ell3 || (size_t)32 * c.Kt > kSwKetBase || c.nb + 1 > 8192 || lds > c.lds_limit) return false;
+  if (!mixed_sw_fits(c)) return false;
+  const size_t lds = mixed_sw_lds(c);
   if (nt <= 1) launch_mixed_sw<T, 1, SYM>(c, eri, x, y, lds);
   else if (nt <= 2) launch_mixed_sw<T, 2, SYM>(c, eri, x, y, lds);
   else if (nt <= 4) launch_mixed_sw<T, 4, SYM>(c, eri, x, y, lds);
@@ -1769,7 +1777,7 @@ bool blk_worth(const Context &c, size_t covered) {
     if (g.nwg == 4 && g.ng == 1) return true;
     if (t.bk_ntask == 0) return g.ng <= 2;
   }
-  const size_t per_cu = std::min<size_t>(2, std::max<size_t>(1, c.lds_limit / (kSwKetBase + 16 * (c.nb + 1))));
+  const size_t per_cu = std::min<size_t>(2, std::max<size_t>(1, c.lds_limit / mixed_sw_lds(c)));
   return c.A.max_s >= 30 && (double)(c.A.max_s * c.n_cu * per_cu) >= 3.5 * (double)c.A.ns;
 }
 
@@ -2017,10 +2025,6 @@ static int mixed_cfg(Context &c, const T *eri, const T *x) {
     throw Error(1, "SBDX_MIXED_EB must be 1, 2, 4 or 16");
   if (env_nt && fix_nt != 1 && fix_nt != 2 && fix_nt != 4 && fix_nt != 8)
     throw Error(1, "SBDX_MIXED_NT must be 1, 2, 4 or 8");
-  T *scratch = scratch_vec(c, x);
-  hipEvent_t e0, e1;
-  SBDX_HIP(hipEventCreate(&e0));
-  SBDX_HIP(hipEventCreate(&e1));
   // Where the signed-triangle table exists (up to 8191 strings) the choice is
   // known: that kernel with the fewest slots per thread that cover a row,
   // or four pairs a round for symmetric FP64 products of small sets.  Of 27
@@ -2047,23 +2051,19 @@ static int mixed_cfg(Context &c, const T *eri, const T *x) {
   if (c.B.has_ell3 && !fix_eb && !fix_nt) {
     int nt = 1;
     while (nt < nt_max && nt < 8) nt *= 2;
-    const size_t per_cu = std::min<size_t>(2, std::max<size_t>(1, c.lds_limit / (kSwKetBase + 16 * (c.nb + 1))));
+    const size_t per_cu = std::min<size_t>(2, std::max<size_t>(1, c.lds_limit / mixed_sw_lds(c)));
     const double shares = (double)(c.A.max_s * c.n_cu * per_cu) / (double)std::max<size_t>(c.A.ns, 1);
     if (nt > 1 && shares >= (SYM ? (nt > 2 ? 1.8 : 2.4) : 4.2)) nt /= 2;
     const int eb = SYM && sizeof(T) == 8 && c.B.n < 400 && c.A.max_s > 1 ? 4 : kEbSigned;
-    SBDX_HIP(hipEventRecord(e0, c.stream));
-    const bool ok = mixed_ell_cfg<SYM>(c, eb, nt, eri, x, scratch);  // false where it does not fit the LDS
-    SBDX_HIP(hipEventRecord(e1, c.stream));
-    SBDX_HIP(hipEventSynchronize(e1));
-    if (ok) {
-      check_launch("k_mixed_ell");
-      SBDX_HIP(hipEventElapsedTime(&c.mixed_best_ms[pi], e0, e1));
-      SBDX_HIP(hipEventDestroy(e0));
-      SBDX_HIP(hipEventDestroy(e1));
+    if (eb == kEbSigned ? mixed_sw_fits(c) : mixed_ell_fits<T>(c, eb)) {
       c.mixed_nt[pi] = nt;
       return c.mixed_eb[pi] = eb;
     }
   }
+  T *scratch = scratch_vec(c, x);
+  hipEvent_t e0, e1;
+  SBDX_HIP(hipEventCreate(&e0));
+  SBDX_HIP(hipEventCreate(&e1));
   // else every configuration timed, in the fixed order (the signed-triangle
   // kernel, then eb descending; nt ascending)
   std::vector<std::array<float, 3>> timed;
