@@ -138,7 +138,7 @@ struct SpinTables {
   int4 rc_range[24];
   int rc_nrange = 0;
   // The singles that no column covers, by pair index rs: each pair's entries
-  // in runs of at most one length, chosen to make up to 8 slices of 64 runs;
+  // in runs of at most one length (of 64 runs a slice, the longest first);
   // entry k of lane l of slice s at pb[pb_off[s] + 64 k + l] = bra | ket <<
   // 15 | (sign<0) << 31 (padding: bra = ket = n), pb_len[s] entries per
   // lane, pb_perm[64 s + l] the lane's pair (0xffffffff for none).
