@@ -366,7 +366,6 @@ void dfree_all(Context &c);
 void dfree(Context &c, void *p);  // one dalloc'ed buffer
 Context *make_sub_context(const Context &c, size_t m);  // first m strings of each set
 void destroy_context(Context *c);
-void *blas_handle(Context &c);     // rocblas_handle bound to the stream
 
 // Waits for the stream at scope exit.  Declared after the host arrays that
 // asynchronous copies read or write, it keeps them until the copies have

@@ -17,8 +17,6 @@
 #include <mutex>
 #include <string>
 
-#include <rocblas/rocblas.h>
-
 #include "common.h"
 
 namespace sbdx {
@@ -716,10 +714,10 @@ static void zero(Context &c, double *p, size_t n) {
   check_launch("k_rdm_zero");
 }
 
-// Working memory of one RDM evaluation: per-string sums, the mixed-term
-// accumulator Tm[K][K], and room for ts_cap single pairs and td_cap double
-// pairs (without G the pair tables are processed in chunks of that many
-// entries; with G only td_cap counts).
+// Working memory of one RDM evaluation: the mixed-term accumulator Tm[K][K]
+// and room for td_cap double pairs; with G its Gram matrix, without it
+// per-string sums and room for ts_cap single pairs (the pair tables are
+// processed in chunks of that many entries).
 struct RdmWork {
   double *rho_a, *rho_b, *Tm, *Ts, *Td;
   size_t ts_cap, td_cap;
@@ -806,18 +804,23 @@ void compute_rdm(Context &c, const double *Wp, double *one, double *two) {
   const size_t K = (size_t)c.K;
   const size_t ns = std::max<size_t>(std::max(c.A.ns, c.B.ns), 1);
   const size_t nd = std::max<size_t>(std::max(c.A.nd, c.B.nd), 1);
-  TmpBuf b_rho_a(sizeof(double) * c.na), b_rho_b(sizeof(double) * c.nb), b_tm(sizeof(double) * K * K),
-      b_ts(sizeof(double) * ns), b_td(sizeof(double) * nd);
-  RdmWork wk{(double *)b_rho_a.p, (double *)b_rho_b.p, (double *)b_tm.p, (double *)b_ts.p, (double *)b_td.p, ns, nd};
-  // the Gram matrices of the double pairs when a quarter of free memory
-  // holds one (else a dot product per pair)
+  TmpBuf b_tm(sizeof(double) * K * K), b_td(sizeof(double) * nd);
+  RdmWork wk{nullptr, nullptr, (double *)b_tm.p, nullptr, (double *)b_td.p, ns, nd};
+  // the Gram matrices of both spins' pairs when a quarter of free memory
+  // holds one, else dot products per string and per pair
   const size_t mx = std::max(c.na, c.nb);
   size_t free_b = 0, total_b = 0;
   SBDX_HIP(hipMemGetInfo(&free_b, &total_b));
-  std::unique_ptr<TmpBuf> b_g;
+  std::unique_ptr<TmpBuf> b_g, b_rho, b_ts;
   if (mx < (1u << 31) && sizeof(double) * mx * mx < free_b / 4) {
     b_g.reset(new TmpBuf(sizeof(double) * mx * mx));
     wk.G = (double *)b_g->p;
+  } else {
+    b_rho.reset(new TmpBuf(sizeof(double) * (c.na + c.nb)));
+    b_ts.reset(new TmpBuf(sizeof(double) * ns));
+    wk.rho_a = (double *)b_rho->p;
+    wk.rho_b = wk.rho_a + c.na;
+    wk.Ts = (double *)b_ts->p;
   }
   rdm_run(c, Wp, one, two, wk);
 }

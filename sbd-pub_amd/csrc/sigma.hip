@@ -2238,8 +2238,6 @@ static rocblas_handle blas(Context &c) {
   return (rocblas_handle)c.blas;
 }
 
-void *blas_handle(Context &c) { return (void *)blas(c); }
-
 void same_dense_release(Context &c) {
   if (c.blas) (void)rocblas_destroy_handle((rocblas_handle)c.blas);
   c.blas = nullptr;
