@@ -230,6 +230,8 @@ struct Context {
   // (FP64: only for small sets; larger ones as tiles.)
   double *Hd_a = nullptr, *Hd_b = nullptr;
   SameTiles tiles_a, tiles_b;
+  double *same_ws = nullptr;  // transposed vectors of a block product's same-spin terms
+  size_t same_ws_cap = 0;     // doubles in it (at most 2 kBlockDoubles)
   float *Hf_a = nullptr, *Hf_b = nullptr;
   void *blas = nullptr;  // rocblas_handle bound to `stream`
   // Same-spin form per precision [0 FP64, 1 FP32]: -1 not chosen yet,
@@ -434,8 +436,9 @@ void host_syev(int n, double *A, double *Q, double *E);
 // H y = theta S y (S positive definite), n x n column-major with leading
 // dimension ld: S-orthonormal eigenvectors Y (n x n, ld n), E ascending
 void host_sygv(int n, const double *H, const double *S, int ld, double *Y, double *E);
-void transpose_into(Context &c, const double *in, double *out, int R, int Cc);  // out = in^T
-void transpose_add(Context &c, const double *in, double *out, int R, int Cc);   // out += in^T
+// out = in^T and out += in^T, for k contiguous matrices
+void transpose_into(Context &c, const double *in, double *out, int R, int Cc, int k = 1);
+void transpose_add(Context &c, const double *in, double *out, int R, int Cc, int k = 1);
 void dense_blocks(Context &c, double *&Ha, double *&Hb);  // the same-spin blocks, dense, built on first use
 
 // same.hip
@@ -444,6 +447,7 @@ size_t same_mm_bytes(const Context &c);  // at most, for what is not built yet
 bool same_mm_fits(const Context &c);
 bool same_mm_worth(const Context &c);
 void same_mm(Context &c, const double *x, double *y, double *xt, double *yt);
+void same_mm_block(Context &c, int k, const double *x, double *y, double *xt, double *yt);
 void same_mm_alpha(Context &c, const double *x, double *G);
 
 // davidson.hip

@@ -677,8 +677,6 @@ __global__ void k_rdm_mixed_place(int L, const double *__restrict__ Tm, double *
   }
 }
 
-void transpose_into(Context &c, const double *in, double *out, int R, int Cc);
-
 template <int NT, int UT, bool ROWS>
 static void launch_rdm_mixed(Context &c, const double *w, double *Tm) {
   auto fn = k_rdm_mixed<NT, UT, ROWS>;

@@ -122,13 +122,16 @@ __global__ void __launch_bounds__(256) k_tiles(int n, int tm, const uint32_t *__
 // instructions' rate over the tiles), as a dense library product 14.3; of 4001 x
 // 4001 1.44 ms (1.09), as a dense library product 1.86; of 2583 x 2583 0.42 ms
 // at 32 x 32 (with whole lists 0.46); both terms at 1000 x 900 0.10 ms with
-// their transposes, in the small form below 0.19.
+// their transposes, in the small form below 0.19.  blockIdx.y: one of several
+// vectors, vs elements from the one before.
 template <int MT, int NT, int KS, bool DIAG>
 __global__ void __launch_bounds__(256, MT == 4 ? 2 : 4)
     k_tile_mm(int n, int M, int ntile, int nchunk, const uint32_t *__restrict__ rows,
               const uint32_t *__restrict__ base, const uint32_t *__restrict__ list, const double *__restrict__ val,
-              const double *__restrict__ x, const double *__restrict__ hii, double *__restrict__ y) {
+              const double *__restrict__ x, const double *__restrict__ hii, double *__restrict__ y, size_t vs) {
   constexpr int TM = 16 * MT;
+  x += blockIdx.y * vs;
+  y += blockIdx.y * vs;
   const unsigned total = (unsigned)ntile * nchunk, per = (total + 7) / 8;
   const unsigned id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
   if ((blockIdx.x >> 3) >= per || id >= total) return;
@@ -239,12 +242,15 @@ __global__ void __launch_bounds__(256, MT == 4 ? 2 : 4)
 // and their sums added at the end.  Bound by the reads of the operands (1 KB
 // an instruction, no reuse between tiles), but one launch: 14 us at 300 x 280
 // strings, where two library GEMMs after a pass for the diagonal took 45.
+// blockIdx.z: one of several contiguous vectors.
 __global__ void __launch_bounds__(256) k_same_small(int na, int nb, const double *__restrict__ Ha,
                                                     const double *__restrict__ Hb, const double *__restrict__ hii,
                                                     const double *__restrict__ x, double *__restrict__ y) {
   __shared__ double part[4][256];
   const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63, q = lane & 15, g = lane >> 4;
   const int r0 = blockIdx.y * 16, c0 = blockIdx.x * 16;
+  x += (size_t)blockIdx.z * na * nb;
+  y += (size_t)blockIdx.z * na * nb;
   const int rq = min(r0 + q, na - 1), cq = min(c0 + q, nb - 1);
   d4 acc = d4{0.0, 0.0, 0.0, 0.0}, odd = acc;
   // step s: kets 4 s + g of H_a x (s < sa), then of x H_b; past the end zeros
@@ -342,18 +348,19 @@ void build_tiles(Context &c, const SpinTables &t, const std::vector<uint64_t> &s
   SBDX_HIP(hipStreamSynchronize(c.stream));
 }
 
+// for k contiguous vectors
 template <bool DIAG>
-void tile_mm(Context &c, const SameTiles &o, int n, int M, const double *x, const double *hii, double *y) {
+void tile_mm(Context &c, const SameTiles &o, int n, int M, const double *x, const double *hii, double *y, int k = 1) {
   const int nchunk = (int)cdiv(M, o.tm == 64 ? 256 : 64);
   if (M < 2 && n > 1) throw Error(3, "same-spin tiles: one column");
   const size_t blocks = (size_t)8 * cdiv((size_t)o.ntile * nchunk, 8);
   if (blocks >= (1ull << 31)) throw Error(3, "sigma: grid too large for one launch");
   if (o.tm == 64)
-    hipLaunchKernelGGL((k_tile_mm<4, 4, 1, DIAG>), dim3((unsigned)blocks), dim3(256), 0, c.stream, n, M, o.ntile,
-                       nchunk, o.rows, o.base, o.list, o.val, x, hii, y);
+    hipLaunchKernelGGL((k_tile_mm<4, 4, 1, DIAG>), dim3((unsigned)blocks, k), dim3(256), 0, c.stream, n, M, o.ntile,
+                       nchunk, o.rows, o.base, o.list, o.val, x, hii, y, (size_t)n * M);
   else
-    hipLaunchKernelGGL((k_tile_mm<2, 2, 2, DIAG>), dim3((unsigned)blocks), dim3(256), 0, c.stream, n, M, o.ntile,
-                       nchunk, o.rows, o.base, o.list, o.val, x, hii, y);
+    hipLaunchKernelGGL((k_tile_mm<2, 2, 2, DIAG>), dim3((unsigned)blocks, k), dim3(256), 0, c.stream, n, M, o.ntile,
+                       nchunk, o.rows, o.base, o.list, o.val, x, hii, y, (size_t)n * M);
   check_launch("k_tile_mm");
 }
 
@@ -407,22 +414,63 @@ bool same_mm_worth(const Context &c) {
   return !small(c) && work <= 60.0 * ent;
 }
 
+// y = hii*x + H_a X + X H_b for k contiguous vectors on the tiles; xt and yt:
+// k N doubles each
+static void tiles_both(Context &c, int k, const double *x, double *y, double *xt, double *yt) {
+  const int na = (int)c.na, nb = (int)c.nb;
+  tile_mm<true>(c, tiles_a(c), na, nb, x, c.hii, y, k);
+  // the beta term with the vectors transposed, so that it gathers rows too
+  transpose_into(c, x, xt, na, nb, k);
+  tile_mm<false>(c, tiles_b(c), nb, na, xt, nullptr, yt, k);
+  transpose_add(c, yt, y, nb, na, k);
+}
+
+static void small_both(Context &c, int k, const double *x, double *y) {
+  const int na = (int)c.na, nb = (int)c.nb;
+  double *Ha, *Hb;
+  dense_blocks(c, Ha, Hb);
+  hipLaunchKernelGGL(k_same_small, dim3(cdiv(nb, 16), cdiv(na, 16), k), dim3(256), 0, c.stream, na, nb,
+                     (const double *)Ha, (const double *)Hb, c.hii, x, y);
+  check_launch("k_same_small");
+}
+
 // y = hii*x + H_a X + X H_b; xt and yt: N doubles each
 void same_mm(Context &c, const double *x, double *y, double *xt, double *yt) {
-  const int na = (int)c.na, nb = (int)c.nb;
-  if (small(c)) {
-    double *Ha, *Hb;
-    dense_blocks(c, Ha, Hb);
-    hipLaunchKernelGGL(k_same_small, dim3(cdiv(nb, 16), cdiv(na, 16)), dim3(256), 0, c.stream, na, nb,
-                       (const double *)Ha, (const double *)Hb, c.hii, x, y);
-    check_launch("k_same_small");
-    return;
+  if (small(c)) small_both(c, 1, x, y);
+  else tiles_both(c, 1, x, y, xt, yt);
+}
+
+// The same for k contiguous vectors: a launch takes as many as kBlockDoubles
+// hold, so that sets whose single vectors leave CUs idle fill the chip.  The
+// one-launch form while its work is small: two vectors of 380 x 380 strings 31
+// us against 38 on the tiles, four 50 and 50, two of 500 x 500 60 and 45.  One
+// vector after the other, eight of 500 x 500 took 257 us, now 107; of 700 x
+// 700 398 and 244 (batched library products 107 and 265).
+void same_mm_block(Context &c, int k, const double *x, double *y, double *xt, double *yt) {
+  constexpr size_t kBlockDoubles = size_t(4) << 20;
+  const size_t N = c.N;
+  const int group = (int)std::min<size_t>({(size_t)k, kBlockDoubles / N, 65535});
+  const bool one = small(c) && (c.na == 1 || c.nb == 1 || (double)group * N * (c.na + c.nb) <= 4e8);
+  if (group > 1 && !one && c.same_ws_cap < 2 * group * N) {
+    try {
+      double *p = (double *)dalloc(c, sizeof(double) * 2 * group * N);
+      dfree(c, c.same_ws);
+      c.same_ws = p;
+      c.same_ws_cap = 2 * group * N;
+    } catch (const Error &) {  // no room: one vector at a time
+    }
   }
-  tile_mm<true>(c, tiles_a(c), na, nb, x, c.hii, y);
-  // the beta term with the vector transposed, so that it gathers rows too
-  transpose_into(c, x, xt, na, nb);
-  tile_mm<false>(c, tiles_b(c), nb, na, xt, nullptr, yt);
-  transpose_add(c, yt, y, nb, na);
+  for (int v = 0, n; v < k; v += n) {
+    n = std::min(group, k - v);
+    if (n > 1 && one) {
+      small_both(c, n, x + v * N, y + v * N);
+    } else if (n > 1 && c.same_ws_cap >= 2 * n * N) {
+      tiles_both(c, n, x + v * N, y + v * N, c.same_ws, c.same_ws + n * N);
+    } else {
+      n = 1;
+      same_mm(c, x + v * N, y + v * N, xt, yt);
+    }
+  }
 }
 
 // G = H_a X (a single string has an empty list)

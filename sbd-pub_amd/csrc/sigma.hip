@@ -108,11 +108,12 @@ __global__ void __launch_bounds__(256) k_same_xcd(int nrows, int M, int nch, int
 // are in flight at once) and by how many blocks run beside each other:
 // k_sym_combine in FP32 at 500 strings 12.8 us with 64 x 64 tiles, 4.6 with
 // 32 x 32, k_symmetrize at 1001 strings 15.6 and 7.3.
-static bool small_tiles(const Context &c, size_t R, size_t C) {
-  return (size_t)cdiv(R, 64) * cdiv(C, 64) < (size_t)4 * c.n_cu;
+static bool small_tiles(const Context &c, size_t R, size_t C, size_t k = 1) {
+  return (size_t)cdiv(R, 64) * cdiv(C, 64) * k < (size_t)4 * c.n_cu;
 }
 
-// out[c][r] (+)= in[r][c] for an R x Cc row-major matrix, TS x TS LDS tiles.
+// out[c][r] (+)= in[r][c] for an R x Cc row-major matrix, TS x TS LDS tiles
+// (blockIdx.z: one of several contiguous matrices).
 template <typename T, bool ACC, int TS>
 __global__ void __launch_bounds__(256) k_transpose(const T *__restrict__ in, T *__restrict__ out,
                                                    int R, int Cc) {
@@ -120,6 +121,8 @@ __global__ void __launch_bounds__(256) k_transpose(const T *__restrict__ in, T *
   __shared__ T tile[TS][TS + 1];
   const int tx = threadIdx.x % TS, ty = threadIdx.x / TS;
   const int c0 = blockIdx.x * TS, r0 = blockIdx.y * TS;
+  in += (size_t)blockIdx.z * R * Cc;
+  out += (size_t)blockIdx.z * R * Cc;
 #pragma unroll
   for (int q = 0, k = ty; q < TS / ST; q++, k += ST) {
     const int r = r0 + k, cc = c0 + tx;
@@ -1543,27 +1546,27 @@ static void sigma_same(Context &c, const SpinTables &t, const T *s_val, const T 
 }
 
 template <typename T, bool ACC>
-static void launch_transpose(Context &c, const T *in, T *out, int R, int Cc) {
-  if (small_tiles(c, R, Cc))
-    hipLaunchKernelGGL((k_transpose<T, ACC, 32>), dim3(cdiv(Cc, 32), cdiv(R, 32)), dim3(256), 0, c.stream, in, out,
+static void launch_transpose(Context &c, const T *in, T *out, int R, int Cc, int k) {
+  if (small_tiles(c, R, Cc, k))
+    hipLaunchKernelGGL((k_transpose<T, ACC, 32>), dim3(cdiv(Cc, 32), cdiv(R, 32), k), dim3(256), 0, c.stream, in, out,
                        R, Cc);
   else
-    hipLaunchKernelGGL((k_transpose<T, ACC, 64>), dim3(cdiv(Cc, 64), cdiv(R, 64)), dim3(256), 0, c.stream, in, out,
+    hipLaunchKernelGGL((k_transpose<T, ACC, 64>), dim3(cdiv(Cc, 64), cdiv(R, 64), k), dim3(256), 0, c.stream, in, out,
                        R, Cc);
   check_launch("k_transpose");
 }
 template <typename T>
 static void transpose(Context &c, const T *in, T *out, int R, int Cc, bool acc) {
-  if (acc) launch_transpose<T, true>(c, in, out, R, Cc);
-  else launch_transpose<T, false>(c, in, out, R, Cc);
+  if (acc) launch_transpose<T, true>(c, in, out, R, Cc, 1);
+  else launch_transpose<T, false>(c, in, out, R, Cc, 1);
 }
 
-void transpose_into(Context &c, const double *in, double *out, int R, int Cc) {
-  transpose<double>(c, in, out, R, Cc, false);
+void transpose_into(Context &c, const double *in, double *out, int R, int Cc, int k) {
+  launch_transpose<double, false>(c, in, out, R, Cc, k);
 }
 
-void transpose_add(Context &c, const double *in, double *out, int R, int Cc) {
-  transpose<double>(c, in, out, R, Cc, true);
+void transpose_add(Context &c, const double *in, double *out, int R, int Cc, int k) {
+  launch_transpose<double, true>(c, in, out, R, Cc, k);
 }
 
 // Rows of the mixed term are split over ceil(slots / (1024*NT)) blocks.
@@ -2322,7 +2325,7 @@ static rocblas_status gemm_batched(rocblas_handle h, int m, int n, int k, const 
 }
 
 static void same_dense_block(Context &c, const SigmaOperands<double> &o, int k, const double *x, double *y) {
-  for (int v = 0; v < k; v++) same_mm(c, x + v * c.N, y + v * c.N, o.T1, o.T2);
+  same_mm_block(c, k, x, y, o.T1, o.T2);
 }
 
 // FP32 dense form for k contiguous vectors: the alpha term as a strided batch
