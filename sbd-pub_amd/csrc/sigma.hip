@@ -1765,8 +1765,8 @@ static BlkGeom blk_geom(const Context &c) {
 //    D 90 x 3000 0.16 : 0.08 ms, HF 10 x 3000 0.11 : 0.05 (up to four bras,
 //    where a product is some 0.1 ms in either, the block kernel is kept: its
 //    further launches and widest images are tested at such sizes).
-// Without k_mixed_sw's table (8192 strings and more) the other forms stage one
-// value at a time: HF 11000 17 : 38 ms, R 0.45 : 0.60; but D 28.9 : 21.0 ms
+// Without k_mixed_sw (8192 strings and more) the other forms stage one value
+// at a time: HF 11000 17 : 38 ms, R 0.45 : 0.60; but D 28.9 : 21.0 ms
 // (fill 0.17), with few singles in blocks 1.19 : 1.54.
 bool blk_worth(const Context &c, size_t covered) {
   const SpinTables &t = c.B;
@@ -1775,7 +1775,7 @@ bool blk_worth(const Context &c, size_t covered) {
   if (c.nb <= 512 || c.na <= 4) return true;
   if (c.nb > 1024 && c.na < (size_t)c.n_cu) return false;
   if (t.bk_ntask > 0 && (double)covered >= 0.27 * 1024.0 * t.bk_mt * t.bk_nstep) return true;
-  if (!t.has_ell3) return (double)covered < 0.25 * (double)t.ns;
+  if (!mixed_sw_fits(c)) return (double)covered < 0.25 * (double)t.ns;
   if (c.na >= (size_t)c.n_cu) {
     if (g.nwg == 4 && g.ng == 1) return true;
     if (t.bk_ntask == 0) return g.ng <= 2;
