@@ -1741,13 +1741,14 @@ static BlkGeom blk_geom(const Context &c) {
 
 // Whether the block kernel is the faster form on the beta set laid out in
 // c.B, `covered` of whose singles lie in blocks.  A step of the matrix waves
-// takes 16 columns over 4 by 16 bk_mt orbitals; where fewer than 0.27 of its
+// takes 16 columns over 4 by 16 bk_mt orbitals; where fewer than 0.28 of its
 // pairs are singles, the matrix instructions take longer than the same
 // singles one by one.  Measured as block kernel against k_mixed_sw (the
-// fastest of its forms), one product's mixed term, over 330 pairs of sets of
-// 60 to 11003 strings in 12 to 43 orbitals: the Hartree-Fock string's
-// excitations (HF), strings drawn with falling occupation (D), at random (R):
-//  - fill 0.27 and more: HF 8000, 36 orbitals, 0.45: 9.9 : 14.3 ms; HF 3997,
+// fastest of its forms), one product's mixed term, over 490 pairs of sets of
+// 16 to 11003 strings in 12 to 43 orbitals: the Hartree-Fock string's
+// excitations (HF), strings drawn with falling occupation (D), at random (R).
+// The rule loses 1% to the better form of each on average, 25% at most.
+//  - fill 0.28 and more: HF 8000, 36 orbitals, 0.45: 9.9 : 14.3 ms; HF 3997,
 //    28 orbitals, 0.54: 4.7 : 8.0; below: HF 3997, 36 orbitals, 0.14: 6.3 :
 //    5.3; D 8000, 0.17: 12.6 : 8.9; R 3997, 24 orbitals, 0.12: 2.35 : 1.44;
 //    N2's 4041, 0.22: 8.9 : 7.1;
@@ -1755,16 +1756,18 @@ static BlkGeom blk_geom(const Context &c) {
 //    R 18.6 : 20.5 us);
 //  - many bras over a short set, in blocks of one group of four waves that
 //    overlap each other's staging: 4000 x 900, HF 2.0 : 2.7 ms, D 1.0 : 1.4;
-//  - where one bra (the Hartree-Fock string) has so many singles that its
-//    rounds last longer than a CU's share of all others: groups of a block
-//    take its rounds in turn.  HF 597, 36 orbitals: 0.30 : 0.89 ms; the line
-//    is at 3.5 shares (2.8: 0.30 : 0.27 ms, D 997);
 //  - without any block, the entry waves alone: R 1997, 28 orbitals, 50 : 73
 //    us; with four groups a block 43 : 33 us (D 1000);
-//  - fewer bras than CUs leave CUs idle that k_mixed_sw's split rows use:
-//    D 90 x 3000 0.16 : 0.08 ms, HF 10 x 3000 0.11 : 0.05 (up to four bras,
-//    where a product is some 0.1 ms in either, the block kernel is kept: its
-//    further launches and widest images are tested at such sizes).
+//  - where one bra (the Hartree-Fock string) has so many singles that its
+//    rounds last longer than a CU's share of all others (`shares` of them):
+//    groups of a block take its rounds in turn.  HF 597, 36 orbitals: 0.30 :
+//    0.89 ms; the line is at 3.5 shares (2.8: 0.30 : 0.27 ms, D 997).  Rows of
+//    more than 1024 strings k_mixed_sw splits over blocks instead, as it does
+//    for fewer bras than CUs: HF 300 x 3000 0.66 : 0.59 ms, D 300 x 3000 0.55 :
+//    0.21, D 90 x 3000 0.16 : 0.08; not so where four groups work on full
+//    steps (HF 100 x 1100, 0.36: 0.21 : 0.30).  Up to four bras, where a
+//    product is some 0.1 ms in either, the block kernel is kept: its further
+//    launches and widest images are tested at such sizes.
 // Without k_mixed_sw (8192 strings and more) the other forms stage one value
 // at a time: HF 11000 17 : 38 ms, R 0.45 : 0.60; but D 28.9 : 21.0 ms
 // (fill 0.17), with few singles in blocks 1.19 : 1.54.
@@ -1773,15 +1776,16 @@ bool blk_worth(const Context &c, size_t covered) {
   const BlkGeom g = blk_geom(c);
   if (g.nmw < 0) return false;
   if (c.nb <= 512 || c.na <= 4) return true;
-  if (c.nb > 1024 && c.na < (size_t)c.n_cu) return false;
-  if (t.bk_ntask > 0 && (double)covered >= 0.27 * 1024.0 * t.bk_mt * t.bk_nstep) return true;
-  if (!mixed_sw_fits(c)) return (double)covered < 0.25 * (double)t.ns;
-  if (c.na >= (size_t)c.n_cu) {
-    if (g.nwg == 4 && g.ng == 1) return true;
-    if (t.bk_ntask == 0) return g.ng <= 2;
-  }
+  const double fill = t.bk_ntask ? (double)covered / (1024.0 * t.bk_mt * t.bk_nstep) : 0.0;
+  if (!mixed_sw_fits(c)) return fill >= 0.28 || (double)covered < 0.25 * (double)t.ns;
   const size_t per_cu = std::min<size_t>(2, std::max<size_t>(1, c.lds_limit / mixed_sw_lds(c)));
-  return c.A.max_s >= 30 && (double)(c.A.max_s * c.n_cu * per_cu) >= 3.5 * (double)c.A.ns;
+  const double shares = (double)(c.A.max_s * c.n_cu * per_cu) / (double)std::max<size_t>(c.A.ns, 1);
+  const bool few = c.na < (size_t)c.n_cu, heavy = c.A.max_s >= 20;
+  if (c.nb > 1024 && (few || (heavy && shares >= 9.0))) return fill >= 0.3 && g.ng == 4;
+  if (fill >= 0.28) return true;
+  if (!few && g.nwg == 4 && g.ng == 1) return true;
+  if (!few && t.bk_ntask == 0) return g.ng <= 2;
+  return c.nb <= 1024 && heavy && shares >= 3.5;
 }
 
 template <int EB, int MT, int NT>

@@ -24,6 +24,8 @@ pytestmark = pytest.mark.gpu
     ("scattered", 24, 5, 2000, 4, 3997, 16),
     ("scattered", 34, 6, 90, 4, 3000, 16),     # few bras
     ("blocks", 30, 6, 10, 6, 3000, 16),
+    ("blocks", 24, 5, 100, 4, 1100, 32),       # few bras, full steps in four groups
+    ("blocks", 30, 6, 300, 5, 3000, 16),       # one long bra, rows split instead
 ])
 def test_mixed_form_by_the_sets(kind, norb, ea, na, eb, nb, width, monkeypatch):
     import sbdx
