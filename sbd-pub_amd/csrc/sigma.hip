@@ -2051,16 +2051,36 @@ static int mixed_cfg(Context &c, const T *eri, const T *x) {
   //    orbitals, 2.8 shares: 506 -> 414 us FP64, 305 -> 254 FP32; 2000 in 36,
   //    2.8: 1.25 -> 1.08 ms; a drawn set of 2.3 shares 182 -> 200 us in FP32), from 1.8
   //    with four slots (2400 in 36, 2.1: 1.64 -> 1.33 ms; 3000 in 40, 1.9:
-  //    2.21 -> 1.88), and from 4.2 in the
-  //    general form (1600 in 40, 4.3: 831 -> 749 us; 3.8: 668 -> 679);
+  //    2.21 -> 1.88);
   //  - four pairs a round where hardly a bra has as many (at most one single:
   //    14.0 -> 11.3 us at 275 random strings in 36 orbitals).
+  // In the general form the sets differ, and few bras over a long row leave
+  // CUs idle unless more blocks share a bra: each of s blocks takes a bra's
+  // rounds again, for nt of its slots.  A round costs 1.6 + nt slots, a bra two
+  // rounds more; the launch lasts as long as its work over the CUs (with 1.1
+  // for blocks that overlap) or as its longest bra, and the nt with the
+  // smaller of these sums is taken.  Over 524 pairs of sets (16 to 4000 bras,
+  // 1100 to 7000 columns, HF, D and R as at blk_worth) that is 1.4% slower than
+  // the best of all nt on average, and 1.55x at most (220 bras with 34 singles
+  // together, 16 : 11 us); the slots that cover a row 18% and 3.4x (HF 60 x 5000:
+  // 271 us at one slot, 756 at eight; 300 x 5000, drawn: 321 : 551).
   if (c.B.has_ell3 && !fix_eb && !fix_nt) {
     int nt = 1;
     while (nt < nt_max && nt < 8) nt *= 2;
-    const size_t per_cu = std::min<size_t>(2, std::max<size_t>(1, c.lds_limit / mixed_sw_lds(c)));
-    const double shares = (double)(c.A.max_s * c.n_cu * per_cu) / (double)std::max<size_t>(c.A.ns, 1);
-    if (nt > 1 && shares >= (SYM ? (nt > 2 ? 1.8 : 2.4) : 4.2)) nt /= 2;
+    if (SYM) {
+      const size_t per_cu = std::min<size_t>(2, std::max<size_t>(1, c.lds_limit / mixed_sw_lds(c)));
+      const double shares = (double)(c.A.max_s * c.n_cu * per_cu) / (double)std::max<size_t>(c.A.ns, 1);
+      if (nt > 1 && shares >= (nt > 2 ? 1.8 : 2.4)) nt /= 2;
+    } else {
+      const double round = sizeof(T) == 4 ? 4.0 : 2.0, slots = (double)c.B.n / 1024.0;  // pairs a round
+      const double work = ((double)c.A.ns / round + 2.0 * (double)c.A.n) / (1.1 * c.n_cu);
+      const double longest = std::ceil((double)c.A.max_s / round) + 2.0;
+      double least = 0.0;
+      for (int k = 1, most = nt; k <= most; k *= 2) {
+        const double t = std::max(work * std::ceil(slots / k), longest) * (1.6 + std::min((double)k, slots));
+        if (k == 1 || t < 0.999 * least) least = t, nt = k;
+      }
+    }
     const int eb = SYM && sizeof(T) == 8 && c.B.n < 400 && c.A.max_s > 1 ? 4 : kEbSigned;
     if (eb == kEbSigned ? mixed_sw_fits(c) : mixed_ell_fits<T>(c, eb)) {
       c.mixed_nt[pi] = nt;
